@@ -70,17 +70,41 @@ __device__ __forceinline__ float wave_sum_f(float v) {
   return v;
 }
 
-// Wave-wide argmax of (e, idx): larger e wins, ties -> smaller idx.
-__device__ __forceinline__ void wave_argmax(double &e, int &idx) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    double e2 = __shfl_xor(e, o, kWave);
-    int i2 = __shfl_xor(idx, o, kWave);
-    if (e2 > e || (e2 == e && i2 < idx)) {
-      e = e2;
-      idx = i2;
-    }
-  }
+// A double moved by a DPP control within the wave; lanes that the control
+// gives no source (or that kRows leaves out) keep their own value.  A register
+// move of a few cycles where __shfl goes through the LDS unit (~100 cycles).
+template <int kCtrl, int kRows = 0xf>
+__device__ __forceinline__ double dpp_move(double v) {
+  const int lo = __double2loint(v), hi = __double2hiint(v);
+  return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, kCtrl, kRows, 0xf, false),
+                          __builtin_amdgcn_update_dpp(lo, lo, kCtrl, kRows, 0xf, false));
+}
+
+// Lane `lane` (uniform) of a double, in every lane.
+__device__ __forceinline__ double lane_value(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// Largest value of the wave, in every lane (row shifts by 1, 2, 4, 8 leave
+// each row's in its last lane, the row broadcasts the wave's in lane 63).
+__device__ __forceinline__ double wave_max(double v) {
+  v = fmax(v, dpp_move<0x111>(v));
+  v = fmax(v, dpp_move<0x112>(v));
+  v = fmax(v, dpp_move<0x114>(v));
+  v = fmax(v, dpp_move<0x118>(v));
+  v = fmax(v, dpp_move<0x142, 0xa>(v));
+  v = fmax(v, dpp_move<0x143, 0xc>(v));
+  return lane_value(v, kWave - 1);
+}
+
+// Smallest value of lanes 0..15, in every lane.
+__device__ __forceinline__ double row0_min(double v) {
+  v = fmin(v, dpp_move<0x111>(v));
+  v = fmin(v, dpp_move<0x112>(v));
+  v = fmin(v, dpp_move<0x114>(v));
+  v = fmin(v, dpp_move<0x118>(v));
+  return lane_value(v, 15);
 }
 
 // Exclusive prefix sum over the wave of a small int; total returned in *tot.

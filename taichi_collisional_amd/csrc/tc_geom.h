@@ -143,78 +143,92 @@ __device__ inline bool candidate_ball(int mask, int ns, const double (&bq)[3],
 constexpr double kBallTol = 1e-13;
 
 // Smallest ball over the points one block of NW waves can enumerate.
-//   get(i, q)   writes point i (uniform index; used for point 0 and the
-//               selected point of each iteration),
-//   scan(f)     calls f(i, q) for this thread's share of the points, in
-//               increasing i.
+//   p0          point 0, where the iteration starts,
+//   scan(b, f)  calls f(i, q) for this thread's share of the points, in any
+//               order; points inside the ball b may be left out.
 // Per iteration the point of largest excess is found with ties going to the
 // lowest index (thread, wave, then block argmax), so the sequence of support
-// sets -- and hence the ball -- does not depend on NW.  s_e / s_i hold 2 x NW
-// slots (double-buffered: one barrier per iteration).
-template <int NW, class Get, class Scan>
-__device__ DBall block_minball(Get get, Scan scan, double *s_e, int *s_i) {
+// sets -- and hence the ball -- does not depend on NW.  s_e / s_i hold 8 x NW
+// and 2 x NW slots (double-buffered: one barrier per iteration).
+//
+// The top levels are a few blocks, whose time is the latency of one iteration
+// after another.  So the reductions are register moves (DPP) instead of
+// shuffles through the LDS unit, the point of largest excess travels with its
+// excess instead of being looked up again, and the winning candidate's ball
+// is read from the lane that solved it.
+template <int NW, class Scan>
+__device__ DBall block_minball(const double (&p0)[3], Scan scan, double *s_e, int *s_i) {
 #pragma clang fp contract(off)
   const int lane = threadIdx.x & (kWave - 1);
   const int wid = threadIdx.x / kWave;
   DBall b;
   double sup[4][3];
   int ns = 1;
-  get(0, sup[0]);
-  for (int d = 0; d < 3; d++) b.c[d] = sup[0][d];
+  for (int d = 0; d < 3; d++) b.c[d] = sup[0][d] = p0[d];
   b.r2 = 0;
   for (int iter = 0; iter < 10000; iter++) {
-    double best = -1;
+    double best = -1, bq[3] = {0, 0, 0};
     int bidx = 0x7fffffff;
-    scan([&](int i, const double *q) {
+    scan(b, [&](int i, const double *q) {
       double e = 0;
       for (int d = 0; d < 3; d++) e += (q[d] - b.c[d]) * (q[d] - b.c[d]);
       e -= b.r2;
-      if (e > best) {
+      if (e > best || (e == best && i < bidx)) {
         best = e;
         bidx = i;
+        for (int d = 0; d < 3; d++) bq[d] = q[d];
       }
     });
-    wave_argmax(best, bidx);
-    if (NW > 1) {
-      const int par = iter & 1;
-      if (lane == 0) {
-        s_e[par * NW + wid] = best;
-        s_i[par * NW + wid] = bidx;
-      }
-      __syncthreads();
-      best = s_e[par * NW];
-      bidx = s_i[par * NW];
-      for (int w = 1; w < NW; w++) {
-        const double e2 = s_e[par * NW + w];
-        const int i2 = s_i[par * NW + w];
-        if (e2 > best || (e2 == best && i2 < bidx)) {
-          best = e2;
-          bidx = i2;
-        }
+    // the wave's point: largest excess, ties to the lowest index
+    const double wbest = wave_max(best);
+    unsigned long long tied = __ballot(best == wbest);
+    int src = __ffsll(tied) - 1, widx = __builtin_amdgcn_readlane(bidx, src);
+    for (tied &= tied - 1; tied && wbest > 0; tied &= tied - 1) {
+      const int l = __ffsll(tied) - 1, i = __builtin_amdgcn_readlane(bidx, l);
+      if (i < widx) {
+        widx = i;
+        src = l;
       }
     }
+    best = wbest;
+    for (int d = 0; d < 3; d++) bq[d] = lane_value(bq[d], src);
+    if (NW > 1) {
+      const int par = iter & 1;
+      double *se = s_e + par * 4 * NW;
+      int *si = s_i + par * NW;
+      if (lane == 0) {
+        se[4 * wid] = best;
+        for (int d = 0; d < 3; d++) se[4 * wid + 1 + d] = bq[d];
+        si[wid] = widx;
+      }
+      __syncthreads();
+      best = se[0];
+      widx = si[0];
+      int wb = 0;
+      for (int w = 1; w < NW; w++) {
+        const double e2 = se[4 * w];
+        const int i2 = si[w];
+        if (e2 > best || (e2 == best && i2 < widx)) {
+          best = e2;
+          widx = i2;
+          wb = w;
+        }
+      }
+      for (int d = 0; d < 3; d++) bq[d] = se[4 * wb + 1 + d];
+    }
     if (best <= kBallTol * b.r2 || best <= 0) break;
-    double bq[3];
-    get(bidx, bq);
     // the <= 15 candidates (subsets of the support) one per lane; the valid
     // one of smallest radius wins, ties to the lowest mask (the order a
     // sequential scan over masks would keep)
     DBall cb;
     const bool ok = candidate_ball(lane, ns, bq, sup, cb);
-    double key = ok ? cb.r2 : INFINITY;
-    int bestmask = lane;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const double k2 = __shfl_xor(key, o, kWave);
-      const int m2 = __shfl_xor(bestmask, o, kWave);
-      if (k2 < key || (k2 == key && m2 < bestmask)) {
-        key = k2;
-        bestmask = m2;
-      }
-    }
-    if (!(key < INFINITY)) break;  // numerically degenerate; keep the current ball
+    const double key = ok ? cb.r2 : INFINITY;
+    const double kmin = row0_min(key);
+    if (!(kmin < INFINITY)) break;  // numerically degenerate; keep the current ball
+    const int bestmask = __ffsll(__ballot(key == kmin)) - 1;
     DBall bestb;
-    candidate_ball(bestmask, ns, bq, sup, bestb);
+    for (int d = 0; d < 3; d++) bestb.c[d] = lane_value(cb.c[d], bestmask);
+    bestb.r2 = kmin;
     double nsup[4][3];
     const int k = gather_support(bestmask, bq, sup, nsup);
 #pragma unroll
@@ -222,22 +236,22 @@ __device__ DBall block_minball(Get get, Scan scan, double *s_e, int *s_i) {
 #pragma unroll
       for (int d = 0; d < 3; d++) sup[s2][d] = nsup[s2][d];
     ns = k;
-    if (bestb.r2 <= b.r2) {
-      b = bestb;
-      break;
-    }
+    const bool grew = bestb.r2 > b.r2;
     b = bestb;
+    if (!grew) break;
   }
   return b;
 }
 
-// One wave, points 0..n-1 from get(), lane-strided scan.
+// One wave, points 0..n-1 (n > 0) from get(), lane-strided scan.
 template <class Get>
 __device__ DBall wave_minball(int n, Get get) {
   const int lane = threadIdx.x & (kWave - 1);
+  double p0[3];
+  get(0, p0);
   return block_minball<1>(
-      get,
-      [&](auto f) {
+      p0,
+      [&](const DBall &, auto f) {
         for (int i = lane; i < n; i += kWave) {
           double q[3];
           get(i, q);

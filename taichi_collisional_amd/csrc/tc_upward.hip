@@ -215,8 +215,8 @@ __global__ __launch_bounds__(256) void k_m2m(CellsDev c, BodiesDev b, const int 
   double *s_td = smem;                                            // t-design
   double(*s_g)[4] = reinterpret_cast<double(*)[4]>(smem + 192);  // grandchild (X, R)
   double(*s_p)[kStage] = reinterpret_cast<double(*)[kStage]>(smem + 192 + 256);
-  __shared__ int s_pre[9], s_base[8], s_leaf[8], s_body[8], s_nstage;
-  __shared__ double s_e[2 * NW];
+  __shared__ int s_pre[9], s_base[8], s_leaf[8], s_body[8], s_gi[64], s_nstage, s_ng;
+  __shared__ double s_e[8 * NW];
   __shared__ int s_i[2 * NW];
   const int tid = threadIdx.x;
   const int ci = ids ? ids[blockIdx.x] : ls + blockIdx.x;
@@ -265,19 +265,21 @@ __global__ __launch_bounds__(256) void k_m2m(CellsDev c, BodiesDev b, const int 
       }
       s_pre[nch] = pre;
       s_nstage = nbs;
+      s_ng = ng;
     }
     __syncthreads();
     const bool staged = s_nstage <= kStage;
     // grandchildren's balls of the internal children: thread 8 k + j takes
-    // grandchild j of child k
+    // grandchild j of child k; s_gi: the index of its sphere's first point
     if (tid < 64) {
       const int k = tid >> 3, j = tid & 7;
       if (k < nch && !s_leaf[k] && j < s_nc2[k]) {
-        const int g = s_g0[k] + j;
-        s_g[s_base[k] + j][0] = c.X[3 * g];
-        s_g[s_base[k] + j][1] = c.X[3 * g + 1];
-        s_g[s_base[k] + j][2] = c.X[3 * g + 2];
-        s_g[s_base[k] + j][3] = c.R[g];
+        const int g = s_g0[k] + j, o = s_base[k] + j;
+        s_g[o][0] = c.X[3 * g];
+        s_g[o][1] = c.X[3 * g + 1];
+        s_g[o][2] = c.X[3 * g + 2];
+        s_g[o][3] = c.R[g];
+        s_gi[o] = s_pre[k] + 64 * j;
       }
     }
     // bodies of the leaf children, all of them strided over the block
@@ -291,40 +293,66 @@ __global__ __launch_bounds__(256) void k_m2m(CellsDev c, BodiesDev b, const int 
         s_p[2][i] = b.z[bi];
       }
     __syncthreads();
-    // point `local` of child k, in the order the reference enumerates them
-    auto point = [&](int k, int local, double *q) {
-      if (s_leaf[k]) {
-        if (staged) {
-          const int o = s_base[k] + local;
-          q[0] = s_p[0][o];
-          q[1] = s_p[1][o];
-          q[2] = s_p[2][o];
-        } else {
-          const int bi = s_body[k] + local;
-          q[0] = b.x[bi];
-          q[1] = b.y[bi];
-          q[2] = b.z[bi];
-        }
+    const int lane = tid & (kWave - 1), wid = tid / kWave, ng = s_ng;
+    // the lane's design point (64 points a sphere: one per lane)
+    const double td[3] = {s_td[3 * lane], s_td[3 * lane + 1], s_td[3 * lane + 2]};
+    auto sphere_point = [&](int g, double *q) {
+      const double Rg = s_g[g][3];
+      for (int d = 0; d < 3; d++) q[d] = s_g[g][d] + Rg * td[d];
+    };
+    auto leaf_body = [&](int k, int local, double *q) {
+      if (staged) {
+        const int o = s_base[k] + local;
+        q[0] = s_p[0][o];
+        q[1] = s_p[1][o];
+        q[2] = s_p[2][o];
       } else {
-        const int g = s_base[k] + (local >> 6), t = local & 63;
-        const double Rg = s_g[g][3];
-        for (int d = 0; d < 3; d++) q[d] = s_g[g][d] + Rg * s_td[3 * t + d];
+        const int bi = s_body[k] + local;
+        q[0] = b.x[bi];
+        q[1] = b.y[bi];
+        q[2] = b.z[bi];
       }
     };
+    // point 0, in the order the reference enumerates them: of the first child
+    // that has any, its first body or its first sphere's first design point
+    double p0[3];
+    int k0 = 0;
+    while (k0 < nch - 1 && s_pre[k0 + 1] == 0) k0++;
+    if (s_leaf[k0]) {
+      leaf_body(k0, 0, p0);
+    } else {
+      for (int d = 0; d < 3; d++) p0[d] = s_g[0][d] + s_g[0][3] * s_td[d];
+    }
     DBall ball = block_minball<NW>(
-        [&](int i, double *q) {
-          int k = 0;
-          while (k < nch - 1 && i >= s_pre[k + 1]) k++;
-          point(k, i - s_pre[k], q);
-        },
-        [&](auto f) {
+        p0,
+        [&](const DBall &bl, auto f) {
           for (int k = 0; k < nch; k++) {
-            const int p0 = s_pre[k], cnt = s_pre[k + 1] - p0;
+            if (!s_leaf[k]) continue;
+            const int i0 = s_pre[k], cnt = s_pre[k + 1] - i0;
             for (int l = tid; l < cnt; l += NW * kWave) {
               double q[3];
-              point(k, l, q);
-              f(p0 + l, q);
+              leaf_body(k, l, q);
+              f(i0 + l, q);
             }
+          }
+          // a sphere well inside the ball (|X_g - c| + 1.2 R_g < r, no design
+          // point being longer than 1.197, with a margin far above the
+          // rounding of its points) has no point of positive excess: lane g
+          // tests sphere g, and the waves share the rest
+          bool out = false;
+          if (lane < ng) {
+            double d2 = 0;
+            for (int d = 0; d < 3; d++) d2 += (s_g[lane][d] - bl.c[d]) * (s_g[lane][d] - bl.c[d]);
+            const double m = sqrt(bl.r2) - 1.2 * s_g[lane][3];
+            out = !(m > 0 && d2 < m * m * (1 - 1e-6));
+          }
+          unsigned long long todo = __ballot(out);
+          for (int r = 0; todo; todo &= todo - 1, r++) {
+            if ((r & (NW - 1)) != wid) continue;
+            const int g = __ffsll(todo) - 1;
+            double q[3];
+            sphere_point(g, q);
+            f(s_gi[g] + lane, q);
           }
         },
         s_e, s_i);
