@@ -22,122 +22,99 @@ struct DBall {
   double r2;
 };
 
-// Smallest ball with the k (1..4) points p[0..k-1] on its boundary: the
-// circumcentre in their affine hull.  Loops have fixed bounds with guards so
-// every array stays in registers; the arithmetic is that of the CPU oracle.
-__device__ inline bool circumball_dev(const double (&p)[4][3], int k, DBall &b) {
+// Candidate masks of a refinement step: lane l < 16 tries the support points
+// whose bits are set in l (at most three).  slot[i]: the i-th of them, 4 where
+// there is none.
+struct BallLane {
+  int slot[3], count;
+};
+__device__ __forceinline__ BallLane ball_lane(int lane) {
+  BallLane t = {{4, 4, 4}, 0};
+#pragma unroll
+  for (int s = 0; s < 4; s++)
+    if (lane & (1 << s)) {
+      if (t.count == 0) t.slot[0] = s;
+      if (t.count == 1) t.slot[1] = s;
+      if (t.count == 2) t.slot[2] = s;
+      t.count++;
+    }
+  return t;
+}
+
+// Candidate `lane` of one refinement step: the smallest ball with bq and the
+// lane's support points on its boundary (the circumcentre in their affine
+// hull), valid when it also holds the other support points.
+//
+// One straight path for one to four points, so that the lanes' different
+// candidates run side by side: a missing point is bq itself (its edge vector
+// is zero) and its row of the Gram matrix the unit row, with which the 3 x 3
+// solution takes, bit for bit, the values of the smaller system.
+__device__ __forceinline__ bool candidate_ball(int lane, const BallLane &t, int ns,
+                                               const double (&bq)[3], const double (&sup)[4][3],
+                                               DBall &cb) {
 #pragma clang fp contract(off)
-  if (k == 1) {
-    for (int d = 0; d < 3; d++) b.c[d] = p[0][d];
-    b.r2 = 0;
-    return true;
-  }
-  double v[3][3];
+  double v[3][3], A[3][3], rhs[3];
 #pragma unroll
-  for (int i = 1; i < 4; i++)
+  for (int i = 0; i < 3; i++)
 #pragma unroll
-    for (int d = 0; d < 3; d++) v[i - 1][d] = i < k ? p[i][d] - p[0][d] : 0.0;
-  const int q = k - 1;
-  double A[3][3], rhs[3];
+    for (int d = 0; d < 3; d++) {
+      double p = bq[d];
+#pragma unroll
+      for (int s = i; s < 4; s++) p = t.slot[i] == s ? sup[s][d] : p;
+      v[i][d] = p - bq[d];
+    }
 #pragma unroll
   for (int i = 0; i < 3; i++) {
 #pragma unroll
-    for (int j = 0; j < 3; j++) A[i][j] = v[i][0] * v[j][0] + v[i][1] * v[j][1] + v[i][2] * v[j][2];
+    for (int j = 0; j <= i; j++)
+      A[i][j] = A[j][i] = v[i][0] * v[j][0] + v[i][1] * v[j][1] + v[i][2] * v[j][2];
     rhs[i] = 0.5 * A[i][i];
+    A[i][i] = i < t.count ? A[i][i] : 1.0;
   }
-  double lam[3] = {0, 0, 0};
-  if (q == 1) {
-    if (!(A[0][0] > 0)) return false;
-    lam[0] = 0.5;
-  } else if (q == 2) {
-    double det = A[0][0] * A[1][1] - A[0][1] * A[1][0];
-    if (!(fabs(det) > 1e-13 * A[0][0] * A[1][1])) return false;
-    lam[0] = (rhs[0] * A[1][1] - A[0][1] * rhs[1]) / det;
-    lam[1] = (A[0][0] * rhs[1] - rhs[0] * A[1][0]) / det;
-  } else {
-    double c00 = A[1][1] * A[2][2] - A[1][2] * A[2][1];
-    double c01 = A[1][2] * A[2][0] - A[1][0] * A[2][2];
-    double c02 = A[1][0] * A[2][1] - A[1][1] * A[2][0];
-    double det = A[0][0] * c00 + A[0][1] * c01 + A[0][2] * c02;
-    if (!(fabs(det) > 1e-13 * A[0][0] * A[1][1] * A[2][2])) return false;
-    double inv[3][3];
-    inv[0][0] = c00;
-    inv[0][1] = A[0][2] * A[2][1] - A[0][1] * A[2][2];
-    inv[0][2] = A[0][1] * A[1][2] - A[0][2] * A[1][1];
-    inv[1][0] = c01;
-    inv[1][1] = A[0][0] * A[2][2] - A[0][2] * A[2][0];
-    inv[1][2] = A[0][2] * A[1][0] - A[0][0] * A[1][2];
-    inv[2][0] = c02;
-    inv[2][1] = A[0][1] * A[2][0] - A[0][0] * A[2][1];
-    inv[2][2] = A[0][0] * A[1][1] - A[0][1] * A[1][0];
+  const double c00 = A[1][1] * A[2][2] - A[1][2] * A[2][1];
+  const double c01 = A[1][2] * A[2][0] - A[1][0] * A[2][2];
+  const double c02 = A[1][0] * A[2][1] - A[1][1] * A[2][0];
+  const double det = A[0][0] * c00 + A[0][1] * c01 + A[0][2] * c02;
+  bool ok = lane < (1 << ns) && t.count <= 3 &&
+            fabs(det) > 1e-13 * A[0][0] * A[1][1] * A[2][2];
+  double inv[3][3];
+  inv[0][0] = c00;
+  inv[0][1] = A[0][2] * A[2][1] - A[0][1] * A[2][2];
+  inv[0][2] = A[0][1] * A[1][2] - A[0][2] * A[1][1];
+  inv[1][0] = c01;
+  inv[1][1] = A[0][0] * A[2][2] - A[0][2] * A[2][0];
+  inv[1][2] = A[0][2] * A[1][0] - A[0][0] * A[1][2];
+  inv[2][0] = c02;
+  inv[2][1] = A[0][1] * A[2][0] - A[0][0] * A[2][1];
+  inv[2][2] = A[0][0] * A[1][1] - A[0][1] * A[1][0];
+  double lam[3];
 #pragma unroll
-    for (int i = 0; i < 3; i++)
-      lam[i] = (inv[i][0] * rhs[0] + inv[i][1] * rhs[1] + inv[i][2] * rhs[2]) / det;
-  }
+  for (int i = 0; i < 3; i++)
+    lam[i] = (inv[i][0] * rhs[0] + inv[i][1] * rhs[1] + inv[i][2] * rhs[2]) / det;
 #pragma unroll
   for (int d = 0; d < 3; d++) {
-    double c = p[0][d];
+    double c = bq[d];
 #pragma unroll
-    for (int i = 0; i < 3; i++)
-      if (i < q) c += lam[i] * v[i][d];
-    b.c[d] = c;
+    for (int i = 0; i < 3; i++) c += lam[i] * v[i][d];
+    cb.c[d] = c;
   }
-  double r2 = 0;
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    if (i >= k) continue;
+  auto dist2 = [&](const double *p) {
     double dd = 0;
 #pragma unroll
-    for (int d = 0; d < 3; d++) dd += (p[i][d] - b.c[d]) * (p[i][d] - b.c[d]);
-    r2 = fmax(r2, dd);
-  }
-  b.r2 = r2;
-  return true;
-}
-
-// Points bq, then the support points selected by mask, in support order.
-__device__ inline int gather_support(int mask, const double (&bq)[3], const double (&sup)[4][3],
-                                     double (&p)[4][3]) {
-#pragma unroll
-  for (int d = 0; d < 3; d++) {
-    p[0][d] = bq[d];
-    p[1][d] = p[2][d] = p[3][d] = 0.0;
-  }
-  int k = 1;
+    for (int d = 0; d < 3; d++) dd += (p[d] - cb.c[d]) * (p[d] - cb.c[d]);
+    return dd;
+  };
+  double ds[4], r2 = dist2(bq);
 #pragma unroll
   for (int s = 0; s < 4; s++) {
-    if (mask & (1 << s)) {
-#pragma unroll
-      for (int d = 0; d < 3; d++) {
-        const double v = sup[s][d];
-        if (k == 1) p[1][d] = v;
-        if (k == 2) p[2][d] = v;
-        if (k == 3) p[3][d] = v;
-      }
-      k++;
-    }
+    ds[s] = dist2(sup[s]);
+    if (lane & (1 << s)) r2 = fmax(r2, ds[s]);
   }
-  return k;
-}
-
-// Candidate `mask` of one refinement step: the ball through bq and the
-// selected support points, valid when it also holds the other support points.
-__device__ inline bool candidate_ball(int mask, int ns, const double (&bq)[3],
-                                      const double (&sup)[4][3], DBall &cb) {
-#pragma clang fp contract(off)
-  if (mask >= (1 << ns) || __popc(mask) > 3) return false;
-  double pts[4][3];
-  const int k = gather_support(mask, bq, sup, pts);
-  if (!circumball_dev(pts, k, cb)) return false;
 #pragma unroll
-  for (int s = 0; s < 4; s++) {
-    if (s >= ns || (mask & (1 << s))) continue;
-    double dd = 0;
-#pragma unroll
-    for (int d = 0; d < 3; d++) dd += (sup[s][d] - cb.c[d]) * (sup[s][d] - cb.c[d]);
-    if (dd > cb.r2 * (1 + 1e-12)) return false;
-  }
-  return true;
+  for (int s = 0; s < 4; s++)
+    if (s < ns && !(lane & (1 << s)) && ds[s] > r2 * (1 + 1e-12)) ok = false;
+  cb.r2 = r2;
+  return ok;
 }
 
 constexpr double kBallTol = 1e-13;
@@ -155,16 +132,18 @@ constexpr double kBallTol = 1e-13;
 // after another.  So the reductions are register moves (DPP) instead of
 // shuffles through the LDS unit, the point of largest excess travels with its
 // excess instead of being looked up again, and the winning candidate's ball
-// is read from the lane that solved it.
+// is read from the lane that solved it.  Plummer N = 2^20, p = 12: leaves 254
+// -> 157 us, the twelve internal levels 1,000 -> 450 us, a top level 65 -> 29 us.
 template <int NW, class Scan>
 __device__ DBall block_minball(const double (&p0)[3], Scan scan, double *s_e, int *s_i) {
 #pragma clang fp contract(off)
   const int lane = threadIdx.x & (kWave - 1);
   const int wid = threadIdx.x / kWave;
+  const BallLane mine = ball_lane(lane);
   DBall b;
   double sup[4][3];
   int ns = 1;
-  for (int d = 0; d < 3; d++) b.c[d] = sup[0][d] = p0[d];
+  for (int d = 0; d < 3; d++) b.c[d] = sup[0][d] = sup[1][d] = sup[2][d] = sup[3][d] = p0[d];
   b.r2 = 0;
   for (int iter = 0; iter < 10000; iter++) {
     double best = -1, bq[3] = {0, 0, 0};
@@ -221,7 +200,7 @@ __device__ DBall block_minball(const double (&p0)[3], Scan scan, double *s_e, in
     // one of smallest radius wins, ties to the lowest mask (the order a
     // sequential scan over masks would keep)
     DBall cb;
-    const bool ok = candidate_ball(lane, ns, bq, sup, cb);
+    const bool ok = candidate_ball(lane, mine, ns, bq, sup, cb);
     const double key = ok ? cb.r2 : INFINITY;
     const double kmin = row0_min(key);
     if (!(kmin < INFINITY)) break;  // numerically degenerate; keep the current ball
@@ -229,8 +208,23 @@ __device__ DBall block_minball(const double (&p0)[3], Scan scan, double *s_e, in
     DBall bestb;
     for (int d = 0; d < 3; d++) bestb.c[d] = lane_value(cb.c[d], bestmask);
     bestb.r2 = kmin;
+    // the new support: bq, then the chosen points in support order
     double nsup[4][3];
-    const int k = gather_support(bestmask, bq, sup, nsup);
+    int k = 1;
+#pragma unroll
+    for (int d = 0; d < 3; d++)
+      nsup[0][d] = nsup[1][d] = nsup[2][d] = nsup[3][d] = bq[d];
+#pragma unroll
+    for (int s2 = 0; s2 < 4; s2++)
+      if (bestmask & (1 << s2)) {
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+          nsup[1][d] = k == 1 ? sup[s2][d] : nsup[1][d];
+          nsup[2][d] = k == 2 ? sup[s2][d] : nsup[2][d];
+          nsup[3][d] = k == 3 ? sup[s2][d] : nsup[3][d];
+        }
+        k++;
+      }
 #pragma unroll
     for (int s2 = 0; s2 < 4; s2++)
 #pragma unroll

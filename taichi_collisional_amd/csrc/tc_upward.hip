@@ -211,11 +211,18 @@ __global__ __launch_bounds__(256) void k_m2m(CellsDev c, BodiesDev b, const int 
   constexpr bool kPar = 16 * 16 * NT <= 60 * 1024;
   constexpr int kBall = 192 + 64 * 4 + 3 * kStage;       // doubles, ball phase
   constexpr int kTrans = kPar ? 2 * 8 * 2 * NT : 3 * 2 * NT;  // doubles, translation
-  __shared__ __attribute__((aligned(16))) double smem[kBall > kTrans ? kBall : kTrans];
+  // (each phase's own size where only one of them is compiled in)
+  constexpr int kSmem = !(kWhat & kUpMoments) ? ((kWhat & kUpGeom) ? kBall : 1)
+                        : !(kWhat & kUpGeom)  ? kTrans
+                        : kBall > kTrans      ? kBall
+                                              : kTrans;
+  __shared__ __attribute__((aligned(16))) double smem[kSmem];
   double *s_td = smem;                                            // t-design
   double(*s_g)[4] = reinterpret_cast<double(*)[4]>(smem + 192);  // grandchild (X, R)
   double(*s_p)[kStage] = reinterpret_cast<double(*)[kStage]>(smem + 192 + 256);
   __shared__ int s_pre[9], s_base[8], s_leaf[8], s_body[8], s_gi[64], s_nstage, s_ng;
+  // s_pi: the staged bodies' indices in the enumeration of points
+  __shared__ int s_pi[(kWhat & kUpGeom) ? kStage : 1];
   __shared__ double s_e[8 * NW];
   __shared__ int s_i[2 * NW];
   const int tid = threadIdx.x;
@@ -291,9 +298,10 @@ __global__ __launch_bounds__(256) void k_m2m(CellsDev c, BodiesDev b, const int 
         s_p[0][i] = b.x[bi];
         s_p[1][i] = b.y[bi];
         s_p[2][i] = b.z[bi];
+        s_pi[i] = s_pre[k] + (i - s_base[k]);
       }
     __syncthreads();
-    const int lane = tid & (kWave - 1), wid = tid / kWave, ng = s_ng;
+    const int lane = tid & (kWave - 1), wid = tid / kWave, ng = s_ng, nstage = s_nstage;
     // the lane's design point (64 points a sphere: one per lane)
     const double td[3] = {s_td[3 * lane], s_td[3 * lane + 1], s_td[3 * lane + 2]};
     auto sphere_point = [&](int g, double *q) {
@@ -326,13 +334,20 @@ __global__ __launch_bounds__(256) void k_m2m(CellsDev c, BodiesDev b, const int 
     DBall ball = block_minball<NW>(
         p0,
         [&](const DBall &bl, auto f) {
-          for (int k = 0; k < nch; k++) {
-            if (!s_leaf[k]) continue;
-            const int i0 = s_pre[k], cnt = s_pre[k + 1] - i0;
-            for (int l = tid; l < cnt; l += NW * kWave) {
-              double q[3];
-              leaf_body(k, l, q);
-              f(i0 + l, q);
+          if (staged) {
+            for (int i = tid; i < nstage; i += NW * kWave) {
+              const double q[3] = {s_p[0][i], s_p[1][i], s_p[2][i]};
+              f(s_pi[i], q);
+            }
+          } else {
+            for (int k = 0; k < nch; k++) {
+              if (!s_leaf[k]) continue;
+              const int i0 = s_pre[k], cnt = s_pre[k + 1] - i0;
+              for (int l = tid; l < cnt; l += NW * kWave) {
+                double q[3];
+                leaf_body(k, l, q);
+                f(i0 + l, q);
+              }
             }
           }
           // a sphere well inside the ball (|X_g - c| + 1.2 R_g < r, no design
