@@ -14,7 +14,7 @@ namespace tcfmm {
   int launch_l2l(int p, CellsDev c, int ls, int le, hipStream_t s);                           \
   int launch_l2l_ids(int p, CellsDev c, const int *ids, int nids, hipStream_t s);             \
   int launch_l2p(int p, CellsDev c, BodiesDev b, ResultsDev r, const int *leaf_ids,           \
-                 int nleaves, hipStream_t s);
+                 int nleaves, hipStream_t s, bool add);
 
 static_assert(TC_NSHARDS == 3, "the routing below names three shards");
 namespace sh0 {
@@ -56,8 +56,8 @@ int launch_l2l_ids(int p, CellsDev c, const int *ids, int nids, hipStream_t s) {
   TC_ROUTE(launch_l2l_ids(p, c, ids, nids, s))
 }
 int launch_l2p(int p, CellsDev c, BodiesDev b, ResultsDev r, const int *leaf_ids, int nleaves,
-               hipStream_t s) {
-  TC_ROUTE(launch_l2p(p, c, b, r, leaf_ids, nleaves, s))
+               hipStream_t s, bool add) {
+  TC_ROUTE(launch_l2p(p, c, b, r, leaf_ids, nleaves, s, add))
 }
 
 }  // namespace tcfmm

@@ -169,13 +169,16 @@ __device__ __forceinline__ void l2p_orders(double dx, double dy, double dz, doub
   }
 }
 
+// kAdd: into the results (which the caller cleared or already holds sums in);
+// otherwise every body's far-field results are written, zeros for bodies that
+// are not sinks, and nothing has to be cleared before.
+//
 // Up to p = 12 the kernel is held to three waves per SIMD (168 VGPRs; at
 // p = 12 that spills 14 of its 196, 60 bytes per lane, and still runs the
 // downward pass 0.02-0.08 ms sooner per 2^20-body evaluation than two waves).
-template <int P>
+template <int P, bool kAdd>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(P <= 12 ? 3 : 1))) void k_l2p(
-    CellsDev c, BodiesDev b, ResultsDev r,
-                                            const int *__restrict__ leaf_ids, int nleaves) {
+    CellsDev c, BodiesDev b, ResultsDev r, const int *__restrict__ leaf_ids, int nleaves) {
   constexpr int NT = nterm(P);
   constexpr int kHalf = kWave / 2;  // lanes per leaf: two leaves per wave
   __shared__ cplx cl[2][NT], cld[2][NT];
@@ -195,26 +198,35 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(P <= 12 ? 3 
     }
   }
   __syncthreads();
-  if (!on) return;
+  if (ci < 0) return;
   const int b0 = c.body[ci], nb = c.nbody[ci];
+  if (!on) {
+    if (!kAdd)
+      for (int i = b0 + u; i < b0 + nb; i += kHalf)
+        r.pot[i] = r.ax[i] = r.ay[i] = r.az[i] = r.jx[i] = r.jy[i] = r.jz[i] = 0.0;
+    return;
+  }
   const double X0 = c.X[3 * ci], X1 = c.X[3 * ci + 1], X2 = c.X[3 * ci + 2];
   for (int base = 0; base < nb; base += kHalf) {
     const int i = b0 + base + u;
     if (base + u >= nb) continue;
-    if (!(b.flags[i] & kSink)) continue;
+    if (!(b.flags[i] & kSink)) {
+      if (!kAdd) r.pot[i] = r.ax[i] = r.ay[i] = r.az[i] = r.jx[i] = r.jy[i] = r.jz[i] = 0.0;
+      continue;
+    }
     const double vx = -b.vx[i], vy = -b.vy[i], vz = -b.vz[i];
     const double dx = X0 - b.x[i], dy = X1 - b.y[i], dz = X2 - b.z[i];
     const double r2 = dx * dx + dy * dy + dz * dz;
     cplx y1[P + 1], y2[P + 1];
     L2PAcc a = {0, 0, 0, 0, 0, 0, {0, 0}, {0, 0}};
     l2p_orders<P, 0>(dx, dy, dz, r2, vx, vy, vz, cl[h], cld[h], y1, y2, a);
-    r.pot[i] += a.p00 + 2.0 * a.h00;
-    r.ax[i] -= a.p11.re;
-    r.ay[i] -= a.p11.im;
-    r.az[i] -= a.p10 + 2.0 * a.h10;
-    r.jx[i] -= a.d11.re;
-    r.jy[i] -= a.d11.im;
-    r.jz[i] -= a.d10 + 2.0 * a.e10;
+    r.pot[i] = (kAdd ? r.pot[i] : 0.0) + (a.p00 + 2.0 * a.h00);
+    r.ax[i] = (kAdd ? r.ax[i] : 0.0) - a.p11.re;
+    r.ay[i] = (kAdd ? r.ay[i] : 0.0) - a.p11.im;
+    r.az[i] = (kAdd ? r.az[i] : 0.0) - (a.p10 + 2.0 * a.h10);
+    r.jx[i] = (kAdd ? r.jx[i] : 0.0) - a.d11.re;
+    r.jy[i] = (kAdd ? r.jy[i] : 0.0) - a.d11.im;
+    r.jz[i] = (kAdd ? r.jz[i] : 0.0) - (a.d10 + 2.0 * a.e10);
   }
 }
 
@@ -223,8 +235,13 @@ static void l2l_go(CellsDev c, const int *ids, int ls, int ncell, hipStream_t s)
   hipLaunchKernelGGL(k_l2l<P>, dim3(2 * ncell), dim3(256), 0, s, c, ids, ls);
 }
 template <int P>
-static void l2p_go(CellsDev c, BodiesDev b, ResultsDev r, const int *ids, int n, hipStream_t s) {
-  hipLaunchKernelGGL(k_l2p<P>, dim3((n + 1) / 2), dim3(64), 0, s, c, b, r, ids, n);
+static void l2p_go(CellsDev c, BodiesDev b, ResultsDev r, const int *ids, int n, bool add,
+                   hipStream_t s) {
+  const dim3 g((n + 1) / 2), t(64);
+  if (add)
+    hipLaunchKernelGGL((k_l2p<P, true>), g, t, 0, s, c, b, r, ids, n);
+  else
+    hipLaunchKernelGGL((k_l2p<P, false>), g, t, 0, s, c, b, r, ids, n);
 }
 
 int launch_l2l(int p, CellsDev c, int ls, int le, hipStream_t s) {
@@ -264,13 +281,13 @@ int launch_l2l_ids(int p, CellsDev c, const int *ids, int nids, hipStream_t s) {
 }
 
 int launch_l2p(int p, CellsDev c, BodiesDev b, ResultsDev r, const int *leaf_ids, int nleaves,
-               hipStream_t s) {
+               hipStream_t s, bool add) {
   if (nleaves <= 0) return 0;
   switch (p) {
 #define TC_CASE(P)\
   case P:\
     if constexpr (in_shard(P, TC_SHARD)) {\
-      l2p_go<P>(c, b, r, leaf_ids, nleaves, s);\
+      l2p_go<P>(c, b, r, leaf_ids, nleaves, add, s);\
       return 0;\
     } else {\
       return -1;\

@@ -78,8 +78,8 @@ static int ensure_cells(tc_context *ctx, int nc, int keep) {
 }
 
 // Tree levels are queued in batches without host reads (TreeState on the
-// device holds the level range and counts); after a batch one small copy says
-// whether the last level had no children.  A level whose children do not fit
+// device holds the level range and counts); a batch's last level reports the
+// state to pinned memory, which says whether it had no children.  A level whose children do not fit
 // the cell arrays ends the build with a flag and what it needed: the arrays
 // grow and the build starts again from the root (a new workload's first
 // evaluation, or a tree that a new root shift makes larger).
@@ -93,7 +93,9 @@ static int build_tree(tc_context *ctx, int n) {
     return e;
   TC_CHECK(ctx->tree_state.ensure(sizeof(TreeState)));
   TC_CHECK(ctx->h_tree.ensure(sizeof(TreeState) / sizeof(int)));
-  TreeState *hst = reinterpret_cast<TreeState *>(ctx->h_tree.p);
+  const TreeState *hst = reinterpret_cast<const TreeState *>(ctx->h_tree.p);
+  TreeState *dst = nullptr;  // the same memory as kernels address it
+  TC_CHECK(hipHostGetDevicePointer((void **)&dst, ctx->h_tree.p, 0));
   for (int attempt = 0;; attempt++) {
     if (attempt > 16) {
       ctx->err = "tree build: cell arrays keep overflowing";
@@ -103,11 +105,8 @@ static int build_tree(tc_context *ctx, int n) {
     TC_CHECK(ctx->split_offs.ensure(sizeof(int) * 8 * (size_t)cap));
     TC_CHECK(ctx->split_nch.ensure(sizeof(int) * 2 * (size_t)cap));
     TC_CHECK(ctx->split_scan.ensure(sizeof(int) * 2 * (size_t)cap));
-    std::memset(hst, 0, sizeof(TreeState));
-    hst->ls = 0;
-    hst->le = ctx->ncl;  // one root, or one per cluster of a forest
-    TC_CHECK(hipMemcpyAsync(ctx->tree_state.p, hst, sizeof(TreeState), hipMemcpyHostToDevice, s));
-    launch_root(cells_of(ctx), n, ctx->tp.as<TreeParams>(), s,
+    // one root, or one per cluster of a forest
+    launch_root(cells_of(ctx), n, ctx->tp.as<TreeParams>(), ctx->tree_state.as<TreeState>(), s,
                 ctx->ncl > 1 ? ctx->cl_start.as<int>() : nullptr, ctx->ncl);
     int queued = 0, batch = std::max(4, ctx->tree_levels + 1);
     for (;;) {
@@ -115,9 +114,7 @@ static int build_tree(tc_context *ctx, int n) {
         launch_tree_level(cells_of(ctx), b, ctx->tree_state.as<TreeState>(), ncrit, cap,
                           ctx->split_offs.as<int>(), ctx->split_nch.as<int>(),
                           ctx->split_scan.as<int>(), ctx->tp.as<TreeParams>(),
-                          ctx->leaf_ids.as<int>(), s);
-      TC_CHECK(hipMemcpyAsync(hst, ctx->tree_state.p, sizeof(TreeState), hipMemcpyDeviceToHost,
-                              s));
+                          ctx->leaf_ids.as<int>(), i == batch - 1 ? dst : nullptr, s);
       TC_CHECK(spin_wait(ctx, s));
       if (hst->done || hst->overflow) break;
       if (queued > 4 * kMaxTreeLevels) {
@@ -171,17 +168,16 @@ static int upward(tc_context *ctx, int how = kUpwardWhole) {
   int p = ctx->cfg.p;
   int nc = ctx->st.ncells;
   size_t NT = (size_t)nterm(p);
-  hipStream_t sz = s;  // where the moments are cleared
   if (how == kUpwardErrMac) {
     TC_CHECK(hipEventRecord(ctx->ev[12], s));  // the tree
     TC_CHECK(hipStreamWaitEvent(s2, ctx->ev[12], 0));
-    sz = s2;
   }
-  TC_CHECK(hipMemsetAsync(ctx->cM.p, 0, sizeof(double) * NT * nc, sz));
-  TC_CHECK(hipMemsetAsync(ctx->cMd.p, 0, sizeof(double) * NT * nc, sz));
-  TC_CHECK(hipMemsetAsync(ctx->cL.p, 0, sizeof(double) * NT * nc, sz));
-  TC_CHECK(hipMemsetAsync(ctx->cLd.p, 0, sizeof(double) * NT * nc, sz));
-  TC_CHECK(hipMemsetAsync(ctx->csink.p, 0, nc, sz));
+  if (how == kUpwardWhole) {
+    // kUpAll adds; the parts of the other arrangements write
+    for (DBuf *q : {&ctx->cM, &ctx->cMd, &ctx->cL, &ctx->cLd})
+      TC_CHECK(hipMemsetAsync(q->p, 0, sizeof(double) * NT * nc, s));
+    TC_CHECK(hipMemsetAsync(ctx->csink.p, 0, nc, s));
+  }
   CellsDev c = cells_of(ctx);
   BodiesDev b = bodies_of(ctx);
   const int L = (int)ctx->level_start.size() - 1;
@@ -227,19 +223,16 @@ static int upward_min(tc_context *ctx) {
 }
 
 // Breadth-first dual traversal from (root, root).  Steps are queued in
-// batches without reading counts back (TravState holds them on the device);
-// after a batch one small copy says whether the frontier is empty.  A step
+// batches without reading counts back (TravState holds them on the device); a
+// batch's last step reports the state to pinned memory, which says whether the
+// frontier is empty.  A step
 // whose output would not fit its buffer ends the walk with a flag and what it
 // needed: the buffers then grow and the walk starts again (in practice only
 // on the first evaluation of a workload).
-__global__ void k_root_pairs(int2 *__restrict__ f, int ncl) {
-  const int k = blockIdx.x * 256 + threadIdx.x;
-  if (k < ncl) f[k] = make_int2(k, k);
-}
-
 static int traverse(tc_context *ctx, int n, const MacArgs &mac) {
   hipStream_t s = ctx->stream;
-  TravState *hst = reinterpret_cast<TravState *>(ctx->h_pin + 40);
+  const TravState *hst = reinterpret_cast<const TravState *>(ctx->h_pin + 40);
+  TravState *dst = reinterpret_cast<TravState *>(ctx->h_pin_dev + 40);
   static_assert(sizeof(TravState) <= 12 * sizeof(int), "pinned slots 40..51 (52, 53: P2P pairs)");
   TC_CHECK(ctx->tstate.ensure(sizeof(TravState)));
   TC_CHECK(ctx->tblk.ensure(sizeof(int) * 6 * kTravBlocks));
@@ -260,11 +253,7 @@ static int traverse(tc_context *ctx, int n, const MacArgs &mac) {
     const long long cm = cap(ctx->m2l), cp = cap(ctx->p2p),
                     cf = std::min({cap(ctx->front_a), cap(ctx->front_b),
                                    (long long)std::min<size_t>(ctx->tcls.bytes, 0x7fffffff)});
-    std::memset(hst, 0, sizeof(TravState));
-    hst->nin[0] = ctx->ncl;  // the root pair (0, 0), or (k, k) for every cluster
-    TC_CHECK(hipMemcpyAsync(ctx->tstate.p, hst, sizeof(TravState), hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_root_pairs, dim3((ctx->ncl + 255) / 256), dim3(256), 0, s,
-                       ctx->front_a.as<int2>(), ctx->ncl);
+    launch_root_pairs(ctx->front_a.as<int2>(), ctx->ncl, ctx->tstate.as<TravState>(), s);
     int k = 0, batch = std::max(8, known + 1);
     for (;;) {
       for (int i = 0; i < batch; i++, k++) {
@@ -277,9 +266,8 @@ static int traverse(tc_context *ctx, int n, const MacArgs &mac) {
         a.cls = ctx->tcls.as<unsigned char>();
         a.mac = mac;
         launch_trav_step(cells_of(ctx), a, ctx->tstate.as<TravState>(), (int)odd,
-                         ctx->tblk.as<int>(), cm, cp, cf, s);
+                         ctx->tblk.as<int>(), cm, cp, cf, i == batch - 1 ? dst : nullptr, s);
       }
-      TC_CHECK(hipMemcpyAsync(hst, ctx->tstate.p, sizeof(TravState), hipMemcpyDeviceToHost, s));
       TC_CHECK(spin_wait(ctx, s));
       if (hst->overflow || hst->nin[k & 1] == 0) break;
       if (k > 100000) {
@@ -309,13 +297,12 @@ static int traverse(tc_context *ctx, int n, const MacArgs &mac) {
 // group (target, source) pairs by target: stable radix sort + run bounds
 // (second: on near_stream with its own sort scratch, so that two lists are
 // grouped at once)
+// chunks (or null): receives the M2L chunk counts of the cells
 static int build_csr(tc_context *ctx, const int2 *pairs, int npairs, DBuf &cnt, DBuf &off,
-                     DBuf &src, bool second = false) {
+                     DBuf &src, bool second = false, int *chunks = nullptr) {
   hipStream_t s = second ? ctx->near_stream : ctx->stream;
   DBuf *sc = second ? ctx->gsort2 : ctx->gsort1;  // target keys in/out, sources in, temp
   int nc = ctx->st.ncells;
-  TC_CHECK(hipMemsetAsync(cnt.p, 0, sizeof(int) * (nc + 1), s));
-  TC_CHECK(hipMemsetAsync(off.p, 0, sizeof(int) * (nc + 1), s));
   size_t m = (size_t)std::max(npairs, 1);
   TC_CHECK(src.ensure(sizeof(int) * m));
   TC_CHECK(sc[0].ensure(sizeof(int) * m));
@@ -325,15 +312,10 @@ static int build_csr(tc_context *ctx, const int2 *pairs, int npairs, DBuf &cnt, 
   int bits = 1;
   while ((1 << bits) < nc) bits++;
   if (launch_group_pairs(pairs, npairs, bits, nc, sc[0].as<int>(), sc[1].as<int>(),
-                         sc[2].as<int>(), src.as<int>(), off.as<int>(), cnt.as<int>(), sc[3].p,
-                         sc[3].bytes, s))
+                         sc[2].as<int>(), src.as<int>(), off.as<int>(), cnt.as<int>(), chunks,
+                         sc[3].p, sc[3].bytes, s))
     return -4;
   return 0;
-}
-
-__global__ void k_chunk_counts(const int *__restrict__ cnt, int n, int *__restrict__ out) {
-  int i = blockIdx.x * 256 + threadIdx.x;
-  if (i <= n) out[i] = i < n ? (cnt[i] + 63) / 64 : 0;
 }
 
 static int build_lists(tc_context *ctx, int &nchunks) {
@@ -350,12 +332,10 @@ static int build_lists(tc_context *ctx, int &nchunks) {
   TC_CHECK(hipMemcpyAsync(ctx->h_pcnt.p, ctx->p2p_cnt.p, sizeof(int) * nc, hipMemcpyDeviceToHost,
                           ctx->near_stream));
   TC_CHECK(hipEventRecord(ctx->ev[15], ctx->near_stream));
-  if (int e = build_csr(ctx, ctx->m2l.as<int2>(), (int)ctx->st.n_m2l, ctx->m2l_cnt, ctx->m2l_off,
-                        ctx->m2l_src))
-    return e;
   // chunks of <= 64 sources per target for M2L
-  hipLaunchKernelGGL(k_chunk_counts, dim3((nc + 1 + 255) / 256), dim3(256), 0, s,
-                     ctx->m2l_cnt.as<int>(), nc, ctx->m2l_cur.as<int>());
+  if (int e = build_csr(ctx, ctx->m2l.as<int2>(), (int)ctx->st.n_m2l, ctx->m2l_cnt, ctx->m2l_off,
+                        ctx->m2l_src, false, ctx->m2l_cur.as<int>()))
+    return e;
   if (launch_scan(ctx->m2l_cur.as<int>(), ctx->m2l_coff.as<int>(), nc + 1, ctx->scan_tmp.p,
                   ctx->scan_tmp.bytes, s))
     return -4;
@@ -501,7 +481,8 @@ static int copy_acc_old(tc_context *ctx, int n, double *out) {
 }
 
 // Bounds, keys, sort, gather into tree order, cells (buildTree,
-// build_tree.h:239-487); the root shift is whatever ctx->dshift holds.
+// build_tree.h:239-487); the root shift is ctx->shift (a forest: one per
+// cluster, in ctx->dshift).
 static int sort_and_build(tc_context *ctx, int n, const double *x, const double *v,
                           const double *m, const unsigned char *flags) {
   hipStream_t s = ctx->stream;
@@ -512,7 +493,7 @@ static int sort_and_build(tc_context *ctx, int n, const double *x, const double 
     launch_cluster_ids(ctx->cl_start.as<int>(), ctx->ncl, n, ctx->cl_id.as<int>(), s);
   } else {
     launch_bounds(x, n, ctx->part.as<double>(), 1024, ctx->tp.as<TreeParams>(),
-                  ctx->dshift.as<double>(), s);
+                  ctx->shift, s);
   }
   launch_morton(x, n, ctx->tp.as<TreeParams>(), ctx->key_hi.as<uint64_t>(),
                 ctx->key_a.as<uint64_t>(), ctx->val_a.as<int>(), s,
@@ -714,9 +695,6 @@ static int eval_device(tc_context *ctx, int n, const double *x, const double *v,
     } else {
       for (int d = 0; d < 3; d++) u[d] = ctx->rng.next() - 0.5;
     }
-    // through pinned memory: a copy from pageable memory is staged and holds the host
-    std::memcpy(ctx->h_pin + 24, u, sizeof(u));
-    TC_CHECK(hipMemcpyAsync(ctx->dshift.p, ctx->h_pin + 24, sizeof(u), hipMemcpyHostToDevice, s));
   }
   std::memcpy(ctx->shift, u, sizeof(u));
   TC_CHECK(hipEventRecord(ctx->ev[0], s));
@@ -803,13 +781,10 @@ static int eval_device(tc_context *ctx, int n, const double *x, const double *v,
   // the tree and the P2P list (already queued on that stream)
   hipStream_t s2 = ctx->near_stream;
   ResultsDev r = results_of(ctx);
-  for (double *q : {r.pot, r.ax, r.ay, r.az, r.jx, r.jy, r.jz})
-    TC_CHECK(hipMemsetAsync(q, 0, sizeof(double) * n, s2));
   TC_CHECK(ctx->p2p_ranges.ensure(sizeof(int2) * (size_t)std::max<long long>(ctx->st.n_p2p_cells, 1)));
   TC_CHECK(ctx->npairs.ensure(sizeof(unsigned long long)));
-  TC_CHECK(hipMemsetAsync(ctx->npairs.p, 0, sizeof(unsigned long long), s2));
-  launch_p2p_ranges(cells_of(ctx), ctx->p2p_src.as<int>(), (int)ctx->st.n_p2p_cells,
-                    ctx->p2p_ranges.as<int2>(), s2);
+  launch_p2p_setup(cells_of(ctx), ctx->p2p_src.as<int>(), (int)ctx->st.n_p2p_cells,
+                   ctx->p2p_ranges.as<int2>(), r, n, ctx->npairs.as<unsigned long long>(), s2);
   // the GPU runs M2L while the host builds the P2P work items
   if (int e = build_p2p_items(ctx)) return e;
   TC_CHECK(hipEventRecord(ctx->ev[5], s));
@@ -828,19 +803,19 @@ static int eval_device(tc_context *ctx, int n, const double *x, const double *v,
   ResultsDev rf = {ctx->fpot.as<double>(), ctx->fax.as<double>(), ctx->fay.as<double>(),
                    ctx->faz.as<double>(), ctx->fjx.as<double>(), ctx->fjy.as<double>(),
                    ctx->fjz.as<double>()};
-  for (double *q : {rf.pot, rf.ax, rf.ay, rf.az, rf.jx, rf.jy, rf.jz})
-    TC_CHECK(hipMemsetAsync(q, 0, sizeof(double) * n, s));
   int L = (int)ctx->level_start.size() - 1;
   for (int l = 0; l < L; l++)
     launch_l2l(cfg.p, cells_of(ctx), ctx->level_start[l], ctx->level_start[l + 1], s);
-  launch_l2p(cfg.p, cells_of(ctx), bodies_of(ctx), rf, ctx->leaf_ids.as<int>(), ctx->nleaves, s);
+  launch_l2p(cfg.p, cells_of(ctx), bodies_of(ctx), rf, ctx->leaf_ids.as<int>(), ctx->nleaves, s,
+             false);
   TC_CHECK(hipEventRecord(ctx->ev[6], s));
   TC_CHECK(hipStreamWaitEvent(s, ctx->ev[10], 0));
-  launch_scatter_results_sum(bodies_of(ctx), r, rf, n, pot, acc, jerk, s);
+  // (with the body pairs evaluated by P2P: statistics, counted inside that kernel)
+  const auto *pairs = reinterpret_cast<const unsigned long long *>(ctx->h_pin + 52);
+  launch_scatter_results_sum(bodies_of(ctx), r, rf, n, pot, acc, jerk,
+                             ctx->npairs.as<unsigned long long>(),
+                             reinterpret_cast<unsigned long long *>(ctx->h_pin_dev + 52), s);
   TC_CHECK(hipEventRecord(ctx->ev[7], s));
-  // body pairs evaluated by P2P (statistics, counted inside the P2P kernel)
-  unsigned long long *pairs = reinterpret_cast<unsigned long long *>(ctx->h_pin + 52);
-  TC_CHECK(hipMemcpyAsync(pairs, ctx->npairs.p, sizeof(*pairs), hipMemcpyDeviceToHost, s));
   TC_CHECK(spin_wait(ctx, s));
   ctx->st.n_p2p_pairs = (long long)*pairs;
   float ms[8];
@@ -1048,11 +1023,6 @@ int master_eval_device(tc_context *ctx, int n, const double *x, const double *v,
     // the master tree has no root shift (the one-launch tree takes none)
     const double zero[3] = {0, 0, 0};
     std::memcpy(ctx->shift, zero, sizeof(zero));
-    if (!small) {
-      std::memcpy(ctx->h_pin + 16, zero, sizeof(zero));
-      TC_CHECK(hipMemcpyAsync(ctx->dshift.p, ctx->h_pin + 16, sizeof(zero),
-                              hipMemcpyHostToDevice, s));
-    }
   }
   TC_CHECK(ctx->mlend.ensure((size_t)n));
   if (!steps && !fmm) {

@@ -69,7 +69,7 @@ struct TreeParams {
 
 // ---- tree (tc_tree.hip)
 int launch_bounds(const double *x3, int n, double *partial, int nblocks_max, TreeParams *d_tp,
-                  const double *shift_frac_dev, hipStream_t s);
+                  const double shift_frac[3], hipStream_t s);
 // cid: cluster of every body (d_tp indexed by it), or null for one tree
 int launch_morton(const double *x3, int n, const TreeParams *d_tp, uint64_t *key_hi,
                   uint64_t *key_lo, int *idx, hipStream_t s, const int *cid = nullptr);
@@ -86,8 +86,6 @@ int launch_sort(uint64_t *key_a, uint64_t *key_b, int *val_a, int *val_b, const 
 int launch_gather(const double *x3, const double *v3, const double *q,
                   const unsigned char *flags_in, const int *perm, int n, BodiesDev b,
                   hipStream_t s);
-int launch_root(CellsDev c, int n, const TreeParams *d_tp, hipStream_t s,
-                const int *start = nullptr, int ncl = 1);
 // Device-side state of a tree build (ints): the level being split [ls, le),
 // leaves and levels so far, the level being placed (cls, cle, its first leaf
 // slot cbase, go), done, overflow (1: the cell arrays are too small, need
@@ -99,10 +97,15 @@ struct TreeState {
   int done, overflow, need, pad;
   int level_start[kMaxTreeLevels + 4];
 };
+// the root cells, and the state of a build that starts with them
+int launch_root(CellsDev c, int n, const TreeParams *d_tp, TreeState *st, hipStream_t s,
+                const int *start = nullptr, int ncl = 1);
 // One level: split (offs, nch), scans (scan), children and leaves.  Arrays of
 // per-level cells hold cap entries (nch and scan: 2 x cap).
+// report (or null): pinned host memory that receives the state after the level.
 int launch_tree_level(CellsDev c, BodiesDev b, TreeState *st, int ncrit, int cap, int *offs,
-                      int *nch, int *scan, const TreeParams *d_tp, int *leaf_ids, hipStream_t s);
+                      int *nch, int *scan, const TreeParams *d_tp, int *leaf_ids,
+                      TreeState *report, hipStream_t s);
 // The whole tree of at most kSmallTree bodies in one launch (one workgroup),
 // for the master time-step sums: bodies gathered into tree order, lend set on
 // the last body of every leaf; out[0] = leaves, out[1] = 0 or 2 (too deep),
@@ -161,12 +164,17 @@ struct TravState {
 };
 constexpr int kTravBlocks = 2048;  // blocks of a walk step; blk holds 6 x kTravBlocks ints
 // One step of the walk (count, offsets, write) on the frontier of parity par;
-// caps are the capacities of the lists and of the next frontier (pairs).
+// caps are the capacities of the lists and of the next frontier (pairs);
+// report (or null): pinned host memory that receives the state after the step.
 int launch_trav_step(CellsDev c, const TravArgs &a, TravState *st, int par, int *blk,
-                     long long cap_m2l, long long cap_p2p, long long cap_front, hipStream_t s);
+                     long long cap_m2l, long long cap_p2p, long long cap_front,
+                     TravState *report, hipStream_t s);
+// the frontier of the ncl root pairs (k, k) and the state that starts the walk
+void launch_root_pairs(int2 *front, int ncl, TravState *st, hipStream_t s);
 size_t pair_sort_temp_bytes(int n);
+// chunks (or null): ncells + 1 ints, ceil(count / 64) per cell and a last 0
 int launch_group_pairs(const int2 *pairs, int n, int key_bits, int ncells, int *tg_a, int *tg_b,
-                       int *src_a, int *src, int *start, int *count, void *temp,
+                       int *src_a, int *src, int *start, int *count, int *chunks, void *temp,
                        size_t temp_bytes, hipStream_t s);
 int launch_make_chunks(const int *offs, const int *count, const int *chunk_offs, int ncells,
                        int4 *chunks, hipStream_t s);
@@ -232,7 +240,10 @@ class P2PSplit {
   std::vector<int> first_{0}, sizes_, choice_{0};
   std::vector<double> cost_{0.0};
 };
-int launch_p2p_ranges(CellsDev c, const int *src, int n, int2 *ranges, hipStream_t s);
+// The near field's set-up in one launch: the source body range of every list
+// entry (nlist), r cleared for nb bodies and *npairs = 0.
+int launch_p2p_setup(CellsDev c, const int *src, int nlist, int2 *ranges, ResultsDev r, int nb,
+                     unsigned long long *npairs, hipStream_t s);
 int launch_direct(BodiesDev b, int n, const int *targets, int nt, double *pot, double *acc,
                   double *jerk, hipStream_t s);
 int launch_direct_sum(BodiesDev b, int n, const int *targets, int nt, double *pot, double *acc,
@@ -265,8 +276,9 @@ int launch_scatter_acc_old(BodiesDev b, int n, double *out, hipStream_t s);
 // ---- downward (tc_downward.hip)
 int launch_l2l(int p, CellsDev c, int ls, int le, hipStream_t s);
 int launch_l2l_ids(int p, CellsDev c, const int *ids, int nids, hipStream_t s);
+// add: into r; otherwise r is written (zeros for bodies that are not sinks)
 int launch_l2p(int p, CellsDev c, BodiesDev b, ResultsDev r, const int *leaf_ids, int nleaves,
-               hipStream_t s);
+               hipStream_t s, bool add = true);
 // master (non-jerk) variant, tc_master.hip
 void launch_iota(int *p, int n, hipStream_t s);
 void launch_zero_u8(unsigned char *p, int n, hipStream_t s);
@@ -355,7 +367,9 @@ void launch_scatter_ts(const BodiesDev &b, const double *ts_sorted, int n, doubl
 
 int launch_scatter_results(BodiesDev b, ResultsDev r, int n, double *pot, double *acc3,
                            double *jerk3, hipStream_t s);
+// also P2P's pair count *npairs to *report (pinned host memory)
 int launch_scatter_results_sum(BodiesDev b, ResultsDev r, ResultsDev f, int n, double *pot,
-                               double *acc3, double *jerk3, hipStream_t s);
+                               double *acc3, double *jerk3, const unsigned long long *npairs,
+                               unsigned long long *report, hipStream_t s);
 
 }  // namespace tcfmm

@@ -419,18 +419,24 @@ __global__ __launch_bounds__(64) TC_P2P_ATTR void k_p2p(CellsDev c, BodiesDev b,
   }
 }
 
-// Source body range (first body, count) of every P2P list entry.
-__global__ void k_p2p_ranges(CellsDev c, const int *__restrict__ src, int n,
-                             int2 *__restrict__ ranges) {
+// Source body range (first body, count) of every P2P list entry; the results
+// that P2P adds to and its pair counter are cleared in the same launch (a
+// memset per array is two launches each: sixteen launches less).
+__global__ void k_p2p_setup(CellsDev c, const int *__restrict__ src, int n,
+                            int2 *__restrict__ ranges, ResultsDev r, int nb,
+                            unsigned long long *npairs) {
   int k = blockIdx.x * 256 + threadIdx.x;
+  if (k < nb) r.pot[k] = r.ax[k] = r.ay[k] = r.az[k] = r.jx[k] = r.jy[k] = r.jz[k] = 0.0;
+  if (k == 0) *npairs = 0;
   if (k >= n) return;
   int j = src[k];
   ranges[k] = make_int2(c.body[j], c.nbody[j]);
 }
 
-int launch_p2p_ranges(CellsDev c, const int *src, int n, int2 *ranges, hipStream_t s) {
-  if (n <= 0) return 0;
-  hipLaunchKernelGGL(k_p2p_ranges, dim3((n + 255) / 256), dim3(256), 0, s, c, src, n, ranges);
+int launch_p2p_setup(CellsDev c, const int *src, int nlist, int2 *ranges, ResultsDev r, int nb,
+                     unsigned long long *npairs, hipStream_t s) {
+  hipLaunchKernelGGL(k_p2p_setup, dim3((std::max({nlist, nb, 1}) + 255) / 256), dim3(256), 0, s,
+                     c, src, nlist, ranges, r, nb, npairs);
   return 0;
 }
 
@@ -630,12 +636,16 @@ __global__ void k_scatter_results(BodiesDev b, ResultsDev r, int n, double *__re
   }
 }
 
-// near + far result sets, summed per body in tree order, to the caller's order
+// near + far result sets, summed per body in tree order, to the caller's
+// order; P2P's pair count to pinned host memory
 __global__ void k_scatter_results_sum(BodiesDev b, ResultsDev r, ResultsDev f, int n,
                                       double *__restrict__ pot, double *__restrict__ acc,
-                                      double *__restrict__ jerk) {
+                                      double *__restrict__ jerk,
+                                      const unsigned long long *__restrict__ npairs,
+                                      unsigned long long *report) {
   int k = blockIdx.x * 256 + threadIdx.x;
   if (k >= n) return;
+  if (k == 0) *report = *npairs;
   int i = b.order[k];
   if (pot) pot[i] = r.pot[k] + f.pot[k];
   if (acc) {
@@ -651,10 +661,11 @@ __global__ void k_scatter_results_sum(BodiesDev b, ResultsDev r, ResultsDev f, i
 }
 
 int launch_scatter_results_sum(BodiesDev b, ResultsDev r, ResultsDev f, int n, double *pot,
-                               double *acc3, double *jerk3, hipStream_t s) {
+                               double *acc3, double *jerk3, const unsigned long long *npairs,
+                               unsigned long long *report, hipStream_t s) {
   if (n <= 0) return 0;
   hipLaunchKernelGGL(k_scatter_results_sum, dim3((n + 255) / 256), dim3(256), 0, s, b, r, f, n,
-                     pot, acc3, jerk3);
+                     pot, acc3, jerk3, npairs, report);
   return 0;
 }
 

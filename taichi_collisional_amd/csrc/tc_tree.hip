@@ -61,9 +61,9 @@ __global__ __launch_bounds__(256) void k_bounds_partial(const double *__restrict
 // One wave: lane-strided min / max over the block partials, then a wave
 // reduction (min and max do not depend on the order); lane 0 finishes.
 __global__ __launch_bounds__(64) void k_bounds_final(const double *__restrict__ part, int nb,
-                                                     const double *__restrict__ shift_frac,
-                                                     TreeParams *tp) {
+                                                     double3 shift, TreeParams *tp) {
 #pragma clang fp contract(off)
+  const double shift_frac[3] = {shift.x, shift.y, shift.z};
   const int lane = threadIdx.x;
   double mn[3], mx[3];
   for (int d = 0; d < 3; d++) mn[d] = part[d], mx[d] = part[3 + d];
@@ -103,12 +103,13 @@ __global__ __launch_bounds__(64) void k_bounds_final(const double *__restrict__ 
 }
 
 int launch_bounds(const double *x3, int n, double *partial, int nblocks_max, TreeParams *d_tp,
-                  const double *shift_frac_dev, hipStream_t s) {
+                  const double shift_frac[3], hipStream_t s) {
   int nb = (n + 255) / 256;
   if (nb > nblocks_max) nb = nblocks_max;
   if (nb < 1) nb = 1;
   hipLaunchKernelGGL(k_bounds_partial, dim3(nb), dim3(256), 0, s, x3, n, partial);
-  hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(64), 0, s, partial, nb, shift_frac_dev, d_tp);
+  hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(64), 0, s, partial, nb,
+                     make_double3(shift_frac[0], shift_frac[1], shift_frac[2]), d_tp);
   return 0;
 }
 
@@ -318,8 +319,14 @@ int launch_gather(const double *x3, const double *v3, const double *q,
 // ---------------------------------------------------------------- cells -----
 // Root cells: one (all n bodies), or one per cluster of a forest (cluster k
 // = [start[k], start[k+1]) with its own TreeParams).
-__global__ void k_root(CellsDev c, int n, const TreeParams *__restrict__ tp,
+// The first block also sets the state of the build.
+__global__ void k_root(CellsDev c, int n, const TreeParams *__restrict__ tp, TreeState *st,
                        const int *__restrict__ start, int ncl) {
+  if (blockIdx.x == 0) {
+    int *w = reinterpret_cast<int *>(st);
+    for (int t = threadIdx.x; t < (int)(sizeof(TreeState) / sizeof(int)); t += 64)
+      w[t] = t == offsetof(TreeState, le) / sizeof(int) ? ncl : 0;
+  }
   const int k = blockIdx.x * 64 + threadIdx.x;
   if (k >= ncl) return;
   c.level[k] = 0;
@@ -331,9 +338,9 @@ __global__ void k_root(CellsDev c, int n, const TreeParams *__restrict__ tp,
   c.Rg[k] = tp[k].R0;
 }
 
-int launch_root(CellsDev c, int n, const TreeParams *d_tp, hipStream_t s, const int *start,
-                int ncl) {
-  hipLaunchKernelGGL(k_root, dim3((ncl + 63) / 64), dim3(64), 0, s, c, n, d_tp, start, ncl);
+int launch_root(CellsDev c, int n, const TreeParams *d_tp, TreeState *st, hipStream_t s,
+                const int *start, int ncl) {
+  hipLaunchKernelGGL(k_root, dim3((ncl + 63) / 64), dim3(64), 0, s, c, n, d_tp, st, start, ncl);
   return 0;
 }
 
@@ -420,11 +427,14 @@ __global__ __launch_bounds__(256) void k_split(CellsDev c, BodiesDev b,
 // kMaxTreeLevels sets overflow = 2.
 __global__ __launch_bounds__(1024) void k_level_scan(const int *__restrict__ nch,
                                                      int *__restrict__ scan, TreeState *st,
-                                                     int cap) {
+                                                     int cap, TreeState *report) {
   __shared__ int wsum[2][16];
   __shared__ int carry[2];
   if (st->done || st->overflow) {
-    if (threadIdx.x == 0) st->go = 0;
+    if (threadIdx.x == 0) {
+      st->go = 0;
+      if (report) *report = *st;
+    }
     return;
   }
   const int ls = st->ls, le = st->le, nl = le - ls;
@@ -504,6 +514,7 @@ __global__ __launch_bounds__(1024) void k_level_scan(const int *__restrict__ nch
         st->le = le + total;
       }
     }
+    if (report) *report = *st;
   }
 }
 
@@ -553,12 +564,14 @@ __global__ __launch_bounds__(256) void k_children(CellsDev c, const TreeState *_
 }
 
 int launch_tree_level(CellsDev c, BodiesDev b, TreeState *st, int ncrit, int cap, int *offs,
-                      int *nch, int *scan, const TreeParams *d_tp, int *leaf_ids, hipStream_t s) {
+                      int *nch, int *scan, const TreeParams *d_tp, int *leaf_ids,
+                      TreeState *report, hipStream_t s) {
   // grids cover the widest levels in a few sweeps; narrow levels leave most
   // blocks idle for a few microseconds
   hipLaunchKernelGGL(k_split, dim3(512), dim3(256), 0, s, c, b, (const TreeState *)st, ncrit, cap,
                      offs, nch);
-  hipLaunchKernelGGL(k_level_scan, dim3(1), dim3(1024), 0, s, (const int *)nch, scan, st, cap);
+  hipLaunchKernelGGL(k_level_scan, dim3(1), dim3(1024), 0, s, (const int *)nch, scan, st, cap,
+                     report);
   hipLaunchKernelGGL(k_children, dim3(256), dim3(256), 0, s, c, (const TreeState *)st, cap,
                      (const int *)offs, (const int *)scan, d_tp, leaf_ids);
   return 0;
@@ -1289,7 +1302,7 @@ __global__ __launch_bounds__(256) void k_trav_count(CellsDev c, const int2 *__re
 // fill the machine with small blocks, which a 1024-thread block waits out.
 __global__ __launch_bounds__(64) void k_trav_scan(int *__restrict__ blk, TravState *st, int par,
                                                   long long cap_m2l, long long cap_p2p,
-                                                  long long cap_front) {
+                                                  long long cap_front, TravState *report) {
   constexpr int G = kTravBlocks, PER = G / kWave;
   static_assert(G % kWave == 0, "whole entries per lane");
   const int t = threadIdx.x;
@@ -1335,6 +1348,7 @@ __global__ __launch_bounds__(64) void k_trav_scan(int *__restrict__ blk, TravSta
       st->write = 0;
       st->nin[par ^ 1] = 0;
     }
+    if (report) *report = *st;
   }
 }
 
@@ -1375,14 +1389,29 @@ __global__ __launch_bounds__(256) void k_trav_write(CellsDev c, TravArgs a,
 }
 
 int launch_trav_step(CellsDev c, const TravArgs &a, TravState *st, int par, int *blk,
-                     long long cap_m2l, long long cap_p2p, long long cap_front, hipStream_t s) {
+                     long long cap_m2l, long long cap_p2p, long long cap_front,
+                     TravState *report, hipStream_t s) {
   hipLaunchKernelGGL(k_trav_count, dim3(kTravBlocks), dim3(256), 0, s, c, a.fin,
                      (const TravState *)st, par, a.mac, blk, a.cls);
   hipLaunchKernelGGL(k_trav_scan, dim3(1), dim3(kWave), 0, s, blk, st, par, cap_m2l, cap_p2p,
-                     cap_front);
+                     cap_front, report);
   hipLaunchKernelGGL(k_trav_write, dim3(kTravBlocks), dim3(256), 0, s, c, a,
                      (const TravState *)st, par, (const int *)blk);
   return 0;
+}
+
+__global__ void k_root_pairs(int2 *__restrict__ f, int ncl, TravState *st) {
+  const int k = blockIdx.x * 256 + threadIdx.x;
+  if (k < ncl) f[k] = make_int2(k, k);
+  if (k == 0) {
+    TravState z = {};
+    z.nin[0] = ncl;  // the root pair (0, 0), or (k, k) for every cluster
+    *st = z;
+  }
+}
+
+void launch_root_pairs(int2 *front, int ncl, TravState *st, hipStream_t s) {
+  hipLaunchKernelGGL(k_root_pairs, dim3((ncl + 255) / 256), dim3(256), 0, s, front, ncl, st);
 }
 
 // Group (target, source) pairs by target: stable radix sort on the target,
@@ -1396,9 +1425,12 @@ size_t pair_sort_temp_bytes(int n) {
   return std::max(b, bk);
 }
 
+// The runs' bounds start, endp (ncells entries) are cleared along the way.
 __global__ void k_split_pairs(const int2 *__restrict__ pairs, int n, int *__restrict__ tg,
-                              int *__restrict__ sr) {
+                              int *__restrict__ sr, int *__restrict__ start,
+                              int *__restrict__ endp, int ncells) {
   int k = blockIdx.x * 256 + threadIdx.x;
+  if (k < ncells) start[k] = endp[k] = 0;
   if (k >= n) return;
   int2 p = pairs[k];
   tg[k] = p.x;
@@ -1406,7 +1438,7 @@ __global__ void k_split_pairs(const int2 *__restrict__ pairs, int n, int *__rest
 }
 
 // Marks runs of equal targets: start[t] = first index, endp[t] = one past the
-// last (both zero-initialized, so targets without entries keep 0 / 0).
+// last (both cleared before, so targets without entries keep 0 / 0).
 __global__ void k_runs(const int *__restrict__ tg, int n, int *__restrict__ start,
                        int *__restrict__ endp) {
   int k = blockIdx.x * 256 + threadIdx.x;
@@ -1416,15 +1448,23 @@ __global__ void k_runs(const int *__restrict__ tg, int n, int *__restrict__ star
   if (k == n - 1 || tg[k + 1] != t) endp[t] = k + 1;
 }
 
-__global__ void k_run_counts(const int *__restrict__ start, int *__restrict__ cnt, int ncells) {
+// Run ends to counts; chunks (or null): the M2L chunks of <= 64 sources of
+// every cell, and 0 at ncells.
+__global__ void k_run_counts(const int *__restrict__ start, int *__restrict__ cnt, int ncells,
+                             int *__restrict__ chunks) {
   int c = blockIdx.x * 256 + threadIdx.x;
-  if (c < ncells) cnt[c] -= start[c];
+  if (c > ncells) return;
+  const int v = c < ncells ? cnt[c] - start[c] : 0;
+  if (c < ncells) cnt[c] = v;
+  if (chunks) chunks[c] = (v + 63) / 64;
 }
 
 // Cell ids below 2^16: one 32-bit word per pair, target above source, so the
 // sort moves half the bytes of a key + value sort (the same stable order).
-__global__ void k_pack_pairs(const int2 *__restrict__ pairs, int n, unsigned *__restrict__ w) {
+__global__ void k_pack_pairs(const int2 *__restrict__ pairs, int n, unsigned *__restrict__ w,
+                             int *__restrict__ start, int *__restrict__ endp, int ncells) {
   const int k = blockIdx.x * 256 + threadIdx.x;
+  if (k < ncells) start[k] = endp[k] = 0;
   if (k >= n) return;
   const int2 p = pairs[k];
   w[k] = ((unsigned)p.x << 16) | (unsigned)p.y;
@@ -1443,32 +1483,36 @@ __global__ void k_runs_packed(const unsigned *__restrict__ w, int n, int *__rest
 }
 
 // After the call: src[] holds sources grouped by target (stable), start[] /
-// count[] (zeroed by the caller) the run of every target.
+// count[] the run of every target (0 / 0 where it has none).
 int launch_group_pairs(const int2 *pairs, int n, int key_bits, int ncells, int *tg_a, int *tg_b,
-                       int *src_a, int *src, int *start, int *count, void *temp,
+                       int *src_a, int *src, int *start, int *count, int *chunks, void *temp,
                        size_t temp_bytes, hipStream_t s) {
-  if (n <= 0) return 0;
+  if (n < 0) n = 0;
+  const dim3 gp((std::max(n, ncells) + 255) / 256), gc((ncells + 1 + 255) / 256);
   if (ncells <= (1 << 16) && key_bits <= 16) {
     unsigned *wa = reinterpret_cast<unsigned *>(tg_a), *wb = reinterpret_cast<unsigned *>(tg_b);
-    hipLaunchKernelGGL(k_pack_pairs, dim3((n + 255) / 256), dim3(256), 0, s, pairs, n, wa);
+    hipLaunchKernelGGL(k_pack_pairs, gp, dim3(256), 0, s, pairs, n, wa, start, count, ncells);
     size_t tb = temp_bytes;
-    if (hipcub::DeviceRadixSort::SortKeys(temp, tb, wa, wb, n, 16, 16 + key_bits, s) !=
-        hipSuccess)
-      return -1;
-    hipLaunchKernelGGL(k_runs_packed, dim3((n + 255) / 256), dim3(256), 0, s, wb, n, start,
-                       count, src);
-    hipLaunchKernelGGL(k_run_counts, dim3((ncells + 255) / 256), dim3(256), 0, s, start, count,
-                       ncells);
+    if (n > 0) {
+      if (hipcub::DeviceRadixSort::SortKeys(temp, tb, wa, wb, n, 16, 16 + key_bits, s) !=
+          hipSuccess)
+        return -1;
+      hipLaunchKernelGGL(k_runs_packed, dim3((n + 255) / 256), dim3(256), 0, s, wb, n, start,
+                         count, src);
+    }
+    hipLaunchKernelGGL(k_run_counts, gc, dim3(256), 0, s, start, count, ncells, chunks);
     return 0;
   }
-  hipLaunchKernelGGL(k_split_pairs, dim3((n + 255) / 256), dim3(256), 0, s, pairs, n, tg_a, src_a);
-  size_t tb = temp_bytes;
-  if (hipcub::DeviceRadixSort::SortPairs(temp, tb, tg_a, tg_b, src_a, src, n, 0, key_bits, s) !=
-      hipSuccess)
-    return -1;
-  hipLaunchKernelGGL(k_runs, dim3((n + 255) / 256), dim3(256), 0, s, tg_b, n, start, count);
-  hipLaunchKernelGGL(k_run_counts, dim3((ncells + 255) / 256), dim3(256), 0, s, start, count,
+  hipLaunchKernelGGL(k_split_pairs, gp, dim3(256), 0, s, pairs, n, tg_a, src_a, start, count,
                      ncells);
+  size_t tb = temp_bytes;
+  if (n > 0) {
+    if (hipcub::DeviceRadixSort::SortPairs(temp, tb, tg_a, tg_b, src_a, src, n, 0, key_bits, s) !=
+        hipSuccess)
+      return -1;
+    hipLaunchKernelGGL(k_runs, dim3((n + 255) / 256), dim3(256), 0, s, tg_b, n, start, count);
+  }
+  hipLaunchKernelGGL(k_run_counts, gc, dim3(256), 0, s, start, count, ncells, chunks);
   return 0;
 }
 

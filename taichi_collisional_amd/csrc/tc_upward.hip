@@ -44,7 +44,7 @@ template <int P, int N>
 __device__ __forceinline__ void p2m_orders(double dx, double dy, double dz, double r2, double vx,
                                            double vy, double vz, double w, cplx *y1, cplx *y2,
                                            double (*red)[2 * (P + 1) + 1], int lane, int cnt,
-                                           double *Mc, double *Mdc) {
+                                           bool add, double *Mc, double *Mdc) {
   cplx yn[P + 1];
   harm_row_c<N>(dx, dy, dz, r2, y1, y2, yn);
   constexpr int s = N * N + N;
@@ -87,7 +87,7 @@ __device__ __forceinline__ void p2m_orders(double dx, double dy, double dz, doub
     const int m = col >> 1, im = col & 1;
     if (col < C && part == 0 && !(m == 0 && im)) {
       double *dst = (pass == 0 ? Mc : Mdc) + (im ? s - m : s + m);
-      *dst += acc;
+      *dst = add ? *dst + acc : acc;
     }
     __syncthreads();
   }
@@ -97,7 +97,8 @@ __device__ __forceinline__ void p2m_orders(double dx, double dy, double dz, doub
       y2[m] = y1[m];
       y1[m] = yn[m];
     }
-    p2m_orders<P, N + 1>(dx, dy, dz, r2, vx, vy, vz, w, y1, y2, red, lane, cnt, Mc, Mdc);
+    p2m_orders<P, N + 1>(dx, dy, dz, r2, vx, vy, vz, w, y1, y2, red, lane, cnt, add, Mc,
+                         Mdc);
   }
 }
 
@@ -106,6 +107,11 @@ __device__ __forceinline__ void p2m_orders(double dx, double dy, double dz, doub
 // walk starts on the geometry while the moments are formed on another stream,
 // and with the error MAC geometry and moments run alongside the pre-pass that
 // min_acc waits for.
+//
+// kUpAll adds to M, Mdot and has_sink, which the caller sets; the parts that
+// an evaluation runs write them, and the geometry clears the cell's L and
+// Ldot, so an evaluation clears no arrays (at p = 12 and 2^20 bodies that was
+// 340 MB of fills, and five launches at every size).
 template <int P, int kWhat>
 __global__ __launch_bounds__(64) void k_p2m(CellsDev c, BodiesDev b,
                                             const int *__restrict__ leaf_ids) {
@@ -172,8 +178,11 @@ __global__ __launch_bounds__(64) void k_p2m(CellsDev c, BodiesDev b,
       for (int d = 0; d < 3; d++) c.X[3 * ci + d] = X[d];
       c.R[ci] = R;
       if (kWhat & kUpMin) c.min_acc[ci] = mina;
-      c.has_sink[ci] = (unsigned char)(c.has_sink[ci] | sink);
+      c.has_sink[ci] = (unsigned char)(kWhat == kUpAll ? c.has_sink[ci] | sink : sink);
     }
+    if constexpr (kWhat != kUpAll)
+      for (int t = lane; t < NT; t += kWave)
+        c.L[(size_t)ci * NT + t] = c.Ld[(size_t)ci * NT + t] = 0.0;
   }
   if constexpr (!(kWhat & kUpMoments)) return;
   double *Mc = c.M + (size_t)ci * NT;
@@ -193,7 +202,8 @@ __global__ __launch_bounds__(64) void k_p2m(CellsDev c, BodiesDev b,
     }
     const double r2 = dx * dx + dy * dy + dz * dz;
     cplx y1[P + 1], y2[P + 1];
-    p2m_orders<P, 0>(dx, dy, dz, r2, vx, vy, vz, w, y1, y2, red, lane, cnt, Mc, Mdc);
+    p2m_orders<P, 0>(dx, dy, dz, r2, vx, vy, vz, w, y1, y2, red, lane, cnt,
+                     kWhat == kUpAll || base > 0, Mc, Mdc);
     if (nb == 0) break;
   }
 }
@@ -205,6 +215,7 @@ __global__ __launch_bounds__(256) void k_m2m(CellsDev c, BodiesDev b, const int 
   constexpr int NT = nterm(P);
   constexpr int NO = tri(P, P) + 1;
   constexpr int NW = 4;
+  constexpr bool kAdd = kWhat == kUpAll;
   constexpr int kStage = 512;  // body points of leaf children staged in LDS
   // Eight children's harmonic tables and moments (complex) side by side, when
   // they fit one work-group's LDS; else one child at a time.
@@ -382,8 +393,11 @@ __global__ __launch_bounds__(256) void k_m2m(CellsDev c, BodiesDev b, const int 
       for (int d = 0; d < 3; d++) c.X[3 * ci + d] = X[d];
       c.R[ci] = sqrt(ball.r2) + 1e-6;
       if (kWhat & kUpMin) c.min_acc[ci] = mina;
-      c.has_sink[ci] = (unsigned char)(c.has_sink[ci] | sink);
+      c.has_sink[ci] = (unsigned char)(kWhat == kUpAll ? c.has_sink[ci] | sink : sink);
     }
+    if constexpr (kWhat != kUpAll)
+      for (int t = tid; t < NT; t += NW * kWave)
+        c.L[(size_t)ci * NT + t] = c.Ld[(size_t)ci * NT + t] = 0.0;
     __syncthreads();  // the ball's buffers are reused below
   }
   if constexpr (!(kWhat & kUpMoments)) return;
@@ -440,8 +454,8 @@ __global__ __launch_bounds__(256) void k_m2m(CellsDev c, BodiesDev b, const int 
         }
         if (k == 0) {
           const int s = n * n + n;
-          dst[s + m] += acc.re;
-          if (m > 0) dst[s - m] += acc.im;
+          dst[s + m] = kAdd ? dst[s + m] + acc.re : acc.re;
+          if (m > 0) dst[s - m] = kAdd ? dst[s - m] + acc.im : acc.im;
         }
       }
       __syncthreads();  // Call is refilled by the next pass
@@ -498,8 +512,8 @@ __global__ __launch_bounds__(256) void k_m2m(CellsDev c, BodiesDev b, const int 
       if (j >= NTASK) continue;
       double *dst = (j >= NO ? c.Md : c.M) + (size_t)ci * NT;
       const int n = tn[r], m = tm[r], s = n * n + n;
-      dst[s + m] += a[r].re;
-      if (m > 0) dst[s - m] += a[r].im;
+      dst[s + m] = kAdd ? dst[s + m] + a[r].re : a[r].re;
+      if (m > 0) dst[s - m] = kAdd ? dst[s - m] + a[r].im : a[r].im;
     }
   }
 }
