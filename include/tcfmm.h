@@ -107,9 +107,10 @@ int tc_set_precision(tc_context *ctx, int p2p_mode, double close_radius);
 /* ---- Launch shape of the near field (no reference counterpart: the
  * reference's P2P, kernel_fast_lean.h:499-699, is a CPU loop over leaf
  * pairs) ----------------------------------------------------------------
- * tile: source bodies per LDS tile (64, 128 or 192); list_slice: P2P-list
- * entries per work item (a leaf's list is split into slices that run as
- * separate waves; 1..65535); stage_rounds: the cost of staging one tile, in
+ * tile: source bodies per LDS tile (64, 128 or 192); list_slice: the most
+ * P2P-list entries per work item (a leaf's list is split into slices that run
+ * as separate waves; 1..65535; an evaluation whose whole list is short takes
+ * smaller slices, down to 16, to fill the GPU); stage_rounds: the cost of staging one tile, in
  * rounds of pair evaluations, that the cut of each leaf into target groups
  * trades against idle lanes (0 favours groups that fill the wave, larger
  * values fewer groups); targets_per_lane: 1 or 2 (one LDS read of a source

@@ -349,14 +349,23 @@ static int build_lists(tc_context *ctx, int &nchunks) {
   return 0;
 }
 
-// P2P work items: every target group x slices of <= p2p_list list entries.
+// P2P work items: every target group x slices of at most p2p_list list entries
+// (fewer where the whole list is short).
 // Each leaf is cut into target groups of <= 64 bodies by the lane model of
 // the kernel (P2PSplit).  The per-leaf list lengths were copied to pinned
 // memory before the M2L launch (and the stream synchronized after that
 // copy), so this host loop runs while the GPU is busy with M2L; the upload is
 // queued behind it.
 static int build_p2p_items(tc_context *ctx) {
-  const int kList = ctx->p2p_list;
+  // Slices so that even a small system's list makes thousands of items: a
+  // wave's time is its chain of tiles, and two or three waves a SIMD leave the
+  // chip waiting for the longest.  P2P, list slice 128 / this rule, in us:
+  // N = 10,007 (95 K entries, 16) 416 / 143; 30,000 (296 K, 16) 729 / 369;
+  // 131,072 (515 K, 16) 852 / 630; 262,144 (2.4 M, 74) 2,705 / 2,480; from 4 M
+  // entries on 64 and 128 are level, while 16 and less restage too often.
+  const int kMinSlice = 16, kSliceShare = 1 << 15;
+  const int kList = std::min<long long>(
+      ctx->p2p_list, std::max<long long>(kMinSlice, ctx->st.n_p2p_cells / kSliceShare));
   TC_CHECK(spin_event(ctx->ev[11]));  // leaf ids and body counts (build_tree)
   TC_CHECK(spin_event(ctx->ev[15]));  // list lengths (build_lists)
   const int *pcnt = ctx->h_pcnt.p, *leaves = ctx->h_leaves.p, *nbd = ctx->h_nbd.p;
