@@ -23,15 +23,23 @@
 // a higher order), and only the terms up to order P are read and added, so
 // one set of coefficient arrays serves pairs of different orders.
 //
-// Work decomposition: a block = one wave = one chunk of <= 64 sources of a
-// single target cell (the chunk list is grouped by target) for one array
-// (M -> L or Mdot -> Ldot); each XCD takes a contiguous range of the
-// (array, chunk) items so neighbouring targets share its L2.  Each order's 2n+1 contributions are
-// summed across the wave through an LDS transpose; the chunk adds its sum
-// into the target's L with one atomic per coefficient.
+// Work decomposition: one wave = one chunk of <= 64 sources of a single target
+// cell (the chunk list is grouped by target) for one array (M -> L or Mdot ->
+// Ldot); each XCD takes a contiguous range of the (array, chunk) items so
+// neighbouring targets share its L2.  The contributions are summed across the
+// wave on the matrix unit (WaveSum); the chunk adds its sum into the target's
+// L with one atomic per coefficient.
+//
+// Bound by FP64 issue and the power it draws.  One launch, before -> after the
+// sums left the vector unit and LDS, the four-wave blocks and the two parts:
+// p = 12, N = 2^20 (theta 0.4, 35.2 M pairs) 14.06 -> 13.2 ms; N = 2^17 (theta
+// 0.5, 1.98 M pairs) p = 16: 3.18 -> 2.11, 18: 4.82 -> 2.79, 20: 11.70 ->
+// 4.94, 24: 37.0 -> 8.29 ms.
 #include "tc_common.h"
 #include "tc_kernels.h"
 #include "swap_tables.h"
+
+#include <algorithm>
 
 #ifndef TC_SHARD
 #error "compiled once per order shard, with -DTC_SHARD=k (see TC_NSHARDS in tc_kernels.h)"
@@ -141,32 +149,81 @@ __device__ __forceinline__ void swap_block(const double *in, double *out) {
   }
 }
 
-// Row stride (doubles) of the LDS reduction buffer: 64 lanes + 16 padding,
-// so rows r and r+1 start 32 banks apart.
-constexpr int kRedStride = kWave + 16;
-// One reduction buffer holds the rows of the largest order.  Orders up to 12
-// fit two waves per SIMD in registers, and a second buffer would then halve
-// occupancy through LDS; from 14 on, one wave per SIMD runs anyway and two
-// buffers alternate between consecutive orders so the reduction of one order
-// overlaps the next order's arithmetic.
-template <int P>
-struct RedBuf {
-  static constexpr int size = (2 * P + 1) * kRedStride;
-  static constexpr bool pipelined = P >= 14;
-  static constexpr int count = pipelined ? 2 : 1;
-};
+// Waves per block, one chunk each.  From p = 14 on the kernel's straight-line
+// code is larger than the 64 KB instruction cache (p = 15: 77 KB, 20: 175 KB,
+// 24: 310 KB); the four waves of a block then go through it together, kept in
+// step by a barrier per order, so that each line is fetched once for four.
+constexpr int m2l_waves(int p) { return p >= 14 ? 4 : 1; }
 
+// Waves per SIMD the registers are cut for (0: as they come, two or more).
+// Two up to p = 19 (p = 19: 3.43 ms against 4.63 with one, N = 2^17), one
+// above, where the second wave's share spills (p = 20: 4.94 against 5.26 with
+// two, p = 24: 8.29 against 12.9).
+constexpr int m2l_occ(int p) { return p < 13 ? 0 : p <= 19 ? 2 : 1; }
+
+// The source orders are taken in two parts, k > m2l_split(p) and then the
+// rest, each rotated, translated and rotated back (the operator is linear):
+// the first part reaches only the target orders n < p - m2l_split, whose
+// backward half costs an eighth of the whole, and each part's rotated moments
+// are about half of all (p = 20: 100 and 121 of 221 doubles, which with the
+// working set would be over 512 registers).  -1: one part, up to p = 13, whose
+// moments fit (p = 12 in two parts: 14.4 ms against 13.2, N = 2^20; p = 14:
+// 1.52 ms in two parts, 1.71 in one, N = 2^17).
+constexpr int m2l_split(int p) { return p >= 14 ? p / 2 : -1; }
+
+// Where the rotated moments M_k^m, |m| <= q(k) = min(k, P - k), of the source
+// orders k = LO..HI are kept between the halves: a register each, and in the
+// orders of four-wave blocks (where LDS is free and registers are not) an LDS
+// slot for those with P - k - |m| <= reach, which the translation reads at
+// most reach + 1 times: as many as fit (80 or 40 KB a SIMD's wave).
 template <int P>
-struct M2LRegs {
-  static constexpr int q(int n) { return n < P - n ? n : P - n; }
-  // offset of order n in the packed rotated-multipole store (|m| <= q(n))
-  static constexpr int off(int n) {
-    int o = 0;
-    for (int k = 0; k < n; k++) o += 2 * q(k) + 1;
-    return o;
-  }
-  static constexpr int total = off(P + 1);
+struct M2LStore {
+  // register index, or -1 - slot; at k^2 + k + m
+  short at[(P + 1) * (P + 1)];
+  int regs, slots;
 };
+constexpr int m2l_q(int p, int k) { return k < p - k ? k : p - k; }
+template <int P>
+constexpr M2LStore<P> m2l_store(int lo, int hi) {
+  const int room = m2l_waves(P) == 1 ? 0 : m2l_occ(P) == 2 ? 39 : 80;
+  int reach = -1;
+  for (int u = 0; u <= P; u++) {
+    int c = 0;
+    for (int k = lo; k <= hi; k++)
+      for (int m = -m2l_q(P, k); m <= m2l_q(P, k); m++) c += P - k - (m < 0 ? -m : m) <= u;
+    if (c > room) break;
+    reach = u;
+  }
+  M2LStore<P> s = {};
+  for (int k = lo; k <= hi; k++)
+    for (int m = -m2l_q(P, k); m <= m2l_q(P, k); m++) {
+      if (P - k - (m < 0 ? -m : m) <= reach)
+        s.at[k * k + k + m] = (short)(-1 - s.slots++);
+      else
+        s.at[k * k + k + m] = (short)s.regs++;
+    }
+  return s;
+}
+template <int P, int LO, int HI>
+struct M2LPart {
+  static constexpr M2LStore<P> store = m2l_store<P>(LO, HI);
+  // largest |m| that reaches target order n, and the largest such order
+  static constexpr int q(int n) {
+    int q = 0;
+    for (int k = LO; k <= HI && k <= P - n; k++) q = m2l_q(P, k) > q ? m2l_q(P, k) : q;
+    return n < q ? n : q;
+  }
+  static constexpr int top = P - LO;
+};
+template <int P, int LO, int HI>
+constexpr M2LStore<P> M2LPart<P, LO, HI>::store;
+
+// M_k^m (compile-time k, m) from where it is kept; ml: the lane's LDS column
+template <class Part>
+__device__ __forceinline__ double kept(const double *mp, const double *ml, int k, int m) {
+  const int w = Part::store.at[k * k + k + m];
+  return w < 0 ? ml[(-1 - w) * kWave] : mp[w];
+}
 
 template <int N>
 __device__ __forceinline__ void load_order(const double *__restrict__ src, double *v) {
@@ -174,39 +231,25 @@ __device__ __forceinline__ void load_order(const double *__restrict__ src, doubl
   for (int r = 0; r < 2 * N + 1; r++) v[r] = src[N * N + r];
 }
 
-// Prefetch distance of the forward half, in orders: the source gathers of
-// orders N-1 .. N-kAhead are in flight while order N computes (one wave per
-// SIMD leaves registers to spare, and a 64-lane gather takes thousands of
-// cycles).
-#ifndef TC_M2L_AHEAD
-#define TC_M2L_AHEAD 1
-#endif
-constexpr int kAhead = TC_M2L_AHEAD;
-static_assert(kAhead >= 1 && kAhead <= 4, "prefetch distance");
-
-template <int N>
-struct OrderBuf {
-  static constexpr int size = N >= 0 ? 2 * N + 1 : 1;
-};
-
-// Forward half for order N of the source moments: scale, rotate by alpha_z,
-// swap, rotate by alpha_x, swap (rows |m| <= min(N, p-N) only), unscale into
-// the rotated-moment store.  b0 holds order N; b1..b3 hold orders N-1..N-3
-// when loaded (kAhead of them); the gather of order N-kAhead is issued first,
-// fenced with scheduling barriers so the compiler neither hoists every
-// order's gathers to the top nor sinks them to their use.
-template <int P, int N>
+// Forward half for the orders N..LO of the source moments, one after another:
+// rotate by alpha_z, swap, rotate by alpha_x, swap (rows |m| <= min(N, p-N)
+// only), into the rotated-moment store.  b0 holds order N; the gather of order
+// N-1 is issued first, fenced with scheduling barriers so the compiler neither
+// hoists every order's gathers to the top nor sinks them to their use (deeper
+// prefetch made no difference).
+template <int P, int LO, int HI, int N>
 __device__ __forceinline__ void m2l_forward_order(const double *__restrict__ src, bool quirk,
                                                   double ezr, double ezi, double exr,
-                                                  double exi, double *b0, double *b1,
-                                                  double *b2, double *b3, double *mp) {
+                                                  double exi, const double *b0, double *mp,
+                                                  double *ml) {
+  using Part = M2LPart<P, LO, HI>;
   constexpr int K = 2 * N + 1;
-  constexpr int Q = M2LRegs<P>::q(N);
-  constexpr int O = M2LRegs<P>::off(N);
-  double nb[OrderBuf<N - kAhead>::size];
-  if constexpr (N - kAhead >= 0) {
+  constexpr int Q = m2l_q(P, N);
+  if constexpr (m2l_waves(P) > 1) __syncthreads();
+  double nb[N > LO ? 2 * N - 1 : 1];
+  if constexpr (N > LO) {
     __builtin_amdgcn_sched_barrier(0);
-    load_order<N - kAhead>(src, nb);
+    load_order<N - 1>(src, nb);
     __builtin_amdgcn_sched_barrier(0);
   }
   // D^-1 S Rx S D Rz with D = diag((n+|m|)!(n-|m|)!) (the reference's scale
@@ -225,151 +268,192 @@ __device__ __forceinline__ void m2l_forward_order(const double *__restrict__ src
   rotate<N, false>(w, exr, exi);
   swap_block<N, Q, N, true>(w, v);
 #pragma unroll
-  for (int m = -Q; m <= Q; m++) mp[O + Q + m] = v[N + m];
-  if constexpr (N > 0) {
-    if constexpr (kAhead == 1)
-      m2l_forward_order<P, N - 1>(src, quirk, ezr, ezi, exr, exi, nb, nullptr, nullptr, nullptr,
-                                  mp);
-    else if constexpr (kAhead == 2)
-      m2l_forward_order<P, N - 1>(src, quirk, ezr, ezi, exr, exi, b1, nb, nullptr, nullptr, mp);
-    else if constexpr (kAhead == 3)
-      m2l_forward_order<P, N - 1>(src, quirk, ezr, ezi, exr, exi, b1, b2, nb, nullptr, mp);
+  for (int m = -Q; m <= Q; m++) {
+    const int at = Part::store.at[N * N + N + m];
+    if (at < 0)
+      ml[(-1 - at) * kWave] = v[N + m];
     else
-      m2l_forward_order<P, N - 1>(src, quirk, ezr, ezi, exr, exi, b1, b2, b3, nb, mp);
+      mp[at] = v[N + m];
   }
+  if constexpr (N > LO)
+    m2l_forward_order<P, LO, HI, N - 1>(src, quirk, ezr, ezi, exr, exi, nb, mp, ml);
 }
 
-// Sum order N's K = 2N+1 contributions over the wave: the lanes' values sit
-// in LDS rows (row stride kRedStride); groups of 8 lanes each sum one row
-// (8 values per lane, a 3-step butterfly inside the group).  A group reads
-// its row as four contiguous 128-byte runs and the padded stride puts
-// neighbouring rows in opposite halves of the 64 banks, so the eight groups of
-// one read fill the banks evenly.  Rows past K are read as row K-1 and
-// written to a per-lane spare slot, which keeps the loop free of divergent
-// branches.
-template <int P, int N>
-__device__ __forceinline__ void reduce_order(const double *red, double *acc_lds, int lane) {
-  constexpr int K = 2 * N + 1;
-  __syncthreads();
-  const int seg = lane & 7, grp = lane >> 3;
+// The sums over the wave's pairs, by the FP64 matrix unit: with one operand
+// the lanes' values u and the other a 0 / 1 selector, a product of four 4 x 4
+// blocks adds lanes l, l + 16, l + 32, l + 48 of one coefficient and puts the
+// sum in one of four columns, so four coefficients share a register; a second
+// product, from the other side, adds the four rows of that register into one
+// row, so sixteen coefficients share one (each summed over 16 lanes), and two
+// rotations within rows of 16 lanes finish them.  Exact selectors: the sums
+// round as additions do.  Coefficients are taken in their storage order t =
+// n^2 + n + m, whatever their order n.
+//
+// Lane layout of v_mfma_f64_4x4x4_4b (b = block): A[i][k] in lane i + 4 b +
+// 16 k, B[k][j] in lane j + 4 b + 16 k, D[i][j] in lane j + 4 b + 16 i.
+struct WaveSum {
+  double sel[4];  // sel[i]: 1 in lanes with lane % 4 == i
+  double four, sixteen, out;
+
+  __device__ __forceinline__ void start(int lane) {
 #pragma unroll
-  for (int g = 0; g < (K + 7) / 8; g++) {
-    const int r = g * 8 + grp;
-    const int rr = r < K ? r : K - 1;
-    double sum = 0.0;
-    const double2 *row = reinterpret_cast<const double2 *>(red + rr * kRedStride);
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      double2 t = row[seg + 8 * q];
-      sum += t.x + t.y;
+    for (int i = 0; i < 4; i++) sel[i] = (lane & 3) == i ? 1.0 : 0.0;
+    four = sixteen = out = 0.0;
+  }
+  // coefficient T of NT (compile-time, increasing); dst: the target's row
+  template <int T, int NT>
+  __device__ __forceinline__ void add(double u, double *dst, bool write, int lane) {
+    four = __builtin_amdgcn_mfma_f64_4x4x4f64(u, sel[T % 4], T % 4 == 0 ? 0.0 : four, 0, 0, 0);
+    if constexpr (T % 4 == 3 || T == NT - 1) {
+      constexpr int G = T / 4;
+      sixteen = __builtin_amdgcn_mfma_f64_4x4x4f64(sel[G % 4], four,
+                                                   G % 4 == 0 ? 0.0 : sixteen, 0, 0, 0);
+      if constexpr (G % 4 == 3 || T == NT - 1) {
+        // lane j + 4 b + 16 i: block b's part of coefficient 16 H + 4 i + j
+        constexpr int H = G / 4;
+        double v = sixteen + dpp_move<0x124>(sixteen);
+        v += dpp_move<0x128>(v);
+        out = ((lane >> 2) & 3) == H % 4 ? v : out;
+        if constexpr (H % 4 == 3 || T == NT - 1) {
+          const int t = 64 * (H / 4) + 16 * ((lane >> 2) & 3) + 4 * (lane >> 4) + (lane & 3);
+          if (write && t <= T) atomicAdd(dst + t, out);
+        }
+      }
     }
-    sum += __shfl_xor(sum, 1, kWave);
-    sum += __shfl_xor(sum, 2, kWave);
-    sum += __shfl_xor(sum, 4, kWave);
-    acc_lds[(seg == 0 && r < K) ? N * N + r : nterm(P) + lane] = sum;
   }
+};
+
+template <int N, int NT, int R = 0>
+__device__ __forceinline__ void sum_order(WaveSum &ws, const double *u, double *dst, bool write,
+                                          int lane) {
+  ws.template add<N * N + R, NT>(u[R], dst, write, lane);
+  if constexpr (R < 2 * N) sum_order<N, NT, R + 1>(ws, u, dst, write, lane);
 }
 
-template <int P, int N>
-__device__ __forceinline__ void m2l_backward_order(const double *mp, double &rpn, double ri,
-                                                   double ezr, double ezi, double exr,
-                                                   double exi, double *czp, double *szp,
-                                                   double *cxp, double *sxp, bool active,
-                                                   double *acc_lds, double *red, int lane) {
+// f: translation factors f[j] = j! r^-(j+1), one table for all orders (order N
+// reads j = N..P, so the entries die off as the rotation powers grow).  Up to
+// p = 15 the powers of both angles are such growing tables; above, they would
+// take 4 p doubles and are formed again in every order, as in the forward half.
+template <int P, int LO, int HI, int N>
+__device__ __forceinline__ void m2l_backward_order(const double *mp, const double *ml,
+                                                   const double *f, double ezr, double ezi,
+                                                   double exr, double exi, double *czp,
+                                                   double *szp, double *cxp, double *sxp,
+                                                   WaveSum &ws, double *dst, bool write,
+                                                   int lane) {
+  using Part = M2LPart<P, LO, HI>;
   constexpr int K = 2 * N + 1;
-  constexpr int Q = M2LRegs<P>::q(N);
+  constexpr int Q = Part::q(N);
+  constexpr int TOP = HI < P - N ? HI : P - N;  // source orders LO..TOP reach order N
+  if constexpr (m2l_waves(P) > 1) __syncthreads();
   // one order at a time: keeps the scheduler from interleaving the
   // register-only work of several orders (which multiplies live state)
   __builtin_amdgcn_sched_barrier(0);
-  // translation factors f[N+k] = (N+k)! r^-(N+k+1), k = 0..P-N, from the
-  // power chain r^-(j+1) = r^-j * r^-1 (rpn = r^-(N+1) on entry)
-  double f[P - N + 1];
-  {
-    double rp = rpn;
-#pragma unroll
-    for (int k = 0; k <= P - N; k++) {
-      f[k] = c_fact[N + k] * rp;
-      rp *= ri;
-    }
-    rpn *= ri;
-  }
   double u[K], w[K];
 #pragma unroll
   for (int r = 0; r < K; r++) u[r] = 0.0;
   // translation along z (kernel_fast_lean.h:1253-1295):
   // L_n^{+-m} += (-1)^m sum_{k=m}^{p-n} M_k^{+-m} (n+k)! r^-(n+k+1)
 #pragma unroll
-  for (int k = 0; k <= P - N; k++) {
-    const int qk = M2LRegs<P>::q(k);
-    const int ok = M2LRegs<P>::off(k);
-    u[N] += mp[ok + qk] * f[k];
-  }
+  for (int k = LO; k <= TOP; k++) u[N] += kept<Part>(mp, ml, k, 0) * f[N + k];
 #pragma unroll
   for (int m = 1; m <= Q; m++) {
 #pragma unroll
-    for (int k = m; k <= P - N; k++) {
-      const int qk = M2LRegs<P>::q(k);
-      const int ok = M2LRegs<P>::off(k);
-      double fk = (m & 1) ? -f[k] : f[k];
-      u[N - m] += mp[ok + qk - m] * fk;
-      u[N + m] += mp[ok + qk + m] * fk;
+    for (int k = LO; k <= TOP; k++) {
+      if (m > m2l_q(P, k)) continue;
+      const double fk = (m & 1) ? -f[N + k] : f[N + k];
+      u[N - m] += kept<Part>(mp, ml, k, -m) * fk;
+      u[N + m] += kept<Part>(mp, ml, k, m) * fk;
     }
   }
-  extend_powers<N>(cxp, sxp, exr, exi);
-  extend_powers<N>(czp, szp, ezr, ezi);
-  swap_block<N, N, Q>(u, w);
-  rotate_tab<N, true>(w, cxp, sxp);
-  swap_block<N, N, N>(w, u);
-  rotate_tab<N, true>(u, czp, szp);
-  if constexpr (RedBuf<P>::pipelined) {
-    // The previous order's rows were written one order ago: reduce them now,
-    // so the barrier finds those writes long complete; then store this
-    // order's rows in the other buffer (reduced after the next order, or at
-    // the end).
-    if constexpr (N > 0)
-      reduce_order<P, N - 1>(red + ((N - 1) & 1) * RedBuf<P>::size, acc_lds, lane);
-#pragma unroll
-    for (int r = 0; r < K; r++) red[(N & 1) * RedBuf<P>::size + r * kRedStride + lane] = u[r];
-    if constexpr (N == P) reduce_order<P, N>(red + (N & 1) * RedBuf<P>::size, acc_lds, lane);
-  } else {
-#pragma unroll
-    for (int r = 0; r < K; r++) red[r * kRedStride + lane] = u[r];
-    reduce_order<P, N>(red, acc_lds, lane);
-    __syncthreads();
+  constexpr bool kTab = P <= 15;
+  if constexpr (kTab) {
+    extend_powers<N>(cxp, sxp, exr, exi);
+    extend_powers<N>(czp, szp, ezr, ezi);
   }
+  swap_block<N, N, Q>(u, w);
+  if constexpr (kTab)
+    rotate_tab<N, true>(w, cxp, sxp);
+  else
+    rotate<N, true>(w, exr, exi);
+  swap_block<N, N, N>(w, u);
+  if constexpr (kTab)
+    rotate_tab<N, true>(u, czp, szp);
+  else
+    rotate<N, true>(u, ezr, ezi);
+  sum_order<N, (Part::top + 1) * (Part::top + 1)>(ws, u, dst, write, lane);
 }
 
-template <int P, int... Ns>
-__device__ __forceinline__ void m2l_backward_all(const double *mp, double rpn, double ri,
-                                                 double ezr, double ezi, double exr, double exi,
-                                                 bool active, double *acc, double *red,
+template <int P, int LO, int HI, int... Ns>
+__device__ __forceinline__ void m2l_backward_all(const double *mp, const double *ml,
+                                                 const double *f, double ezr, double ezi,
+                                                 double exr, double exi, double *dst, bool write,
                                                  int lane, IntSeq<Ns...>) {
+  WaveSum ws;
+  ws.start(lane);
   double czp[P + 1], szp[P + 1], cxp[P + 1], sxp[P + 1];
-  (m2l_backward_order<P, Ns>(mp, rpn, ri, ezr, ezi, exr, exi, czp, szp, cxp, sxp, active, acc,
-                             red, lane),
+  (m2l_backward_order<P, LO, HI, Ns>(mp, ml, f, ezr, ezi, exr, exi, czp, szp, cxp, sxp, ws, dst,
+                                     write, lane),
    ...);
 }
 
+// Source orders LO..HI of the chunk's pairs, added to the target's row dst.
+template <int P, int LO, int HI>
+__device__ __forceinline__ void m2l_part(const double *__restrict__ src, bool quirk, double ezr,
+                                         double ezi, double exr, double exi, double ri,
+                                         bool active, double *dst, bool write, int lane,
+                                         double *ml) {
+  using Part = M2LPart<P, LO, HI>;
+  // Orders run from HI down: the large orders (biggest working set) run while
+  // few rotated moments are live.
+  double mp[Part::store.regs], v0[2 * HI + 1];
+  load_order<HI>(src, v0);
+  m2l_forward_order<P, LO, HI, HI>(src, quirk, ezr, ezi, exr, exi, v0, mp, ml);
+  // Fence the rotated moments: without it, IR-level code motion interleaves
+  // the forward and backward halves and roughly doubles the live registers
+  // (p = 12: 512 registers plus scratch spills instead of ~310, no spills).
+#pragma unroll
+  for (int t = 0; t < Part::store.regs; t++) asm volatile("" : "+v"(mp[t]));
+  __builtin_amdgcn_sched_barrier(0);
+  // translation factors j! r^-(j+1); zero on idle lanes, which zeroes their
+  // whole contribution
+  double f[P + 1];
+  {
+    double rp = active ? ri : 0.0;
+#pragma unroll
+    for (int k = 0; k <= P; k++) {
+      f[k] = c_fact[k] * rp;
+      rp *= ri;
+    }
+  }
+  m2l_backward_all<P, LO, HI>(mp, ml, f, ezr, ezi, exr, exi, dst, write, lane,
+                              MakeIntSeq<Part::top + 1>{});
+}
+
 template <int P>
-__global__ __launch_bounds__(64) void k_m2l(const int4 *__restrict__ chunks,
-                                            const int *__restrict__ src_list,
-                                            const double *__restrict__ cX,
-                                            const unsigned char *__restrict__ has_sink,
-                                            const double *__restrict__ M,
-                                            const double *__restrict__ Md,
-                                            double *__restrict__ L, double *__restrict__ Ld,
-                                            int quirk, int stride) {
-  constexpr int NT = nterm(P);
-  __shared__ double acc[NT + kWave];  // + one spare slot per lane
-  __shared__ __attribute__((aligned(16))) double red[RedBuf<P>::count * RedBuf<P>::size];
-  const int lane = threadIdx.x;
-  // (chunk, array) from the linear block id, contiguous per XCD
-  const int nchunk = gridDim.x;
-  const int item = xcd_contiguous(blockIdx.y * nchunk + blockIdx.x, 2 * nchunk);
+__global__ __launch_bounds__(64 * m2l_waves(P))
+    __attribute__((amdgpu_waves_per_eu(m2l_occ(P) > 0 ? m2l_occ(P) : 1))) void k_m2l(
+    const int4 *__restrict__ chunks, int nchunk, const int *__restrict__ src_list,
+    const double *__restrict__ cX, const unsigned char *__restrict__ has_sink,
+    const double *__restrict__ M, const double *__restrict__ Md, double *__restrict__ L,
+    double *__restrict__ Ld, int quirk, int stride) {
+  constexpr int W = m2l_waves(P);
+  const int lane = threadIdx.x & (kWave - 1);
+  // (chunk, array) from the linear block id, contiguous per XCD; waves past
+  // the last item, or whose target has no sink, repeat a chunk and write
+  // nothing (a block of such waves ends at once)
+  const int first = xcd_contiguous(blockIdx.x, gridDim.x) * W;
+  auto live = [&](int k) { return k < 2 * nchunk && has_sink[chunks[k % nchunk].x]; };
+  bool any = false;
+#pragma unroll
+  for (int k = 0; k < W; k++) any |= live(first + k);
+  if (!any) return;
+  const int mine = first + __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+  const bool write = W == 1 || live(mine);
+  const int item = min(mine, 2 * nchunk - 1);
   const int which = item >= nchunk;
   const int4 ch = chunks[item - which * nchunk];
   const int tgt = ch.x, start = ch.y, cnt = ch.z;
-  if (!has_sink[tgt]) return;
   const double *Msrc = which ? Md : M;
   double *Lout = which ? Ld : L;
   const bool active = lane < cnt;
@@ -390,33 +474,18 @@ __global__ __launch_bounds__(64) void k_m2l(const int4 *__restrict__ chunks,
     ezr = dy * q;
     ezi = dx * q;
   }
-  double mp[M2LRegs<P>::total];
+  constexpr int S = m2l_split(P);
+  constexpr int kSlots = std::max(M2LPart<P, S + 1, P>::store.slots,
+                                  S >= 0 ? M2LPart<P, 0, S >= 0 ? S : P>::store.slots : 0);
+  __shared__ double s_mp[kSlots > 0 ? W * kSlots * kWave : 1];
+  double *ml = s_mp + (kSlots > 0 ? ((int)threadIdx.x / kWave) * kSlots * kWave + lane : 0);
   const double *src = Msrc + (size_t)j * stride;
-  // Orders run from p down to 0: the large orders (biggest working set) run
-  // while few rotated moments are live.
-  // orders P .. P-kAhead+1 are gathered up front
-  double v0[OrderBuf<P>::size], v1[OrderBuf<P - 1>::size], v2[OrderBuf<P - 2>::size],
-      v3[OrderBuf<P - 3>::size];
-  load_order<P>(src, v0);
-  if constexpr (kAhead >= 2 && P - 1 >= 0) load_order<P - 1>(src, v1);
-  if constexpr (kAhead >= 3 && P - 2 >= 0) load_order<P - 2>(src, v2);
-  if constexpr (kAhead >= 4 && P - 3 >= 0) load_order<P - 3>(src, v3);
-  m2l_forward_order<P, P>(src, quirk != 0, ezr, ezi, exr, exi, v0, v1, v2, v3, mp);
-  // Fence the rotated moments: without it, IR-level code motion interleaves
-  // the forward and backward halves and roughly doubles the live registers
-  // (p = 12: 512 registers plus scratch spills instead of ~310, no spills).
-#pragma unroll
-  for (int t = 0; t < M2LRegs<P>::total; t++) asm volatile("" : "+v"(mp[t]));
-  __builtin_amdgcn_sched_barrier(0);
-  // translation factors (n+k)! r^-(n+k+1) are formed per order from the power
-  // chain starting at r^-1; zero on idle lanes, which zeroes their whole
-  // contribution
-  const double rp0 = active ? ri : 0.0;
-  m2l_backward_all<P>(mp, rp0, ri, ezr, ezi, exr, exi, active, acc, red, lane,
-                      MakeIntSeq<P + 1>{});
-  __syncthreads();
   double *dst = Lout + (size_t)tgt * stride;
-  for (int t = lane; t < NT; t += kWave) atomicAdd(dst + t, acc[t]);
+  m2l_part<P, S + 1, P>(src, quirk != 0, ezr, ezi, exr, exi, ri, active, dst, write, lane, ml);
+  if constexpr (S >= 0) {
+    __builtin_amdgcn_sched_barrier(0);
+    m2l_part<P, 0, S>(src, false, ezr, ezi, exr, exi, ri, active, dst, write, lane, ml);
+  }
 }
 
 void m2l_init_tables(int p, int quirk) {
@@ -433,8 +502,9 @@ void m2l_init_tables(int p, int quirk) {
 template <int P>
 static void launch(const M2LArgs &a, hipStream_t s) {
   if (a.nchunks <= 0) return;
-  dim3 grid(a.nchunks, 2);
-  hipLaunchKernelGGL(k_m2l<P>, grid, dim3(64), 0, s, a.chunks, a.src, a.cX, a.has_sink, a.M,
+  constexpr int W = m2l_waves(P);
+  const dim3 grid((2 * a.nchunks + W - 1) / W);
+  hipLaunchKernelGGL(k_m2l<P>, grid, dim3(64 * W), 0, s, a.chunks, a.nchunks, a.src, a.cX, a.has_sink, a.M,
                      a.Md, a.L, a.Ld, a.quirk, a.stride > 0 ? a.stride : nterm(P));
 }
 
