@@ -121,7 +121,7 @@ struct Batch {
   CellsDev cells() const {
     // the tree geometry (Xg, Rg) is not part of a Cell record; the ball stands in
     return {level.as<int>(), dnchild.as<int>(), dchild.as<int>(), dbody.as<int>(),
-            dnbody.as<int>(), dX.as<double>(), dR.as<double>(), dX.as<double>(),
+            dnbody.as<int>(), nullptr, dX.as<double>(), dR.as<double>(), dX.as<double>(),
             dR.as<double>(), dmin.as<double>(), dsink.as<unsigned char>(), dM.as<double>(),
             dMd.as<double>(), dL.as<double>(), dLd.as<double>()};
   }

@@ -11,7 +11,7 @@ namespace tcfmm {
   int launch_m2m(int p, CellsDev c, BodiesDev b, int ls, int le, hipStream_t s, int what);    \
   int launch_m2m_ids(int p, CellsDev c, BodiesDev b, const int *ids, int nids, hipStream_t s); \
   int launch_m2l(int p, const M2LArgs &a, hipStream_t s);                                     \
-  int launch_l2l(int p, CellsDev c, int ls, int le, hipStream_t s);                           \
+  int launch_l2l(int p, CellsDev c, int ls, int le, bool beside, hipStream_t s);              \
   int launch_l2l_ids(int p, CellsDev c, const int *ids, int nids, hipStream_t s);             \
   int launch_l2p(int p, CellsDev c, BodiesDev b, ResultsDev r, const int *leaf_ids,           \
                  int nleaves, hipStream_t s, bool add);
@@ -49,8 +49,8 @@ int launch_m2m_ids(int p, CellsDev c, BodiesDev b, const int *ids, int nids, hip
   TC_ROUTE(launch_m2m_ids(p, c, b, ids, nids, s))
 }
 int launch_m2l(int p, const M2LArgs &a, hipStream_t s) { TC_ROUTE(launch_m2l(p, a, s)) }
-int launch_l2l(int p, CellsDev c, int ls, int le, hipStream_t s) {
-  TC_ROUTE(launch_l2l(p, c, ls, le, s))
+int launch_l2l(int p, CellsDev c, int ls, int le, bool beside, hipStream_t s) {
+  TC_ROUTE(launch_l2l(p, c, ls, le, beside, s))
 }
 int launch_l2l_ids(int p, CellsDev c, const int *ids, int nids, hipStream_t s) {
   TC_ROUTE(launch_l2l_ids(p, c, ids, nids, s))

@@ -5,16 +5,18 @@
 //
 //   L2L (kernel_fast_lean.h:1001-1058): for each child,
 //       L_child[n,m] += sum_{k<=p-n} sum_{|l|<=k} L[n+k, m+l] conj Y_k^l(X - X_child)
-//       two blocks of 256 threads per parent cell, four children each: 64
-//       threads per child, each thread a strided share of the child's (output
-//       term, L or Ldot) tasks; the four harmonic tables and the parent's
-//       expansion sit in LDS (16 KB at p = 12).  The P2P kernel running
-//       alongside holds 12 one-wave blocks per CU (154 KB of LDS, all but 8
-//       VGPRs per SIMD lane), so a level launched while it runs waits for its
-//       blocks to drain.  A task's sum runs over contiguous runs of both
-//       tables, two terms at a time into two partial sums: the top levels are
-//       a few blocks each, and their time (35-40 us) is that of one thread's
-//       chain of LDS reads and adds.
+//       one block per child, with the harmonic table and the parent's
+//       expansions in LDS (8 KB at p = 12); each thread takes a share of the
+//       output terms, whose sums run over contiguous runs of both tables, two
+//       terms at a time into two partial sums.  The levels are a chain, and a
+//       level of a few blocks takes the latency of one thread's sums, so there
+//       are two shapes:
+//       * one wave per child.  Beside a long P2P launch only blocks that fit
+//         the slot of one finished P2P wave get in: levels of 256-thread
+//         blocks waited for P2P's last blocks (at N = 2^20 the pass ended
+//         1.4 ms after P2P; now it ends 4 ms before P2P does).
+//       * 512 threads per child, two per output, on levels of at most 1,024
+//         cells where P2P is short: a level 35 -> 13 us at p = 12.
 //   L2P (kernel_fast_lean.h:1060-1128): two leaves per wave, 32 lanes each
 //       (leaves average ~19 bodies: one leaf per wave left 70% of the lanes
 //       idle); lane = body, Y = Y(X_c - x_b) and
@@ -33,49 +35,51 @@
 namespace tcfmm {
 namespace TC_SHARD_NS(TC_SHARD) {
 
-template <int P>
-__global__ __launch_bounds__(256) void k_l2l(CellsDev c, const int *__restrict__ ids, int ls) {
+// T threads per child, S of them sharing each output's sum (over every S-th
+// source order).  ids (or null): parents, eight blocks each, block 8 i + k for
+// child k; otherwise the blocks are the cells from `first` on.
+template <int P, int T, int S>
+__global__ __launch_bounds__(T) void k_l2l(CellsDev c, const int *__restrict__ ids, int first) {
   constexpr int NT = nterm(P);
   constexpr int NO = tri(P, P) + 1;
-  constexpr int kGroup = 64;  // threads per child
-  static_assert(P + 1 <= kGroup, "one thread per harmonic column");
-  __shared__ cplx G[4][NT], cl[NT], cld[NT];
-  const int tid = threadIdx.x;
-  const int cell = blockIdx.x >> 1, half = blockIdx.x & 1;
-  const int ci = ids ? ids[cell] : ls + cell;
-  const int nch = c.nchild[ci] - 4 * half;  // children of this block's half
-  if (nch <= 0) return;
-  const int ch0 = c.child[ci] + 4 * half;
+  static_assert(P + 1 <= T && T % kWave == 0 && (S == 1 || S == 2), "shape");
+  __shared__ cplx G[NT], cl[NT], cld[NT];
+  const int u = threadIdx.x;
+  int ci, ch;
+  if (ids) {
+    ci = ids[blockIdx.x >> 3];
+    if ((int)(blockIdx.x & 7) >= c.nchild[ci]) return;
+    ch = c.child[ci] + (blockIdx.x & 7);
+  } else {
+    ch = first + blockIdx.x;
+    ci = c.parent[ch];
+  }
   const double *Lp = c.L + (size_t)ci * NT;
   const double *Ldp = c.Ld + (size_t)ci * NT;
-  for (int t = tid; t < NT; t += blockDim.x) {
+  for (int t = u; t < NT; t += T) {
     int n = 0;
     while ((n + 1) * (n + 1) <= t) n++;
     const int m = t - n * n - n;
     cl[t] = packed_to_c(Lp, n, m);
     cld[t] = packed_to_c(Ldp, n, m);
   }
-  const int k = tid / kGroup, u = tid - k * kGroup;
-  const int ch = ch0 + k;
-  if (k < nch)
-    harm_table_col<P>(u, c.X[3 * ci] - c.X[3 * ch], c.X[3 * ci + 1] - c.X[3 * ch + 1],
-                      c.X[3 * ci + 2] - c.X[3 * ch + 2], G[k]);
+  harm_table_col<P>(u, c.X[3 * ci] - c.X[3 * ch], c.X[3 * ci + 1] - c.X[3 * ch + 1],
+                    c.X[3 * ci + 2] - c.X[3 * ch + 2], G);
   __syncthreads();
-  if (k >= nch) return;
   double *Lc = c.L + (size_t)ch * NT;
   double *Ldc = c.Ld + (size_t)ch * NT;
-  const cplx *Gk = G[k];
-  // tasks (output term, L or Ldot) of this child, strided over the group
-  for (int j = u; j < 2 * NO; j += kGroup) {
+  // tasks (output term, L or Ldot), strided over the block
+  const int part = S > 1 ? u & 1 : 0;
+  for (int j = u / S; j < 2 * NO; j += T / S) {
     const int which = j >= NO, o = j - which * NO;
     int n = 0;
     while (tri(n + 1, 0) <= o) n++;
     const int m = o - tri(n, 0);
     const cplx *src = which ? cld : cl;
     cplx a = {0, 0}, a2 = {0, 0};
-    for (int kk = 0; kk <= P - n; kk++) {
-      // l = -kk..kk: src[ixnm(n + kk, m + l)] and Gk[ixnm(kk, l)] run contiguously
-      const cplx *sr = src + ixnm(n + kk, m - kk), *gr = Gk + ixnm(kk, -kk);
+    for (int kk = part; kk <= P - n; kk += S) {
+      // l = -kk..kk: src[ixnm(n + kk, m + l)] and G[ixnm(kk, l)] run contiguously
+      const cplx *sr = src + ixnm(n + kk, m - kk), *gr = G + ixnm(kk, -kk);
       const int len = 2 * kk + 1;
       int t = 0;
       for (; t + 1 < len; t += 2) {
@@ -85,10 +89,16 @@ __global__ __launch_bounds__(256) void k_l2l(CellsDev c, const int *__restrict__
       if (t < len) a = cadd(a, cmul(sr[t], cconj(gr[t])));
     }
     a = cadd(a, a2);
-    double *dst = which ? Ldc : Lc;
-    const int s = n * n + n;
-    dst[s + m] += a.re;
-    if (m > 0) dst[s - m] += a.im;
+    if (S > 1) {
+      a.re += dpp_move<0xb1>(a.re);  // the neighbour's part (lanes 2 i, 2 i + 1)
+      a.im += dpp_move<0xb1>(a.im);
+    }
+    if (part == 0) {
+      double *dst = which ? Ldc : Lc;
+      const int s = n * n + n;
+      dst[s + m] += a.re;
+      if (m > 0) dst[s - m] += a.im;
+    }
   }
 }
 
@@ -231,8 +241,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(P <= 12 ? 3 
 }
 
 template <int P>
-static void l2l_go(CellsDev c, const int *ids, int ls, int ncell, hipStream_t s) {
-  hipLaunchKernelGGL(k_l2l<P>, dim3(2 * ncell), dim3(256), 0, s, c, ids, ls);
+static void l2l_go(CellsDev c, const int *ids, int first, int nblocks, bool wide, hipStream_t s) {
+  if (wide)
+    hipLaunchKernelGGL((k_l2l<P, 512, 2>), dim3(nblocks), dim3(512), 0, s, c, ids, first);
+  else
+    hipLaunchKernelGGL((k_l2l<P, 64, 1>), dim3(nblocks), dim3(64), 0, s, c, ids, first);
 }
 template <int P>
 static void l2p_go(CellsDev c, BodiesDev b, ResultsDev r, const int *ids, int n, bool add,
@@ -244,13 +257,23 @@ static void l2p_go(CellsDev c, BodiesDev b, ResultsDev r, const int *ids, int n,
     hipLaunchKernelGGL((k_l2p<P, false>), g, t, 0, s, c, b, r, ids, n);
 }
 
-int launch_l2l(int p, CellsDev c, int ls, int le, hipStream_t s) {
+// Whether a level of `cells` takes 512 threads per cell: up to 1,024 cells
+// (four blocks a CU), and at any size above p = 13, where the tables (48 bytes
+// a coefficient) leave room for few one-wave blocks on a CU (p = 20, N = 2^17:
+// the three widest levels 108, 197, 207 us with one wave per cell, 52, 80, 109
+// with eight).
+template <int P>
+constexpr bool l2l_wide(int cells) {
+  return cells <= 1024 || 48 * nterm(P) > 10 * 1024;
+}
+
+int launch_l2l(int p, CellsDev c, int ls, int le, bool beside, hipStream_t s) {
   if (le <= ls) return 0;
   switch (p) {
 #define TC_CASE(P)\
   case P:\
     if constexpr (in_shard(P, TC_SHARD)) {\
-      l2l_go<P>(c, nullptr, ls, le - ls, s);\
+      l2l_go<P>(c, nullptr, ls, le - ls, !beside && l2l_wide<P>(le - ls), s);\
       return 0;\
     } else {\
       return -1;\
@@ -268,7 +291,7 @@ int launch_l2l_ids(int p, CellsDev c, const int *ids, int nids, hipStream_t s) {
 #define TC_CASE(P)\
   case P:\
     if constexpr (in_shard(P, TC_SHARD)) {\
-      l2l_go<P>(c, ids, 0, nids, s);\
+      l2l_go<P>(c, ids, 0, 8 * nids, l2l_wide<P>(8 * nids), s);\
       return 0;\
     } else {\
       return -1;\

@@ -113,7 +113,7 @@ struct tc_context {
   DBuf key_hi, key_a, key_b, val_a, val_b, sort_tmp, part, tp, dshift;
   // cells
   int cap_c = 0;
-  DBuf clevel, cnchild, cchild, cbody, cnbody, cXg, cRg, cX, cR, cmin, csink;
+  DBuf clevel, cnchild, cchild, cbody, cnbody, cparent, cXg, cRg, cX, cR, cmin, csink;
   DBuf cM, cMd, cL, cLd;
   DBuf split_offs, split_nch, split_scan, scan_tmp;
   std::vector<int> level_start;
@@ -264,7 +264,8 @@ inline BodiesDev bodies_of(tc_context *ctx) {
 
 inline CellsDev cells_of(tc_context *ctx) {
   return {ctx->clevel.as<int>(), ctx->cnchild.as<int>(), ctx->cchild.as<int>(),
-          ctx->cbody.as<int>(),  ctx->cnbody.as<int>(),  ctx->cXg.as<double>(),
+          ctx->cbody.as<int>(),  ctx->cnbody.as<int>(),  ctx->cparent.as<int>(),
+          ctx->cXg.as<double>(),
           ctx->cRg.as<double>(), ctx->cX.as<double>(),   ctx->cR.as<double>(),
           ctx->cmin.as<double>(), ctx->csink.as<unsigned char>(), ctx->cM.as<double>(),
           ctx->cMd.as<double>(), ctx->cL.as<double>(),   ctx->cLd.as<double>()};

@@ -55,6 +55,7 @@ static int ensure_cells(tc_context *ctx, int nc, int keep) {
   TC_CHECK(ctx->clevel.ensure(sizeof(int) * cap, ki, s));
   TC_CHECK(ctx->cnchild.ensure(sizeof(int) * cap, ki, s));
   TC_CHECK(ctx->cchild.ensure(sizeof(int) * cap, ki, s));
+  TC_CHECK(ctx->cparent.ensure(sizeof(int) * cap, ki, s));
   TC_CHECK(ctx->cbody.ensure(sizeof(int) * cap, ki, s));
   TC_CHECK(ctx->cnbody.ensure(sizeof(int) * cap, ki, s));
   TC_CHECK(ctx->cXg.ensure(sizeof(double) * 3 * cap, 3 * kd, s));
@@ -318,7 +319,32 @@ static int build_csr(tc_context *ctx, const int2 *pairs, int npairs, DBuf &cnt, 
   return 0;
 }
 
-static int build_lists(tc_context *ctx, int &nchunks) {
+static int build_p2p_items(tc_context *ctx);
+
+// The near field on near_stream, queued after the P2P list's grouping: ranges
+// and cleared results, work items (built on the host once the list's lengths
+// are there), P2P.  after (or null): an event that P2P waits for.
+static int near_field(tc_context *ctx, int n, hipEvent_t after) {
+  hipStream_t s2 = ctx->near_stream;
+  const ResultsDev r = results_of(ctx);
+  TC_CHECK(ctx->p2p_ranges.ensure(sizeof(int2) * (size_t)std::max<long long>(ctx->st.n_p2p_cells, 1)));
+  TC_CHECK(ctx->npairs.ensure(sizeof(unsigned long long)));
+  launch_p2p_setup(cells_of(ctx), ctx->p2p_src.as<int>(), (int)ctx->st.n_p2p_cells,
+                   ctx->p2p_ranges.as<int2>(), r, n, ctx->npairs.as<unsigned long long>(), s2);
+  if (int e = build_p2p_items(ctx)) return e;
+  if (after) TC_CHECK(hipStreamWaitEvent(s2, after, 0));
+  TC_CHECK(hipEventRecord(ctx->ev[9], s2));
+  launch_p2p(cells_of(ctx), bodies_of(ctx), r, ctx->p2p_items.as<int4>(), (int)ctx->n_items,
+             ctx->p2p_off.as<int>(), ctx->p2p_cnt.as<int>(), ctx->p2p_ranges.as<int2>(),
+             ctx->npairs.as<unsigned long long>(), s2, ctx->p2p_mode, ctx->close_radius,
+             ctx->p2p_tile, p2p_targets_per_lane(ctx->p2p_mode, ctx->p2p_per_lane));
+  TC_CHECK(hipEventRecord(ctx->ev[10], s2));
+  ctx->p2p_ready = true;
+  return 0;
+}
+
+// near: also queue the near field (n bodies) as soon as its list is grouped
+static int build_lists(tc_context *ctx, int &nchunks, bool near = false, int n = 0) {
   hipStream_t s = ctx->stream;
   int nc = ctx->st.ncells;
   // the P2P list on near_stream meanwhile (after the walk that wrote it), with
@@ -341,7 +367,10 @@ static int build_lists(tc_context *ctx, int &nchunks) {
     return -4;
   TC_CHECK(hipMemcpyAsync(ctx->h_pin + 10, ctx->m2l_coff.as<int>() + nc, sizeof(int),
                           hipMemcpyDeviceToHost, s));
-  TC_CHECK(spin_wait(ctx, s));
+  TC_CHECK(hipEventRecord(ctx->ev_wait, s));
+  if (near)
+    if (int e = near_field(ctx, n, nullptr)) return e;
+  TC_CHECK(spin_event(ctx->ev_wait));
   nchunks = ctx->h_pin[10];
   TC_CHECK(ctx->m2l_chunks.ensure(sizeof(int4) * (size_t)std::max(nchunks, 1)));
   launch_make_chunks(ctx->m2l_off.as<int>(), ctx->m2l_cnt.as<int>(), ctx->m2l_coff.as<int>(), nc,
@@ -353,9 +382,8 @@ static int build_lists(tc_context *ctx, int &nchunks) {
 // (fewer where the whole list is short).
 // Each leaf is cut into target groups of <= 64 bodies by the lane model of
 // the kernel (P2PSplit).  The per-leaf list lengths were copied to pinned
-// memory before the M2L launch (and the stream synchronized after that
-// copy), so this host loop runs while the GPU is busy with M2L; the upload is
-// queued behind it.
+// memory on near_stream, where the upload is queued too; the host loop runs
+// while the GPU groups the M2L list or runs M2L.
 static int build_p2p_items(tc_context *ctx) {
   // Slices so that even a small system's list makes thousands of items: a
   // wave's time is its chain of tiles, and two or three waves a SIMD leave the
@@ -397,7 +425,7 @@ static int build_p2p_items(tc_context *ctx) {
   ctx->n_items = nitem;
   TC_CHECK(ctx->p2p_items.ensure(sizeof(int4) * std::max<size_t>(nitem, 1)));
   TC_CHECK(hipMemcpyAsync(ctx->p2p_items.p, items, sizeof(int4) * nitem, hipMemcpyHostToDevice,
-                          ctx->stream));
+                          ctx->near_stream));
   return 0;
 }
 
@@ -761,8 +789,13 @@ static int eval_device(tc_context *ctx, int n, const double *x, const double *v,
     if (int e = traverse(ctx, n, mac_args(ctx, err_mac ? kMacError : kMacTheta))) return e;
   }
   TC_CHECK(hipEventRecord(ctx->ev[3], s));
+  // P2P takes about 1 ms per million list entries.  A short one runs as soon as
+  // its list is there, beside the M2L list's grouping, whose small sorts leave
+  // the chip idle, and is out of the way of the downward pass; a long one runs
+  // after M2L and hides the downward pass.
+  const bool near_late = ctx->st.n_p2p_cells > 1000000;
   int nchunks = 0;
-  if (int e = build_lists(ctx, nchunks)) return e;
+  if (int e = build_lists(ctx, nchunks, !near_late, n)) return e;
   if (!err_mac) TC_CHECK(hipStreamWaitEvent(s, ctx->ev[13], 0));  // the moments
   TC_CHECK(hipEventRecord(ctx->ev[4], s));
   // ---- far field
@@ -786,42 +819,24 @@ static int eval_device(tc_context *ctx, int n, const double *x, const double *v,
     }
     ctx->m2l_by_order[cfg.p] = ctx->st.n_m2l;
   }
-  // the near field's set-up on the second stream, beside M2L: it reads only
-  // the tree and the P2P list (already queued on that stream)
-  hipStream_t s2 = ctx->near_stream;
-  ResultsDev r = results_of(ctx);
-  TC_CHECK(ctx->p2p_ranges.ensure(sizeof(int2) * (size_t)std::max<long long>(ctx->st.n_p2p_cells, 1)));
-  TC_CHECK(ctx->npairs.ensure(sizeof(unsigned long long)));
-  launch_p2p_setup(cells_of(ctx), ctx->p2p_src.as<int>(), (int)ctx->st.n_p2p_cells,
-                   ctx->p2p_ranges.as<int2>(), r, n, ctx->npairs.as<unsigned long long>(), s2);
-  // the GPU runs M2L while the host builds the P2P work items
-  if (int e = build_p2p_items(ctx)) return e;
   TC_CHECK(hipEventRecord(ctx->ev[5], s));
-  // ---- near field on the second stream, after M2L (and the work-item upload
-  // queued behind it), alongside the downward pass
-  TC_CHECK(hipStreamWaitEvent(s2, ctx->ev[5], 0));
-  TC_CHECK(hipEventRecord(ctx->ev[9], s2));
-  launch_p2p(cells_of(ctx), bodies_of(ctx), r, ctx->p2p_items.as<int4>(),
-             (int)ctx->n_items, ctx->p2p_off.as<int>(), ctx->p2p_cnt.as<int>(),
-             ctx->p2p_ranges.as<int2>(), ctx->npairs.as<unsigned long long>(), s2,
-             ctx->p2p_mode, ctx->close_radius, ctx->p2p_tile,
-             p2p_targets_per_lane(ctx->p2p_mode, ctx->p2p_per_lane));
-  TC_CHECK(hipEventRecord(ctx->ev[10], s2));
-  ctx->p2p_ready = true;
+  // the GPU runs M2L while the host builds the P2P work items
+  if (near_late)
+    if (int e = near_field(ctx, n, ctx->ev[5])) return e;
   // ---- downward into the far-field result set
   ResultsDev rf = {ctx->fpot.as<double>(), ctx->fax.as<double>(), ctx->fay.as<double>(),
                    ctx->faz.as<double>(), ctx->fjx.as<double>(), ctx->fjy.as<double>(),
                    ctx->fjz.as<double>()};
   int L = (int)ctx->level_start.size() - 1;
-  for (int l = 0; l < L; l++)
-    launch_l2l(cfg.p, cells_of(ctx), ctx->level_start[l], ctx->level_start[l + 1], s);
+  for (int l = 1; l < L; l++)
+    launch_l2l(cfg.p, cells_of(ctx), ctx->level_start[l], ctx->level_start[l + 1], near_late, s);
   launch_l2p(cfg.p, cells_of(ctx), bodies_of(ctx), rf, ctx->leaf_ids.as<int>(), ctx->nleaves, s,
              false);
   TC_CHECK(hipEventRecord(ctx->ev[6], s));
   TC_CHECK(hipStreamWaitEvent(s, ctx->ev[10], 0));
   // (with the body pairs evaluated by P2P: statistics, counted inside that kernel)
   const auto *pairs = reinterpret_cast<const unsigned long long *>(ctx->h_pin + 52);
-  launch_scatter_results_sum(bodies_of(ctx), r, rf, n, pot, acc, jerk,
+  launch_scatter_results_sum(bodies_of(ctx), results_of(ctx), rf, n, pot, acc, jerk,
                              ctx->npairs.as<unsigned long long>(),
                              reinterpret_cast<unsigned long long *>(ctx->h_pin_dev + 52), s);
   TC_CHECK(hipEventRecord(ctx->ev[7], s));
@@ -960,8 +975,8 @@ static int master_fmm_device(tc_context *ctx, int n, bool steps, bool pair_mass,
   TC_CHECK(hipEventRecord(ctx->ev[6], s));
   // ---- downward
   int L = (int)ctx->level_start.size() - 1;
-  for (int l = 0; l < L; l++)
-    launch_l2l(cfg.p, c, ctx->level_start[l], ctx->level_start[l + 1], s);
+  for (int l = 1; l < L; l++)
+    launch_l2l(cfg.p, c, ctx->level_start[l], ctx->level_start[l + 1], false, s);
   launch_l2p(cfg.p, c, b, r, ctx->leaf_ids.as<int>(), ctx->nleaves, s);
   launch_scatter_results(b, r, n, pot, acc, nullptr, s);
   if (steps) launch_scatter_ts(b, ctx->mts_sorted.as<double>(), n, tstep, s);
@@ -1211,7 +1226,7 @@ int tc_destroy(tc_context *ctx) {
                  &ctx->bflags, &ctx->border, &ctx->bacc, &ctx->rpot, &ctx->rax, &ctx->ray,
                  &ctx->raz, &ctx->rjx, &ctx->rjy, &ctx->rjz, &ctx->key_hi, &ctx->key_a,
                  &ctx->key_b, &ctx->val_a, &ctx->val_b, &ctx->sort_tmp, &ctx->part, &ctx->tp,
-                 &ctx->dshift, &ctx->clevel, &ctx->cnchild, &ctx->cchild, &ctx->cbody,
+                 &ctx->dshift, &ctx->clevel, &ctx->cnchild, &ctx->cchild, &ctx->cparent, &ctx->cbody,
                  &ctx->cnbody, &ctx->cXg, &ctx->cRg, &ctx->cX, &ctx->cR, &ctx->cmin, &ctx->csink,
                  &ctx->cM, &ctx->cMd, &ctx->cL, &ctx->cLd, &ctx->split_offs, &ctx->split_nch,
                  &ctx->split_scan, &ctx->scan_tmp, &ctx->leaf_ids, &ctx->front_a, &ctx->front_b,
@@ -1365,7 +1380,7 @@ int tc_tune_p2p(tc_context *ctx, int reps, double *best_ms, double *default_ms,
     ctx->p2p_list = list;
     ctx->p2p_stage = stage;
     if (int e = build_p2p_items(ctx)) return e;
-    TC_CHECK(hipStreamSynchronize(ctx->stream));  // the item upload
+    TC_CHECK(hipStreamSynchronize(s2));  // the item upload
     float best = 1e30f;
     for (int r = 0; r < reps; r++) {
       TC_CHECK(hipEventRecord(ctx->ev[9], s2));

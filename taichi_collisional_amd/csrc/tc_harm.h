@@ -187,12 +187,6 @@ __device__ __forceinline__ void harm_table_col(int m, double dx, double dy, doub
   }
 }
 
-// Whole table by the block's first P+1 threads.
-template <int P>
-__device__ __forceinline__ void harm_table_lds(double dx, double dy, double dz, cplx *G) {
-  harm_table_col<P>((int)threadIdx.x, dx, dy, dz, G);
-}
-
 // Complex form of a real-packed expansion (real_2_complex,
 // kernel_fast_lean.h:164-179): c_n^m = (a[s+m], a[s-m]), c_n^-m = (-1)^m conj.
 __device__ __forceinline__ cplx packed_to_c(const double *a, int n, int m) {

@@ -1,7 +1,7 @@
 // Kernel launch interfaces shared by the tcfmm host engine and the HIP
 // translation units.  Device layout (all device pointers, sorted body order):
 //   bodies  SoA x,y,z,vx,vy,vz,q (double), flags (kSink|kSource), order (orig idx)
-//   cells   SoA level, nchild, child (first child), body (first body), nbody,
+//   cells   SoA level, nchild, child (first child), body (first body), nbody, parent,
 //           Xg[3], Rg (tree geometry), X[3], R (bounding-ball geometry),
 //           has_sink, min_acc; coefficients M, Md, L, Ld: [cell][NT] doubles
 #pragma once
@@ -53,6 +53,7 @@ struct BodiesDev {
 
 struct CellsDev {
   int *level, *nchild, *child, *body, *nbody;
+  int *parent;  // (a tree's cells only; the roots' are not set)
   double *Xg, *Rg, *X, *R, *min_acc;
   unsigned char *has_sink;
   double *M, *Md, *L, *Ld;
@@ -274,7 +275,9 @@ int launch_pn(const double *M, int nc, int p, const FactTable &ft, double *Pn, h
 int launch_scatter_acc_old(BodiesDev b, int n, double *out, hipStream_t s);
 
 // ---- downward (tc_downward.hip)
-int launch_l2l(int p, CellsDev c, int ls, int le, hipStream_t s);
+// into the cells [ls, le) from their parents; beside: a long P2P launch runs on
+// the other stream
+int launch_l2l(int p, CellsDev c, int ls, int le, bool beside, hipStream_t s);
 int launch_l2l_ids(int p, CellsDev c, const int *ids, int nids, hipStream_t s);
 // add: into r; otherwise r is written (zeros for bodies that are not sinks)
 int launch_l2p(int p, CellsDev c, BodiesDev b, ResultsDev r, const int *leaf_ids, int nleaves,

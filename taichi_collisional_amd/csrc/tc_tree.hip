@@ -554,6 +554,7 @@ __global__ __launch_bounds__(256) void k_children(CellsDev c, const TreeState *_
         c.Xg[3 * cc + d] = c.Xg[3 * ci + d] + r * (((i >> d) & 1) * 2 - 1);
       c.Rg[cc] = r;
       c.level[cc] = level + 1;
+      c.parent[cc] = ci;
       c.body[cc] = o;
       c.nbody[cc] = size;
       c.nchild[cc] = 0;

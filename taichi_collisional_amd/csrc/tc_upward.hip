@@ -16,7 +16,7 @@
 //          M_parent[n,m] += sum_{k,l} M_child[n-k, m-l] Y_k^l(X_child - X_parent)
 //        with the eight children's harmonics and moments in LDS and lanes
 //        over (output term, child), the children's sums added across lanes
-//        (M first, then Mdot); one child at a time when that does not fit.
+//        (M first, then Mdot).
 #include "tc_common.h"
 #include "tc_geom.h"
 #include "tc_harm.h"
@@ -208,20 +208,25 @@ __global__ __launch_bounds__(64) void k_p2m(CellsDev c, BodiesDev b,
   }
 }
 
+// Threads per block: four waves; sixteen where the moments' tables take more
+// than 60 KB of LDS (p > 14), so that one block fills its CU.
+constexpr int m2m_threads(int p, int what) {
+  return (what & kUpMoments) && 16 * 16 * nterm(p) > 60 * 1024 ? 1024 : 256;
+}
+
 template <int P, int kWhat>
-__global__ __launch_bounds__(256) void k_m2m(CellsDev c, BodiesDev b, const int *__restrict__ ids,
+__global__ __launch_bounds__(m2m_threads(P, kWhat)) void k_m2m(CellsDev c, BodiesDev b, const int *__restrict__ ids,
                                              int ls) {
 #pragma clang fp contract(off)
   constexpr int NT = nterm(P);
   constexpr int NO = tri(P, P) + 1;
-  constexpr int NW = 4;
+  constexpr int NW = m2m_threads(P, kWhat) / kWave;
   constexpr bool kAdd = kWhat == kUpAll;
   constexpr int kStage = 512;  // body points of leaf children staged in LDS
-  // Eight children's harmonic tables and moments (complex) side by side, when
-  // they fit one work-group's LDS; else one child at a time.
-  constexpr bool kPar = 16 * 16 * NT <= 60 * 1024;
+  // Eight children's harmonic tables and moments (complex) side by side
+  // (160,000 of the CU's 163,840 bytes of LDS at p = 24).
   constexpr int kBall = 192 + 64 * 4 + 3 * kStage;       // doubles, ball phase
-  constexpr int kTrans = kPar ? 2 * 8 * 2 * NT : 3 * 2 * NT;  // doubles, translation
+  constexpr int kTrans = 2 * 8 * 2 * NT;               // doubles, translation
   // (each phase's own size where only one of them is compiled in)
   constexpr int kSmem = !(kWhat & kUpMoments) ? ((kWhat & kUpGeom) ? kBall : 1)
                         : !(kWhat & kUpGeom)  ? kTrans
@@ -401,7 +406,7 @@ __global__ __launch_bounds__(256) void k_m2m(CellsDev c, BodiesDev b, const int 
     __syncthreads();  // the ball's buffers are reused below
   }
   if constexpr (!(kWhat & kUpMoments)) return;
-  if constexpr (kPar) {
+  {
     // translation, children in parallel: lane = (task group g, child k) with
     // k fastest, each lane a strided share of the output terms of child k;
     // the 8 children's partial sums of one term sit in 8 neighbouring lanes
@@ -426,7 +431,7 @@ __global__ __launch_bounds__(256) void k_m2m(CellsDev c, BodiesDev b, const int 
       __syncthreads();
       double *dst = (pass ? c.Md : c.M) + (size_t)ci * NT;
       const cplx *src = Call + k * NT, *Gk = Gall + k * NT;
-      for (int o = g; o < NO; o += 32) {
+      for (int o = g; o < NO; o += NW * kWave / 8) {
         int n = 0;
         while (tri(n + 1, 0) <= o && n < P) n++;
         const int m = o - tri(n, 0);
@@ -460,61 +465,6 @@ __global__ __launch_bounds__(256) void k_m2m(CellsDev c, BodiesDev b, const int 
       }
       __syncthreads();  // Call is refilled by the next pass
     }
-  } else {
-    // translation, one child at a time: tasks (output term, M or Mdot)
-    // strided over the block, the child's harmonics and moments in LDS
-    cplx *G = reinterpret_cast<cplx *>(smem), *cm = G + NT, *cmd = cm + NT;
-    constexpr int NTASK = 2 * NO, NRT = (NTASK + 255) / 256;
-    cplx a[NRT];
-    int tn[NRT], tm[NRT];
-#pragma unroll
-    for (int r = 0; r < NRT; r++) {
-      a[r] = {0, 0};
-      const int j = tid + 256 * r, o = j % NO;
-      int n = 0;
-      while (tri(n + 1, 0) <= o && n < P) n++;
-      tn[r] = n;
-      tm[r] = o - tri(n, 0);
-    }
-    for (int kc = 0; kc < nch; kc++) {
-      const int ch = ch0 + kc;
-      __syncthreads();
-      harm_table_lds<P>(c.X[3 * ch] - X[0], c.X[3 * ch + 1] - X[1], c.X[3 * ch + 2] - X[2], G);
-      const double *Mch = c.M + (size_t)ch * NT;
-      const double *Mdch = c.Md + (size_t)ch * NT;
-      for (int t = tid; t < NT; t += blockDim.x) {
-        int nn = 0;
-        while ((nn + 1) * (nn + 1) <= t) nn++;
-        const int mm = t - nn * nn - nn;
-        cm[t] = packed_to_c(Mch, nn, mm);
-        cmd[t] = packed_to_c(Mdch, nn, mm);
-      }
-      __syncthreads();
-#pragma unroll
-      for (int r = 0; r < NRT; r++) {
-        const int j = tid + 256 * r;
-        if (j >= NTASK) continue;
-        const cplx *src = j >= NO ? cmd : cm;
-        const int n = tn[r], m = tm[r];
-        cplx acc = a[r];
-        for (int kk = 0; kk <= n; kk++) {
-          const int lo = -kk > m - n + kk ? -kk : m - n + kk;
-          const int hi = kk < m + n - kk ? kk : m + n - kk;
-          for (int l = lo; l <= hi; l++)
-            acc = cadd(acc, cmul(src[ixnm(n - kk, m - l)], G[ixnm(kk, l)]));
-        }
-        a[r] = acc;
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < NRT; r++) {
-      const int j = tid + 256 * r;
-      if (j >= NTASK) continue;
-      double *dst = (j >= NO ? c.Md : c.M) + (size_t)ci * NT;
-      const int n = tn[r], m = tm[r], s = n * n + n;
-      dst[s + m] = kAdd ? dst[s + m] + a[r].re : a[r].re;
-      if (m > 0) dst[s - m] = kAdd ? dst[s - m] + a[r].im : a[r].im;
-    }
   }
 }
 
@@ -545,22 +495,23 @@ static void p2m_launch(CellsDev c, BodiesDev b, const int *leaf_ids, int nleaves
 template <int P>
 static void m2m_launch(CellsDev c, BodiesDev b, const int *ids, int ls, int ncell, int what,
                        hipStream_t s) {
-  const dim3 g(ncell), t(256);
+  const dim3 g(ncell);
+  auto t = [](int w) { return dim3(m2m_threads(P, w)); };
   switch (what) {
     case kUpGeom | kUpMin:
-      hipLaunchKernelGGL((k_m2m<P, kUpGeom | kUpMin>), g, t, 0, s, c, b, ids, ls);
+      hipLaunchKernelGGL((k_m2m<P, kUpGeom | kUpMin>), g, t(kUpGeom | kUpMin), 0, s, c, b, ids, ls);
       break;
     case kUpMoments:
-      hipLaunchKernelGGL((k_m2m<P, kUpMoments>), g, t, 0, s, c, b, ids, ls);
+      hipLaunchKernelGGL((k_m2m<P, kUpMoments>), g, t(kUpMoments), 0, s, c, b, ids, ls);
       break;
     case kUpGeom | kUpMoments:
-      hipLaunchKernelGGL((k_m2m<P, kUpGeom | kUpMoments>), g, t, 0, s, c, b, ids, ls);
+      hipLaunchKernelGGL((k_m2m<P, kUpGeom | kUpMoments>), g, t(kUpGeom | kUpMoments), 0, s, c, b, ids, ls);
       break;
     case kUpMin:
-      hipLaunchKernelGGL((k_m2m<P, kUpMin>), g, t, 0, s, c, b, ids, ls);
+      hipLaunchKernelGGL((k_m2m<P, kUpMin>), g, t(kUpMin), 0, s, c, b, ids, ls);
       break;
     default:
-      hipLaunchKernelGGL((k_m2m<P, kUpAll>), g, t, 0, s, c, b, ids, ls);
+      hipLaunchKernelGGL((k_m2m<P, kUpAll>), g, t(kUpAll), 0, s, c, b, ids, ls);
   }
 }
 
