@@ -126,7 +126,8 @@ struct tc_context {
   DBuf p2p_items, p2p_ranges, npairs;
   int nleaves = 0;
   // traversal / lists
-  DBuf front_a, front_b, m2l, p2p, tcnt, tblk, tscan, tstate, tcls;
+  DBuf front_a, front_b, m2l, p2p, tstate, twords, tcls;
+  unsigned trav_tag = 0;  // of the last walk step (the scan words' tags)
   int trav_steps[4] = {0, 0, 0, 0};  // steps of the last walk per MAC mode (batch size)
   DBuf gsort1[4], gsort2[4];  // list grouping scratch per stream: keys in, out, sources, temp
   int *h_pin = nullptr;  // small pinned host buffer for per-step counts (256 ints)

@@ -232,17 +232,17 @@ static int upward_min(tc_context *ctx) {
 // on the first evaluation of a workload).
 static int traverse(tc_context *ctx, int n, const MacArgs &mac) {
   hipStream_t s = ctx->stream;
-  const TravState *hst = reinterpret_cast<const TravState *>(ctx->h_pin + 40);
-  TravState *dst = reinterpret_cast<TravState *>(ctx->h_pin_dev + 40);
-  static_assert(sizeof(TravState) <= 12 * sizeof(int), "pinned slots 40..51 (52, 53: P2P pairs)");
+  const TravState *hst = reinterpret_cast<const TravState *>(ctx->h_pin + 144);
+  TravState *dst = reinterpret_cast<TravState *>(ctx->h_pin_dev + 144);
+  static_assert(sizeof(TravState) <= 16 * sizeof(int), "pinned slots 144..159");
   TC_CHECK(ctx->tstate.ensure(sizeof(TravState)));
-  TC_CHECK(ctx->tblk.ensure(sizeof(int) * 6 * kTravBlocks));
   TC_CHECK(ctx->front_a.ensure(sizeof(int2) * (size_t)std::max(1 << 16, 4 * n)));
   TC_CHECK(ctx->front_b.ensure(ctx->front_a.bytes));
   TC_CHECK(ctx->tcls.ensure(ctx->front_a.bytes / sizeof(int2)));
   TC_CHECK(ctx->m2l.ensure(sizeof(int2) * (size_t)std::max(1 << 16, 24 * n)));
   TC_CHECK(ctx->p2p.ensure(sizeof(int2) * (size_t)std::max(1 << 16, 8 * n)));
   int &known = ctx->trav_steps[mac.mode & 3];
+  int last = 0;  // parity of the state after the walk's last queued step
   for (int attempt = 0;; attempt++) {
     if (attempt > 16) {
       ctx->err = "traversal: list buffers keep overflowing";
@@ -254,6 +254,16 @@ static int traverse(tc_context *ctx, int n, const MacArgs &mac) {
     const long long cm = cap(ctx->m2l), cp = cap(ctx->p2p),
                     cf = std::min({cap(ctx->front_a), cap(ctx->front_b),
                                    (long long)std::min<size_t>(ctx->tcls.bytes, 0x7fffffff)});
+    // the scan's words: cleared when they are new or the tags run out, so that
+    // no step finds its own tag there
+    const size_t wb = sizeof(unsigned long long) * kTravWords;
+    if (ctx->twords.bytes < wb || ctx->trav_tag > (1u << 27)) {
+      TC_CHECK(ctx->twords.ensure(wb));
+      TC_CHECK(hipMemsetAsync(ctx->twords.p, 0, ctx->twords.bytes, s));
+      ctx->trav_tag = 0;
+    }
+    // a small system's frontiers are a few pairs per body
+    const int nblocks = std::min(kTravBlocks, std::max(64, n / 32));
     launch_root_pairs(ctx->front_a.as<int2>(), ctx->ncl, ctx->tstate.as<TravState>(), s);
     int k = 0, batch = std::max(8, known + 1);
     for (;;) {
@@ -267,10 +277,12 @@ static int traverse(tc_context *ctx, int n, const MacArgs &mac) {
         a.cls = ctx->tcls.as<unsigned char>();
         a.mac = mac;
         launch_trav_step(cells_of(ctx), a, ctx->tstate.as<TravState>(), (int)odd,
-                         ctx->tblk.as<int>(), cm, cp, cf, i == batch - 1 ? dst : nullptr, s);
+                         ++ctx->trav_tag, ctx->twords.as<unsigned long long>(), nblocks, cm, cp,
+                         cf, i == batch - 1 ? dst : nullptr, s);
       }
       TC_CHECK(spin_wait(ctx, s));
-      if (hst->overflow || hst->nin[k & 1] == 0) break;
+      last = k & 1;
+      if (hst->overflow || hst->nin[last] == 0) break;
       if (k > 100000) {
         ctx->err = "traversal does not end";
         return -3;
@@ -290,8 +302,8 @@ static int traverse(tc_context *ctx, int n, const MacArgs &mac) {
     }
   }
   known = hst->steps;
-  ctx->st.n_m2l = hst->nm2l;
-  ctx->st.n_p2p_cells = hst->np2p;
+  ctx->st.n_m2l = hst->nm2l[last];
+  ctx->st.n_p2p_cells = hst->np2p[last];
   return 0;
 }
 
@@ -1230,7 +1242,7 @@ int tc_destroy(tc_context *ctx) {
                  &ctx->cnbody, &ctx->cXg, &ctx->cRg, &ctx->cX, &ctx->cR, &ctx->cmin, &ctx->csink,
                  &ctx->cM, &ctx->cMd, &ctx->cL, &ctx->cLd, &ctx->split_offs, &ctx->split_nch,
                  &ctx->split_scan, &ctx->scan_tmp, &ctx->leaf_ids, &ctx->front_a, &ctx->front_b,
-                 &ctx->m2l, &ctx->p2p, &ctx->tcnt, &ctx->tblk, &ctx->tscan, &ctx->tstate, &ctx->tcls, &ctx->tree_state,
+                 &ctx->m2l, &ctx->p2p, &ctx->tstate, &ctx->twords, &ctx->tcls, &ctx->tree_state,
                  &ctx->gsort1[0], &ctx->gsort1[1], &ctx->gsort1[2], &ctx->gsort1[3], &ctx->gsort2[0], &ctx->gsort2[1], &ctx->gsort2[2], &ctx->gsort2[3], &ctx->m2l_cnt, &ctx->m2l_off, &ctx->m2l_cur,
                  &ctx->m2l_src, &ctx->m2l_coff, &ctx->m2l_chunks, &ctx->p2p_cnt, &ctx->p2p_off,
                  &ctx->p2p_cur, &ctx->p2p_src, &ctx->dtg, &ctx->dpot, &ctx->dacc, &ctx->djerk,

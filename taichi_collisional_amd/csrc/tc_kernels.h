@@ -151,25 +151,28 @@ struct TravArgs {
   const int2 *fin;  // this step's frontier
   int2 *fout;       // the next step's
   int2 *m2l, *p2p;  // the lists, appended to
-  unsigned char *cls;  // per frontier pair: kind << 4 | child pairs (pass 1 -> pass 2)
+  unsigned char *cls;  // a class per frontier pair (scratch)
   MacArgs mac;
 };
-// Device-side state of a walk (ints): frontier sizes nin[step parity], list
-// lengths so far, this step's list offsets, whether pass 2 writes, steps
-// taken, and on overflow what the failing step needed.
+// Device-side state of a walk, by step parity: frontier size, list lengths so
+// far, ranges taken; and steps taken, whether a buffer overflowed and what the
+// failing step needed.  A walk that has taken k steps has its results at
+// parity k & 1.
 struct TravState {
-  int nin[2];
-  int nm2l, np2p, base_m2l, base_p2p;
-  int write, overflow, steps;
-  int need_m2l, need_p2p, need_front;
+  int nin[2], nm2l[2], np2p[2], ticket[2];
+  int overflow, steps;
+  int need_m2l, need_p2p, need_front, pad;
 };
-constexpr int kTravBlocks = 2048;  // blocks of a walk step; blk holds 6 x kTravBlocks ints
-// One step of the walk (count, offsets, write) on the frontier of parity par;
+constexpr int kTravThreads = 256, kTravBlocks = 1024;  // four blocks a CU
+// words of the scan over a step's blocks
+constexpr size_t kTravWords = 6 * kTravBlocks;
+// One step of the walk on the frontier of parity par, by nblocks <= kTravBlocks
+// blocks; tag: a value of 28 bits that the words hold from no other step;
 // caps are the capacities of the lists and of the next frontier (pairs);
 // report (or null): pinned host memory that receives the state after the step.
-int launch_trav_step(CellsDev c, const TravArgs &a, TravState *st, int par, int *blk,
-                     long long cap_m2l, long long cap_p2p, long long cap_front,
-                     TravState *report, hipStream_t s);
+int launch_trav_step(CellsDev c, const TravArgs &a, TravState *st, int par, unsigned tag,
+                     unsigned long long *words, int nblocks, long long cap_m2l,
+                     long long cap_p2p, long long cap_front, TravState *report, hipStream_t s);
 // the frontier of the ncl root pairs (k, k) and the state that starts the walk
 void launch_root_pairs(int2 *front, int ncl, TravState *st, hipStream_t s);
 size_t pair_sort_temp_bytes(int n);

@@ -17,9 +17,8 @@
 //   recursion from (root, root) is run breadth-first over a frontier of cell
 //   pairs; each pair is accepted for M2L by the theta-MAC, sent to P2P when
 //   both are leaves, or split (Ci if Cj is a leaf or Ci is larger, else Cj).
-//   Each step runs in two passes (count per block, scan, write at the scanned
-//   offsets), so the lists are written without atomics and in a fixed order;
-//   they are then grouped by target cell with a stable radix sort, and the
+//   Each step is one launch that counts, scans and writes, so the lists come
+//   out in a fixed order; they are then grouped by target cell with a stable radix sort, and the
 //   M2L list is cut into chunks of <= 64 sources.
 #include <hipcub/hipcub.hpp>
 
@@ -1132,11 +1131,11 @@ int launch_scan(const int *in, int *out, int n, void *temp, size_t temp_bytes, h
 }
 
 // ------------------------------------------------------------ traversal -----
-// One breadth-first step, in two passes so that no shared counter is hit by
-// every wave: pass 1 classifies each frontier pair, keeps the class and writes
-// per-block totals (M2L, P2P, child pairs); the totals are scanned over
-// blocks; pass 2 writes every output at its scanned position, so the lists
-// come out in frontier order (deterministic).
+// One breadth-first step in one launch: every block classifies its range of
+// the frontier, its counts (M2L, P2P, child pairs) are turned into list
+// positions by a scan over the blocks that runs while they do (decoupled
+// look-back, below), and it writes its outputs there, so the lists come out in
+// frontier order (deterministic).
 // The walks' squared distance norm(dX) (kernel_fast_lean.h:113-116) and one
 // error-MAC term (traverse_eager.h:80-88, master :82-90) rounded as the
 // reference's x86-64 build evaluates them: GCC -O3 contracts the sum of
@@ -1255,149 +1254,176 @@ __device__ __forceinline__ int3 block_excl_scan3_n(int3 v, int3 *tot) {
   return make_int3(base.x + ex, base.y + ey, base.z + ez);
 }
 
-// Steps of the walk queued without host reads: the frontier size, the list
-// lengths and the step's offsets live in TravState.  Block b of the
-// kTravBlocks blocks owns frontier pairs [b R, (b + 1) R), R = ceil(nin /
-// kTravBlocks), walked 256 at a time, so the outputs keep frontier order.
-__device__ __forceinline__ void trav_range(int nin, int &lo, int &hi) {
-  const int R = (nin + kTravBlocks - 1) / kTravBlocks;
-  const long long l = (long long)blockIdx.x * R;
-  lo = l < nin ? (int)l : nin;
-  hi = nin - lo < R ? nin : lo + R;
+__device__ __forceinline__ int wave_sum_i(int v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
+  return v;
 }
 
-// pass 1: per-block totals of M2L pairs, P2P pairs and child pairs; each
-// pair's class (kind << 4 | child pairs) is kept for pass 2
-__global__ __launch_bounds__(256) void k_trav_count(CellsDev c, const int2 *__restrict__ fin,
-                                                    const TravState *__restrict__ st, int par,
-                                                    MacArgs mac, int *__restrict__ blk,
-                                                    unsigned char *__restrict__ cls) {
-  int lo, hi;
-  trav_range(st->nin[par], lo, hi);
-  int3 acc = make_int3(0, 0, 0);
-  for (int base = lo; base < hi; base += 256) {
-    const int t = base + (int)threadIdx.x;
-    int3 v = make_int3(0, 0, 0);
-    if (t < hi) {
-      const int2 pr = fin[t];
-      int ns;
-      const int kind = trav_classify(c, mac, pr.x, pr.y, &ns);
-      v = make_int3(kind == 1, kind == 2, ns);
-      cls[t] = (unsigned char)(kind << 4 | ns);
-    }
-    int3 tot;
-    block_excl_scan3_n<4>(v, &tot);
-    acc = make_int3(acc.x + tot.x, acc.y + tot.y, acc.z + tot.z);
-  }
-  if (threadIdx.x == 0) {
-    blk[blockIdx.x] = acc.x;
-    blk[kTravBlocks + blockIdx.x] = acc.y;
-    blk[2 * kTravBlocks + blockIdx.x] = acc.z;
-  }
+// A block's words for the scan over the blocks: its own three counts and,
+// later, the sums up to and with it.  A word is the value and, above
+// kTravTagShift, the step's tag: words of other steps read as not there yet, so
+// nothing is cleared between steps, and value and tag arrive together (one
+// 64-bit store), so no ordering is needed between the words.
+constexpr int kTravTagShift = 36;
+__device__ __forceinline__ void trav_put(unsigned long long *w, int v, unsigned tag) {
+  __hip_atomic_store(w, (unsigned long long)(unsigned)v | (unsigned long long)tag << kTravTagShift,
+                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ unsigned long long trav_get(const unsigned long long *w) {
+  return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// the block offsets (exclusive scans of pass 1's totals, to blk[3 G ..]) and
-// the state for pass 2 and the next step; a step whose output would not fit
-// sets the overflow flag, records what it needed and ends the walk.  One
-// wave: it must find room on a CU while the upward moments (second stream)
-// fill the machine with small blocks, which a 1024-thread block waits out.
-__global__ __launch_bounds__(64) void k_trav_scan(int *__restrict__ blk, TravState *st, int par,
-                                                  long long cap_m2l, long long cap_p2p,
-                                                  long long cap_front, TravState *report) {
-  constexpr int G = kTravBlocks, PER = G / kWave;
-  static_assert(G % kWave == 0, "whole entries per lane");
-  const int t = threadIdx.x;
+// Sums of the counts of the ranges before `range`, by one wave: 64 ranges at a
+// time, nearest first, until one whose sums are known.  Ranges are numbered in
+// the order in which blocks start on them, and a range's counts are stored
+// before its block waits for anything, so every word looked for here arrives.
+__device__ __forceinline__ int3 trav_look_back(const unsigned long long *words, int range,
+                                               unsigned tag) {
+  const int lane = threadIdx.x & (kWave - 1);
   int3 sum = make_int3(0, 0, 0);
-  for (int k = 0; k < PER; k++) {
-    const int i = t * PER + k;
-    sum = make_int3(sum.x + blk[i], sum.y + blk[G + i], sum.z + blk[2 * G + i]);
+  for (int last = range - 1; last >= 0;) {
+    const int k = last - lane;
+    unsigned long long w[6] = {0, 0, 0, 0, 0, 0};
+    if (k >= 0)
+      for (int q = 0; q < 6; q++) w[q] = trav_get(words + 6 * k + q);
+    auto here = [&](int q) { return (unsigned)(w[q] >> kTravTagShift) == tag; };
+    const bool counts = here(0) && here(1) && here(2), sums = here(3) && here(4) && here(5);
+    const unsigned long long known = __ballot(k >= 0 && sums);
+    const unsigned long long ready = __ballot(k < 0 || sums || counts);
+    const int stop = known ? __ffsll(known) - 1 : kWave;  // lanes before it add their counts
+    const unsigned long long need = stop < kWave ? (1ull << stop) - 1 : ~0ull;
+    if ((ready & need) != need) {
+      __builtin_amdgcn_s_sleep(1);
+      continue;
+    }
+    int3 v = make_int3(0, 0, 0);
+    if (k >= 0 && lane < stop) v = make_int3((int)(unsigned)w[0], (int)(unsigned)w[1],
+                                             (int)(unsigned)w[2]);
+    if (k >= 0 && lane == stop) v = make_int3((int)(unsigned)w[3], (int)(unsigned)w[4],
+                                              (int)(unsigned)w[5]);
+    sum = make_int3(sum.x + wave_sum_i(v.x), sum.y + wave_sum_i(v.y), sum.z + wave_sum_i(v.z));
+    if (known) break;
+    last -= kWave;
+  }
+  return sum;
+}
+
+// One step.  The frontier size, list lengths and the counter of ranges taken
+// live in TravState, two of each by step parity: this step reads its own and
+// the block of its last range sets the next step's.  A range is as many whole
+// rounds of the block's threads as leave no block without one; over one round,
+// the pairs' classes wait in memory for the positions.  More, shorter ranges
+// than blocks would lengthen the look-back's chain (some 4 us per 64 ranges:
+// ranges of 1,024 pairs took 350 us in the widest step at N = 2^20, 5,000 of
+// them, where these take 190).  Blocks of 512 threads found no room beside the
+// upward moments (0.5 ms).
+// A list that its buffer cannot hold sets the overflow flag, records what the
+// step needed and ends the walk (nothing is written past a buffer's end).
+// N = 10,007: a step 14 us in three launches (count, scan, write), 7 in one.
+__global__ __launch_bounds__(kTravThreads) void k_trav_step(
+    CellsDev c, TravArgs a, TravState *st, int par, unsigned tag,
+    unsigned long long *__restrict__ words, long long cap_m2l, long long cap_p2p,
+    long long cap_front, TravState *report) {
+  constexpr int T = kTravThreads, NW = T / kWave;
+  __shared__ int s_range;
+  __shared__ int3 s_before;
+  const int t = threadIdx.x;
+  const int nin = st->nin[par], bm = st->nm2l[par], bp = st->np2p[par];
+  if (nin == 0) {
+    if (blockIdx.x == 0 && t == 0) {
+      st->nin[par ^ 1] = 0;
+      st->nm2l[par ^ 1] = bm;
+      st->np2p[par ^ 1] = bp;
+      st->ticket[par ^ 1] = 0;
+      if (report) *report = *st;
+    }
+    return;
+  }
+  const int rounds = (nin + T * (int)gridDim.x - 1) / (T * (int)gridDim.x);
+  const int nranges = (nin + T * rounds - 1) / (T * rounds);
+  if ((int)blockIdx.x >= nranges) return;
+  if (t == 0) s_range = atomicAdd(&st->ticket[par], 1);
+  __syncthreads();
+  const int range = s_range;
+  const int lo = range * (T * rounds), hi = min(nin, lo + T * rounds);
+  int2 pr = make_int2(0, 0);
+  int cls = 0;  // kind << 4 | child pairs
+  int3 v = make_int3(0, 0, 0);
+  for (int i = lo + t; i < hi; i += T) {
+    int ns;
+    pr = a.fin[i];
+    const int kind = trav_classify(c, a.mac, pr.x, pr.y, &ns);
+    v = make_int3(v.x + (kind == 1), v.y + (kind == 2), v.z + ns);
+    cls = kind << 4 | ns;
+    if (rounds > 1) a.cls[i] = (unsigned char)cls;
   }
   int3 tot;
-  int3 run;
-  run.x = wave_excl_scan(sum.x, &tot.x);
-  run.y = wave_excl_scan(sum.y, &tot.y);
-  run.z = wave_excl_scan(sum.z, &tot.z);
-  for (int k = 0; k < PER; k++) {
-    const int i = t * PER + k;
-    const int3 a = make_int3(blk[i], blk[G + i], blk[2 * G + i]);
-    blk[3 * G + i] = run.x;
-    blk[4 * G + i] = run.y;
-    blk[5 * G + i] = run.z;
-    run = make_int3(run.x + a.x, run.y + a.y, run.z + a.z);
-  }
-  if (t == 0) {
-    const int nin = st->nin[par];
-    const long long nm = st->nm2l, np = st->np2p;
-    const bool fits = !st->overflow && nm + tot.x <= cap_m2l && np + tot.y <= cap_p2p &&
-                      tot.z <= cap_front;
-    if (fits) {
-      st->base_m2l = (int)nm;
-      st->base_p2p = (int)np;
-      st->nm2l = (int)(nm + tot.x);
-      st->np2p = (int)(np + tot.y);
-      st->nin[par ^ 1] = tot.z;
-      st->write = 1;
-      if (nin > 0) st->steps++;
-    } else {
-      if (!st->overflow) {
-        const long long big = 0x7fffffff;
-        st->need_m2l = (int)(nm + tot.x < big ? nm + tot.x : big);
-        st->need_p2p = (int)(np + tot.y < big ? np + tot.y : big);
-        st->need_front = tot.z;
+  int3 ex = block_excl_scan3_n<NW>(v, &tot);
+  if (t < kWave) {
+    unsigned long long *w = words + 6 * range;
+    if (t == 0) {
+      trav_put(w, tot.x, tag);
+      trav_put(w + 1, tot.y, tag);
+      trav_put(w + 2, tot.z, tag);
+    }
+    const int3 before = trav_look_back(words, range, tag);
+    if (t == 0) {
+      const int3 s = make_int3(before.x + tot.x, before.y + tot.y, before.z + tot.z);
+      trav_put(w + 3, s.x, tag);
+      trav_put(w + 4, s.y, tag);
+      trav_put(w + 5, s.z, tag);
+      s_before = before;
+      if (range == nranges - 1) {
+        const long long nm = (long long)bm + s.x, np = (long long)bp + s.y, big = 0x7fffffff;
+        const bool fits = !st->overflow && nm <= cap_m2l && np <= cap_p2p && s.z <= cap_front;
+        if (!fits && !st->overflow) {
+          st->need_m2l = (int)(nm < big ? nm : big);
+          st->need_p2p = (int)(np < big ? np : big);
+          st->need_front = s.z;
+          st->overflow = 1;
+        }
+        st->nin[par ^ 1] = fits ? s.z : 0;
+        st->nm2l[par ^ 1] = (int)(nm < big ? nm : big);
+        st->np2p[par ^ 1] = (int)(np < big ? np : big);
+        st->ticket[par ^ 1] = 0;
+        st->steps++;
+        if (report) *report = *st;
       }
-      st->overflow = 1;
-      st->write = 0;
-      st->nin[par ^ 1] = 0;
     }
-    if (report) *report = *st;
   }
-}
-
-// pass 2: every output at its place (block offset + running count within the
-// block + rank within the 256-pair slice)
-__global__ __launch_bounds__(256) void k_trav_write(CellsDev c, TravArgs a,
-                                                    const TravState *__restrict__ st, int par,
-                                                    const int *__restrict__ blk) {
-  if (!st->write) return;
-  int lo, hi;
-  trav_range(st->nin[par], lo, hi);
-  const int b = blockIdx.x;
-  int3 run = make_int3(blk[3 * kTravBlocks + b], blk[4 * kTravBlocks + b],
-                       blk[5 * kTravBlocks + b]);
-  const int bm = st->base_m2l, bp = st->base_p2p;
-  for (int base = lo; base < hi; base += 256) {
-    const int t = base + (int)threadIdx.x;
-    int kind = 0, ns = 0;
-    int2 pr = make_int2(0, 0);
-    if (t < hi) {
-      pr = a.fin[t];
-      const int k = a.cls[t];
-      kind = k >> 4;
-      ns = k & 15;
+  __syncthreads();
+  // the positions of the range's outputs, round by round
+  long long om = (long long)bm + s_before.x, op = (long long)bp + s_before.y, of = s_before.z;
+  for (int base = lo; base < hi; base += T) {
+    if (rounds > 1) {
+      const int i = base + t;
+      cls = 0;
+      if (i < hi) {
+        pr = a.fin[i];
+        cls = a.cls[i];
+      }
     }
-    int3 tot;
-    const int3 ex = block_excl_scan3_n<4>(make_int3(kind == 1, kind == 2, ns), &tot);
-    if (kind == 1) a.m2l[bm + run.x + ex.x] = pr;
-    if (kind == 2) a.p2p[bp + run.y + ex.y] = pr;
-    if (kind >= 3) {
-      const int o = run.z + ex.z;
+    const int kind = cls >> 4, ns = cls & 15;
+    if (rounds > 1) ex = block_excl_scan3_n<NW>(make_int3(kind == 1, kind == 2, ns), &tot);
+    if (kind == 1 && om + ex.x < cap_m2l) a.m2l[om + ex.x] = pr;
+    if (kind == 2 && op + ex.y < cap_p2p) a.p2p[op + ex.y] = pr;
+    if (kind >= 3 && of + ex.z + ns <= cap_front) {
       const int c0 = c.child[kind == 3 ? pr.x : pr.y];
       for (int k = 0; k < ns; k++)
-        a.fout[o + k] = kind == 3 ? make_int2(c0 + k, pr.y) : make_int2(pr.x, c0 + k);
+        a.fout[of + ex.z + k] = kind == 3 ? make_int2(c0 + k, pr.y) : make_int2(pr.x, c0 + k);
     }
-    run = make_int3(run.x + tot.x, run.y + tot.y, run.z + tot.z);
+    om += tot.x;
+    op += tot.y;
+    of += tot.z;
   }
 }
 
-int launch_trav_step(CellsDev c, const TravArgs &a, TravState *st, int par, int *blk,
-                     long long cap_m2l, long long cap_p2p, long long cap_front,
-                     TravState *report, hipStream_t s) {
-  hipLaunchKernelGGL(k_trav_count, dim3(kTravBlocks), dim3(256), 0, s, c, a.fin,
-                     (const TravState *)st, par, a.mac, blk, a.cls);
-  hipLaunchKernelGGL(k_trav_scan, dim3(1), dim3(kWave), 0, s, blk, st, par, cap_m2l, cap_p2p,
-                     cap_front, report);
-  hipLaunchKernelGGL(k_trav_write, dim3(kTravBlocks), dim3(256), 0, s, c, a,
-                     (const TravState *)st, par, (const int *)blk);
+int launch_trav_step(CellsDev c, const TravArgs &a, TravState *st, int par, unsigned tag,
+                     unsigned long long *words, int nblocks, long long cap_m2l,
+                     long long cap_p2p, long long cap_front, TravState *report, hipStream_t s) {
+  hipLaunchKernelGGL(k_trav_step, dim3(nblocks), dim3(kTravThreads), 0, s, c, a, st, par, tag,
+                     words, cap_m2l, cap_p2p, cap_front, report);
   return 0;
 }
 
