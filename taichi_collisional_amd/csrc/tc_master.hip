@@ -242,9 +242,12 @@ __global__ __launch_bounds__(kMT) void k_master_direct(Src src, BodiesDev b, int
       for (int r = 0; r < kR; r++) {
         const double dx = sk.x - xi[r], dy = sk.y - yi[r], dz = sk.z - zi[r];
         const double r2 = dx * dx + dy * dy + dz * dz;
-        // r2 = 0 masked
-        const double ir = rsqrt_fp64(r2 > 0 ? r2 : 1e38);
-        const double w = r2 > 0 ? sk.w * ir : 0.0;
+        // r2 = 0 masked by clearing the high word of the reciprocal square root
+        // (+inf or the default NaN there, whose low word is zero): one 32-bit
+        // select where masking the argument and the weight takes four
+        const double rq = rsqrt_fp64(r2);
+        const double ir = __hiloint2double(r2 > 0 ? __double2hiint(rq) : 0, __double2loint(rq));
+        const double w = sk.w * ir;
         pt[r] += w;
         const double w3 = w * ir * ir;
         ax[r] += dx * w3;
@@ -285,15 +288,74 @@ __global__ __launch_bounds__(kMT) void k_master_direct(Src src, BodiesDev b, int
 // uniform: a slab starting inside a leaf starts mi where the leaf's running
 // sum would be there -- q_i + pmx[j0], less q_i itself when the target sits
 // in that leaf before j0 -- and each slab reports, per target, its leaf
-// pieces: the first and the last (leaf id = last index, running minimum) and
+// pieces: the first and the last (leaf id = last index, largest rate 1 / tau) and
 // the sum over the leaves it holds whole; k_master_direct_merge joins the
-// pieces of a leaf across slabs (minimum), then adds min^-4 per leaf, slab by
+// pieces of a leaf across slabs (maximum), then adds rate^4 per leaf, slab by
 // slab.  Otherwise (the level-built tree, or coincident bodies) the slabs are
 // leaf-aligned as in k_master_direct and the same format and merge serve.
 // part: [slab][9][n] doubles: potential, acceleration (3), the whole leaves'
-// sum, first piece minimum, last piece minimum, first and last piece ids.
+// sum, first piece's rate, last piece's rate, first and last piece ids.
 constexpr int kStepCols = 9;
 
+__device__ __forceinline__ double pow4(double r) {
+  r *= r;
+  return r * r;
+}
+
+// One pair of the vector form into the force sums and the running largest rate
+// 1 / tau of the source leaf.  With a = 1 / tau, a capped rate term turns
+// tau / (1 - min(c tau vdr, 1) / 2) into 1 / max(a - c vdr / 2, a / 2), so the
+// divisions go and the minimum of tau is the maximum of these rates:
+//   free fall  a = sqrt(2) / dt sqrt(M / r^3),  c = 3 / 2
+//   fly-by     a = |dv| / (dt r),               c = 1 + M / (r |dv|^2)
+// (three reciprocal square roots a pair; the tau form took five reciprocals).
+// M grows along the leaf by every source met with r > 0; |dv|^2 carries
+// +1e-20; r = 0 stands for r^2 = 1e38 in the rates and adds no force.  rate
+// and full collect max(a - c vdr / 2) and max(a); the piece's rate is the
+// larger of rate and full / 2.
+struct StepPair {
+  double pt, ax, ay, az, rate, full, mi;
+};
+// the larger of two numbers, a NaN giving way (fmax, without the quieting of
+// its operands that the compiler adds for loop-carried ones)
+__device__ __forceinline__ double max_f64(double a, double b) {
+  double r;
+  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ void pair_rate(double dx, double dy, double dz, double dvx, double dvy,
+                                          double dvz, double r2, double q, double qs, double kff,
+                                          double kfb, StepPair &s) {
+  if (__builtin_expect(__any(!(r2 > 0)), 0)) {
+    q = r2 > 0 ? q : 0.0;
+    qs = r2 > 0 ? qs : 0.0;
+    r2 = r2 > 0 ? r2 : 1e38;
+  }
+  const double ir = rsqrt_fp64(r2);
+  const double ir2 = ir * ir, ir3 = ir * ir2;
+  s.pt = fma(qs, ir, s.pt);
+  const double w3 = qs * ir3;
+  s.ax = fma(dx, w3, s.ax);
+  s.ay = fma(dy, w3, s.ay);
+  s.az = fma(dz, w3, s.az);
+  s.mi += q;
+  const double vdr = fma(dz, dvz, fma(dy, dvy, dx * dvx)) * ir2;
+  const double y = s.mi * ir3;
+  const double aff = y * rsqrt_fp64(y) * kff;
+  s.rate = max_f64(s.rate, fma(-0.75, vdr, aff));
+  const double v2 = fma(dvz, dvz, fma(dvy, dvy, fma(dvx, dvx, 1e-20)));
+  const double iv = rsqrt_fp64(v2);
+  const double afb = v2 * iv * (ir * kfb);
+  const double c = fma(vdr, s.mi * ir * (iv * iv), vdr);
+  s.rate = max_f64(s.rate, fma(-0.5, c, afb));
+  s.full = max_f64(max_f64(s.full, aff), afb);
+}
+
+// The sources of a tile run leaf piece by leaf piece: the leaf ends of 64
+// sources are one ballot, and between two ends the loop tests nothing.  Bound
+// by FP64 issue, 79 slots a pair in the vector form: N = 65,536 (ncrit 300)
+// 14.2 -> 9.7 ms, N = 4,096 65 -> 48 us against the tau form with a flag byte
+// and a branch per source.
 template <bool kPairMass>
 __global__ __launch_bounds__(kMT) void k_master_direct_steps(BodiesDev b,
                                                              const unsigned char *lend,
@@ -302,8 +364,9 @@ __global__ __launch_bounds__(kMT) void k_master_direct_steps(BodiesDev b,
                                                              const int *__restrict__ flag, int n,
                                                              int slab, double dt,
                                                              double *__restrict__ part) {
-  __shared__ double sx[kMT], sy[kMT], sz[kMT], sq[kMT], svx[kMT], svy[kMT], svz[kMT];
-  __shared__ unsigned char sf[kMT];
+  // a source: (x, y, z, mass), (velocity, mass as a source: 0 if it is none)
+  __shared__ double4 sp[kMT], sv[kMT];
+  __shared__ unsigned long long s_end[kMT / kWave];
   const int t = threadIdx.x;
   // uniform slabs: the small tree's leaf data, and (vector form) no zero
   // distances between distinct bodies
@@ -320,64 +383,76 @@ __global__ __launch_bounds__(kMT) void k_master_direct_steps(BodiesDev b,
   const double vxi = live ? b.vx[i] : 0.0, vyi = live ? b.vy[i] : 0.0,
                vzi = live ? b.vz[i] : 0.0;
   const double qi = live ? b.q[i] : 1.0;
-  double ax = 0, ay = 0, az = 0, pt = 0, ts = 1e38, mi = qi;
+  const double kff = M_SQRT2 / dt, kfb = 1.0 / dt;
+  // the running piece: the largest rate (vector form) or the smallest tau
+  constexpr double kNoTau = 1e38, kNoRate = 1e-38;
+  StepPair s = {0, 0, 0, 0, kNoRate, kNoRate, qi};
+  double ts = kNoTau;
   if (uniform && !kPairMass && j0 < j1 && j0 > 0 && !lend[j0 - 1]) {
     // the slab starts inside a leaf: its running mass up to j0
     const bool own = live && lidx[i] == lidx[j0] && i < j0;
-    mi = own ? pmx[j0] : qi + pmx[j0];
+    s.mi = own ? pmx[j0] : qi + pmx[j0];
   }
-  // pieces: first (fid, fmin), whole leaves (whole), the one open (cid)
-  double fmin_ = 0, whole = 0, lmin = 0;
+  // pieces: first (fid, first), whole leaves (whole), the one open (lid, last)
+  double first = 0, whole = 0, last = 0;
   int fid = -1, lid = -1;
   for (int base = j0; base < j1; base += kMT) {
     __syncthreads();
     const int j = base + t;
+    bool end = false;
     if (j < j1) {
-      sx[t] = b.x[j];
-      sy[t] = b.y[j];
-      sz[t] = b.z[j];
-      sq[t] = b.q[j];
-      svx[t] = b.vx[j];
-      svy[t] = b.vy[j];
-      svz[t] = b.vz[j];
-      sf[t] = ((b.flags[j] & kSource) ? 1 : 0) | (lend[j] ? 2 : 0);
+      const double q = b.q[j];
+      sp[t] = make_double4(b.x[j], b.y[j], b.z[j], q);
+      sv[t] = make_double4(b.vx[j], b.vy[j], b.vz[j], (b.flags[j] & kSource) ? q : 0.0);
+      end = lend[j] != 0;
     }
+    const unsigned long long ends = __ballot(end);
+    if ((t & (kWave - 1)) == 0) s_end[t / kWave] = ends;
     __syncthreads();
     const int cnt = min(kMT, j1 - base);
+    for (int k = 0; k < cnt;) {
+      // sources up to and with the next leaf end, within this group of 64
+      const unsigned long long m = s_end[k / kWave] >> (k & (kWave - 1));
+      int len = kWave - (k & (kWave - 1));
+      const bool close = m != 0;
+      if (close) len = __ffsll(m);
+      const int k1 = __builtin_amdgcn_readfirstlane(min(cnt, k + len));
+      k = __builtin_amdgcn_readfirstlane(k);
 #pragma unroll TC_MDS_UNROLL
-    for (int k = 0; k < cnt; k++) {
-      const double dx = sx[k] - xi, dy = sy[k] - yi, dz = sz[k] - zi;
-      const double r2 = dx * dx + dy * dy + dz * dz;
-      const unsigned char f = sf[k];
-      const double ir = rsqrt_fp64(r2 > 0 ? r2 : 1e38);
-      pair_tau<kPairMass>(dx, dy, dz, svx[k] - vxi, svy[k] - vyi, svz[k] - vzi, r2, ir, qi,
-                          sq[k], dt, mi, ts);
-      const bool use = (f & 1) && r2 > 0;
-      const double w = use ? sq[k] * ir : 0.0;
-      pt += w;
-      const double w3 = w * ir * ir;
-      ax += dx * w3;
-      ay += dy * w3;
-      az += dz * w3;
-      const bool end = (f & 2) != 0;
-      if (end || base + k == j1 - 1) {
+      for (; k < k1; k++) {
+        const double4 p = sp[k], v = sv[k];
+        const double dx = p.x - xi, dy = p.y - yi, dz = p.z - zi;
+        const double dvx = v.x - vxi, dvy = v.y - vyi, dvz = v.z - vzi;
+        const double r2 = dx * dx + dy * dy + dz * dz;
+        if (kPairMass) {
+          const double ir = rsqrt_fp64(r2 > 0 ? r2 : 1e38);
+          pair_tau<true>(dx, dy, dz, dvx, dvy, dvz, r2, ir, qi, p.w, dt, s.mi, ts);
+          const double w = r2 > 0 ? v.w * ir : 0.0;
+          s.pt += w;
+          const double w3 = w * ir * ir;
+          s.ax += dx * w3;
+          s.ay += dy * w3;
+          s.az += dz * w3;
+        } else {
+          pair_rate(dx, dy, dz, dvx, dvy, dvz, r2, p.w, v.w, kff, kfb, s);
+        }
+      }
+      if (close || base + k == j1) {
         // a piece closes: at the end of its leaf, or at the end of the slab
-        const int id = end ? base + k : lidx[base + k];
+        const int id = close ? base + k - 1 : lidx[base + k - 1];
+        const double rate = kPairMass ? 1.0 / ts : fmax(s.rate, 0.5 * s.full);
         if (fid < 0) {
           fid = id;
-          fmin_ = ts;
+          first = rate;
         } else {
-          if (lid >= 0) {
-            double t4 = lmin * lmin;
-            t4 *= t4;
-            whole += 1.0 / t4;
-          }
+          if (lid >= 0) whole += pow4(last);
           lid = id;
-          lmin = ts;
+          last = rate;
         }
-        if (end) {
-          ts = 1e38;
-          mi = qi;
+        if (close) {
+          ts = kNoTau;
+          s.rate = s.full = kNoRate;
+          s.mi = qi;
         }
       }
     }
@@ -385,38 +460,32 @@ __global__ __launch_bounds__(kMT) void k_master_direct_steps(BodiesDev b,
   if (!live) return;
   if (lid < 0) {  // one piece (or none, for an empty slab)
     lid = fid;
-    lmin = fmin_;
+    last = first;
   }
   double *o = part + (size_t)blockIdx.y * kStepCols * n + i;
-  o[0] = pt;
-  o[(size_t)n] = ax;
-  o[2 * (size_t)n] = ay;
-  o[3 * (size_t)n] = az;
+  o[0] = s.pt;
+  o[(size_t)n] = s.ax;
+  o[2 * (size_t)n] = s.ay;
+  o[3 * (size_t)n] = s.az;
   o[4 * (size_t)n] = whole;
-  o[5 * (size_t)n] = fmin_;
-  o[6 * (size_t)n] = lmin;
+  o[5 * (size_t)n] = first;
+  o[6 * (size_t)n] = last;
   o[7 * (size_t)n] = (double)fid;
   o[8 * (size_t)n] = (double)lid;
 }
 
 // A run of consecutive slabs, per target: the force sums, and its source
-// leaf pieces -- the first (id fid = the leaf's last body, running minimum
-// fmin), the sum of min^-4 over the leaves strictly between (whole), and the
-// last (lid, lmin); fid == lid for a single piece, fid = -1 for no source.
+// leaf pieces -- the first (id fid = the leaf's last body, largest rate 1 / tau
+// frate), the sum of rate^4 over the leaves strictly between (whole), and the
+// last (lid, lrate); fid == lid for a single piece, fid = -1 for no source.
 struct StepRun {
-  double v[4], whole, fmin, lmin;
+  double v[4], whole, frate, lrate;
   int fid, lid;
 };
 
-__device__ __forceinline__ double inv4(double m) {
-  double t4 = m * m;
-  t4 *= t4;
-  return 1.0 / t4;
-}
-
 // a then b: a leaf cut between the two (a's last piece and b's first have
-// one id) joins by the minimum; a piece that ends up between the new first
-// and last adds its min^-4 to whole
+// one id) joins by the maximum; a piece that ends up between the new first
+// and last adds its rate^4 to whole
 __device__ __forceinline__ StepRun join_runs(const StepRun &a, const StepRun &b) {
   StepRun r;
 #pragma unroll
@@ -424,26 +493,26 @@ __device__ __forceinline__ StepRun join_runs(const StepRun &a, const StepRun &b)
   if (a.fid < 0 || b.fid < 0) {
     const StepRun &c = a.fid < 0 ? b : a;
     r.whole = c.whole;
-    r.fmin = c.fmin;
-    r.lmin = c.lmin;
+    r.frate = c.frate;
+    r.lrate = c.lrate;
     r.fid = c.fid;
     r.lid = c.lid;
     return r;
   }
   const bool sa = a.fid == a.lid, sb = b.fid == b.lid;
   r.fid = a.fid;
-  r.fmin = a.fmin;
+  r.frate = a.frate;
   r.lid = b.lid;
-  r.lmin = b.lmin;
+  r.lrate = b.lrate;
   r.whole = a.whole + b.whole;
   if (a.lid == b.fid) {
-    const double m = fmin(a.lmin, b.fmin);
-    if (sa) r.fmin = m;
-    if (sb) r.lmin = m;
-    if (!sa && !sb) r.whole += inv4(m);
+    const double m = fmax(a.lrate, b.frate);
+    if (sa) r.frate = m;
+    if (sb) r.lrate = m;
+    if (!sa && !sb) r.whole += pow4(m);
   } else {
-    if (!sa) r.whole += inv4(a.lmin);
-    if (!sb) r.whole += inv4(b.fmin);
+    if (!sa) r.whole += pow4(a.lrate);
+    if (!sb) r.whole += pow4(b.frate);
   }
   return r;
 }
@@ -451,7 +520,7 @@ __device__ __forceinline__ StepRun join_runs(const StepRun &a, const StepRun &b)
 // Per target, the slabs' runs joined in slab order: kMergeGroups groups of
 // threads take consecutive ranges of slabs for the same 64 targets, then the
 // first group joins the groups' runs; the time-step sum is the first piece's
-// min^-4, whole, and the last piece's (for more than one piece).  Results go
+// rate^4, whole, and the last piece's (for more than one piece).  Results go
 // to the caller's order for sinks.
 constexpr int kMergeGroups = 8;
 __global__ __launch_bounds__(64 * kMergeGroups) void k_master_direct_merge(
@@ -465,7 +534,7 @@ __global__ __launch_bounds__(64 * kMergeGroups) void k_master_direct_merge(
   StepRun acc_run;
 #pragma unroll
   for (int k = 0; k < 4; k++) acc_run.v[k] = 0.0;
-  acc_run.whole = acc_run.fmin = acc_run.lmin = 0.0;
+  acc_run.whole = acc_run.frate = acc_run.lrate = 0.0;
   acc_run.fid = acc_run.lid = -1;
   if (i < n)
     for (int q = q0; q < q1; q++) {
@@ -474,8 +543,8 @@ __global__ __launch_bounds__(64 * kMergeGroups) void k_master_direct_merge(
 #pragma unroll
       for (int k = 0; k < 4; k++) c.v[k] = r[(size_t)k * n];
       c.whole = r[4 * (size_t)n];
-      c.fmin = r[5 * (size_t)n];
-      c.lmin = r[6 * (size_t)n];
+      c.frate = r[5 * (size_t)n];
+      c.lrate = r[6 * (size_t)n];
       c.fid = (int)r[7 * (size_t)n];
       c.lid = (int)r[8 * (size_t)n];
       acc_run = join_runs(acc_run, c);
@@ -486,8 +555,8 @@ __global__ __launch_bounds__(64 * kMergeGroups) void k_master_direct_merge(
   for (int u = 1; u < kMergeGroups; u++) acc_run = join_runs(acc_run, runs[u][lane]);
   double tsum = 0.0;
   if (acc_run.fid >= 0) {
-    tsum = inv4(acc_run.fmin) + acc_run.whole;
-    if (acc_run.lid != acc_run.fid) tsum += inv4(acc_run.lmin);
+    tsum = pow4(acc_run.frate) + acc_run.whole;
+    if (acc_run.lid != acc_run.fid) tsum += pow4(acc_run.lrate);
   }
   const bool sink = b.flags[i] & kSink;
   const int o = b.order[i];
