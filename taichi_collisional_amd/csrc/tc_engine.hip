@@ -696,22 +696,6 @@ static int m2l_by_order(tc_context *ctx, M2LArgs ma, int nchunks) {
   return 0;
 }
 
-// The all-pairs branch's sums (caller order) into the outputs; bodies that
-// are not sinks get zeros (any output may be null).
-__global__ void k_direct_out(const unsigned char *__restrict__ flags, int n,
-                             const double *__restrict__ p, const double *__restrict__ a,
-                             const double *__restrict__ j, double *__restrict__ pot,
-                             double *__restrict__ acc, double *__restrict__ jerk) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  const bool sink = !flags || (flags[i] & kSink);
-  if (pot) pot[i] = sink ? p[i] : 0.0;
-  for (int d = 0; d < 3; d++) {
-    if (acc) acc[3 * (size_t)i + d] = sink ? a[3 * (size_t)i + d] : 0.0;
-    if (jerk) jerk[3 * (size_t)i + d] = sink ? j[3 * (size_t)i + d] : 0.0;
-  }
-}
-
 static int eval_device(tc_context *ctx, int n, const double *x, const double *v, const double *m,
                        const unsigned char *flags, double *pot, double *acc, double *jerk) {
   hipStream_t s = ctx->stream;
@@ -725,7 +709,6 @@ static int eval_device(tc_context *ctx, int n, const double *x, const double *v,
     ctx->err = "n must be positive";
     return -1;
   }
-  if (int e = ensure_bodies(ctx, n)) return e;
   // root-shift values: three drand48() per evaluation, as getBounds draws them
   // (a forest: three per cluster, in cluster order)
   double u[3];
@@ -750,24 +733,14 @@ static int eval_device(tc_context *ctx, int n, const double *x, const double *v,
 
   if (cfg.direct_below > 0 && n < cfg.direct_below && ctx->ncl == 1) {
     // all-pairs sum in the caller's order (direct(), traverse_eager.h:295-304)
-    BodiesDev b = bodies_of(ctx);
-    TC_CHECK(ctx->dtg.ensure(sizeof(int) * n));
-    launch_iota(ctx->dtg.as<int>(), n, s);
-    launch_gather(x, v, m, flags, ctx->dtg.as<int>(), n, b, s);
-    TC_CHECK(ctx->dpot.ensure(sizeof(double) * n));
-    TC_CHECK(ctx->dacc.ensure(sizeof(double) * 3 * n));
-    TC_CHECK(ctx->djerk.ensure(sizeof(double) * 3 * n));
-    launch_direct(b, n, ctx->dtg.as<int>(), n, ctx->dpot.as<double>(), ctx->dacc.as<double>(),
-                  ctx->djerk.as<double>(), s);
-    // to the outputs; non-sinks receive nothing
-    hipLaunchKernelGGL(k_direct_out, dim3((n + 255) / 256), dim3(256), 0, s, flags, n,
-                       ctx->dpot.as<double>(), ctx->dacc.as<double>(), ctx->djerk.as<double>(),
-                       pot, acc, jerk);
-    TC_CHECK(hipStreamSynchronize(s));
+    TC_CHECK(ctx->mdpart.ensure(sizeof(double) * 7 * (size_t)direct_eval_slabs(n) * n));
+    launch_direct_eval(x, v, m, flags, n, ctx->mdpart.as<double>(), pot, acc, jerk, s);
+    TC_CHECK(spin_wait(ctx, s));
     TC_CHECK(hipGetLastError());
     return 0;
   }
 
+  if (int e = ensure_bodies(ctx, n)) return e;
   // ---- tree
   if (int e = sort_and_build(ctx, n, x, v, m, flags)) return e;
   const bool err_mac = cfg.mac == TC_MAC_ERROR;

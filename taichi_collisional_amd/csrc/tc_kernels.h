@@ -253,6 +253,12 @@ int launch_direct(BodiesDev b, int n, const int *targets, int nt, double *pot, d
 int launch_direct_sum(BodiesDev b, int n, const int *targets, int nt, double *pot, double *acc,
                       double *jerk, hipStream_t s);
 void launch_zero_f64(double *p, size_t n, hipStream_t s);
+// all pairs of n bodies in the caller's order (flags may be null); part: scratch
+// of 7 n direct_eval_slabs(n) doubles
+int direct_eval_slabs(int n);
+int launch_direct_eval(const double *x3, const double *v3, const double *m,
+                       const unsigned char *flags, int n, double *part, double *pot,
+                       double *acc3, double *jerk3, hipStream_t s);
 
 // ---- p = 2 pre-pass and multipole norms (tc_low.hip)
 int launch_low_upward(CellsDev c, BodiesDev b, const int *leaf_ids, int nleaves,

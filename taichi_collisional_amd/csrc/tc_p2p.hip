@@ -617,6 +617,94 @@ int launch_direct_sum(BodiesDev b, int n, const int *targets, int nt, double *po
   return 0;
 }
 
+// The all-pairs evaluation of a small system in the caller's order, straight
+// from its arrays: a block sums one slab of sources (staged in LDS) for 256
+// targets into part[slab][7][n], and k_direct_join adds the slabs in order and
+// writes the outputs (zeros for bodies that are not sinks).  Two launches; the
+// gather, six clears and the sum with atomics that k_direct needs were ten, and
+// its slabs of at least 256 sources left most of the chip idle: N = 1,009 91 ->
+// 33 us (6 and 5 us of them the kernels), N = 7,999 152 -> 115.
+__global__ __launch_bounds__(256) void k_direct_slab(const double *__restrict__ x3,
+                                                     const double *__restrict__ v3,
+                                                     const double *__restrict__ m,
+                                                     const unsigned char *__restrict__ flags,
+                                                     int n, int slab,
+                                                     double *__restrict__ part) {
+  __shared__ double4 sp[256], sv[256];
+  const int t = threadIdx.x, i = blockIdx.x * 256 + t;
+  const int j0 = blockIdx.y * slab, j1 = min(n, j0 + slab);
+  const size_t ii = i < n ? i : 0;
+  const double xi = x3[3 * ii], yi = x3[3 * ii + 1], zi = x3[3 * ii + 2];
+  const double vxi = v3[3 * ii], vyi = v3[3 * ii + 1], vzi = v3[3 * ii + 2];
+  Acc7 a = {0, 0, 0, 0, 0, 0, 0};
+  double kx = 0, ky = 0, kz = 0;
+  for (int base = j0; base < j1; base += 256) {
+    __syncthreads();
+    const size_t j = base + t;
+    if ((int)j < j1) {
+      const bool src = !flags || (flags[j] & kSource);
+      sp[t] = make_double4(x3[3 * j], x3[3 * j + 1], x3[3 * j + 2], src ? m[j] : 0.0);
+      sv[t] = make_double4(v3[3 * j], v3[3 * j + 1], v3[3 * j + 2], 0.0);
+    }
+    __syncthreads();
+    const int cnt = min(256, j1 - base);
+#pragma unroll 2
+    for (int q = 0; q < cnt; q++)
+      pair_fp64k(xi, yi, zi, vxi, vyi, vzi, sp[q], sv[q], a, kx, ky, kz);
+  }
+  if (i >= n) return;
+  double *o = part + (size_t)blockIdx.y * 7 * n + i;
+  o[0] = a.p;
+  o[(size_t)n] = a.ax;
+  o[2 * (size_t)n] = a.ay;
+  o[3 * (size_t)n] = a.az;
+  o[4 * (size_t)n] = a.jx - 3.0 * kx;
+  o[5 * (size_t)n] = a.jy - 3.0 * ky;
+  o[6 * (size_t)n] = a.jz - 3.0 * kz;
+}
+
+__global__ __launch_bounds__(64) void k_direct_join(const double *__restrict__ part, int nslab,
+                                                    const unsigned char *__restrict__ flags,
+                                                    int n, double *__restrict__ pot,
+                                                    double *__restrict__ acc,
+                                                    double *__restrict__ jerk) {
+  const int i = blockIdx.x * 64 + threadIdx.x, c = blockIdx.y;  // component c of body i
+  if (i >= n) return;
+  const double *p = part + (size_t)c * n + i;
+  double s = 0.0;
+#pragma unroll 8
+  for (int q = 0; q < nslab; q++) s += p[(size_t)q * 7 * n];
+  if (flags && !(flags[i] & kSink)) s = 0.0;
+  if (c == 0) {
+    if (pot) pot[i] = s;
+  } else if (c < 4) {
+    if (acc) acc[3 * (size_t)i + c - 1] = s;
+  } else {
+    if (jerk) jerk[3 * (size_t)i + c - 4] = s;
+  }
+}
+
+// Slabs of at least 16 sources: about 1,024 blocks (four waves a SIMD), and
+// for systems of more than 32 target blocks (a direct_below that large) at
+// least 2,048, so that the last round of blocks is a small part.
+int direct_eval_slabs(int n) {
+  const int bx = (n + 255) / 256;
+  return std::max(1, std::min((n + 15) / 16, bx <= 32 ? 1024 / bx : (2048 + bx - 1) / bx));
+}
+
+int launch_direct_eval(const double *x3, const double *v3, const double *m,
+                       const unsigned char *flags, int n, double *part, double *pot,
+                       double *acc3, double *jerk3, hipStream_t s) {
+  if (n <= 0) return 0;
+  const int want = direct_eval_slabs(n), slab = (n + want - 1) / want;
+  const int nslab = (n + slab - 1) / slab;
+  hipLaunchKernelGGL(k_direct_slab, dim3((n + 255) / 256, nslab), dim3(256), 0, s, x3, v3, m,
+                     flags, n, slab, part);
+  hipLaunchKernelGGL(k_direct_join, dim3((n + 63) / 64, 7), dim3(64), 0, s, part, nslab, flags,
+                     n, pot, acc3, jerk3);
+  return 0;
+}
+
 // ---- results back to the caller's body order (after the downward pass)
 __global__ void k_scatter_results(BodiesDev b, ResultsDev r, int n, double *__restrict__ pot,
                                   double *__restrict__ acc, double *__restrict__ jerk) {
