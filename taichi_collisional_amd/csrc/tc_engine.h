@@ -115,7 +115,7 @@ struct tc_context {
   int cap_c = 0;
   DBuf clevel, cnchild, cchild, cbody, cnbody, cparent, cXg, cRg, cX, cR, cmin, csink;
   DBuf cM, cMd, cL, cLd;
-  DBuf split_offs, split_nch, split_scan, scan_tmp;
+  DBuf scan_tmp;
   std::vector<int> level_start;
   DBuf leaf_ids;
   HBuf<int> h_leaves, h_nbd, h_pcnt, h_tree;
@@ -127,7 +127,7 @@ struct tc_context {
   int nleaves = 0;
   // traversal / lists
   DBuf front_a, front_b, m2l, p2p, tstate, twords, tcls;
-  unsigned trav_tag = 0;  // of the last walk step (the scan words' tags)
+  unsigned scan_tag = 0;  // of the last tree level or walk step (the scan words' tags)
   int trav_steps[4] = {0, 0, 0, 0};  // steps of the last walk per MAC mode (batch size)
   DBuf gsort1[4], gsort2[4];  // list grouping scratch per stream: keys in, out, sources, temp
   int *h_pin = nullptr;  // small pinned host buffer for per-step counts (256 ints)

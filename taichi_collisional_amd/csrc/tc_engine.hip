@@ -78,9 +78,23 @@ static int ensure_cells(tc_context *ctx, int nc, int keep) {
   return 0;
 }
 
+// The scan words of tree levels and walk steps: cleared when they are new or
+// the tags run out, so that no launch finds its own tag there (a tag per
+// launch, fewer than 2^20 between two calls).
+static int scan_words(tc_context *ctx, size_t words) {
+  const size_t bytes = sizeof(unsigned long long) * words;
+  if (ctx->twords.bytes < bytes || ctx->scan_tag > (1u << 27)) {
+    TC_CHECK(ctx->twords.ensure(bytes));
+    TC_CHECK(hipMemsetAsync(ctx->twords.p, 0, ctx->twords.bytes, ctx->stream));
+    ctx->scan_tag = 0;
+  }
+  return 0;
+}
+
 // Tree levels are queued in batches without host reads (TreeState on the
 // device holds the level range and counts); a batch's last level reports the
-// state to pinned memory, which says whether it had no children.  A level whose children do not fit
+// state to pinned memory, which says whether it had no children.  A level whose
+// children do not fit
 // the cell arrays ends the build with a flag and what it needed: the arrays
 // grow and the build starts again from the root (a new workload's first
 // evaluation, or a tree that a new root shift makes larger).
@@ -97,27 +111,28 @@ static int build_tree(tc_context *ctx, int n) {
   const TreeState *hst = reinterpret_cast<const TreeState *>(ctx->h_tree.p);
   TreeState *dst = nullptr;  // the same memory as kernels address it
   TC_CHECK(hipHostGetDevicePointer((void **)&dst, ctx->h_tree.p, 0));
+  int last = 0;  // parity of the state after the last queued level
   for (int attempt = 0;; attempt++) {
     if (attempt > 16) {
       ctx->err = "tree build: cell arrays keep overflowing";
       return -3;
     }
     const int cap = ctx->cap_c;
-    TC_CHECK(ctx->split_offs.ensure(sizeof(int) * 8 * (size_t)cap));
-    TC_CHECK(ctx->split_nch.ensure(sizeof(int) * 2 * (size_t)cap));
-    TC_CHECK(ctx->split_scan.ensure(sizeof(int) * 2 * (size_t)cap));
+    if (int e = scan_words(ctx, tree_words((size_t)cap))) return e;
+    // two blocks a CU; a small system's levels are a cell per thousand bodies
+    const int nblocks = std::min(512, std::max(8, n / 512));
     // one root, or one per cluster of a forest
     launch_root(cells_of(ctx), n, ctx->tp.as<TreeParams>(), ctx->tree_state.as<TreeState>(), s,
                 ctx->ncl > 1 ? ctx->cl_start.as<int>() : nullptr, ctx->ncl);
     int queued = 0, batch = std::max(4, ctx->tree_levels + 1);
     for (;;) {
       for (int i = 0; i < batch; i++, queued++)
-        launch_tree_level(cells_of(ctx), b, ctx->tree_state.as<TreeState>(), ncrit, cap,
-                          ctx->split_offs.as<int>(), ctx->split_nch.as<int>(),
-                          ctx->split_scan.as<int>(), ctx->tp.as<TreeParams>(),
-                          ctx->leaf_ids.as<int>(), i == batch - 1 ? dst : nullptr, s);
+        launch_tree_level(cells_of(ctx), b, ctx->tree_state.as<TreeState>(), queued & 1,
+                          ++ctx->scan_tag, ctx->twords.as<unsigned long long>(), nblocks, ncrit,
+                          cap, ctx->leaf_ids.as<int>(), i == batch - 1 ? dst : nullptr, s);
       TC_CHECK(spin_wait(ctx, s));
-      if (hst->done || hst->overflow) break;
+      last = queued & 1;
+      if (hst->ls[last] == hst->le[last] || hst->overflow) break;
       if (queued > 4 * kMaxTreeLevels) {
         ctx->err = "tree build does not end";
         return -3;
@@ -131,9 +146,9 @@ static int build_tree(tc_context *ctx, int n) {
     if (!hst->overflow) break;
     if (int e = ensure_cells(ctx, hst->need, 0)) return e;
   }
-  ctx->tree_levels = hst->nlev;
-  ctx->level_start.assign(hst->level_start, hst->level_start + hst->nlev + 1);
-  const int depth = hst->nlev - 1, nleaf = hst->nleaf;
+  const int nlev = hst->nlev[last], nleaf = hst->nleaf[last], depth = nlev - 1;
+  ctx->tree_levels = nlev;
+  ctx->level_start.assign(hst->level_start, hst->level_start + nlev + 1);
   // level_start holds the start of every level and, last, the total cell count
   int nc = ctx->level_start.back();
   ctx->st.ncells = nc;
@@ -254,14 +269,7 @@ static int traverse(tc_context *ctx, int n, const MacArgs &mac) {
     const long long cm = cap(ctx->m2l), cp = cap(ctx->p2p),
                     cf = std::min({cap(ctx->front_a), cap(ctx->front_b),
                                    (long long)std::min<size_t>(ctx->tcls.bytes, 0x7fffffff)});
-    // the scan's words: cleared when they are new or the tags run out, so that
-    // no step finds its own tag there
-    const size_t wb = sizeof(unsigned long long) * kTravWords;
-    if (ctx->twords.bytes < wb || ctx->trav_tag > (1u << 27)) {
-      TC_CHECK(ctx->twords.ensure(wb));
-      TC_CHECK(hipMemsetAsync(ctx->twords.p, 0, ctx->twords.bytes, s));
-      ctx->trav_tag = 0;
-    }
+    if (int e = scan_words(ctx, kTravWords)) return e;
     // a small system's frontiers are a few pairs per body
     const int nblocks = std::min(kTravBlocks, std::max(64, n / 32));
     launch_root_pairs(ctx->front_a.as<int2>(), ctx->ncl, ctx->tstate.as<TravState>(), s);
@@ -277,7 +285,7 @@ static int traverse(tc_context *ctx, int n, const MacArgs &mac) {
         a.cls = ctx->tcls.as<unsigned char>();
         a.mac = mac;
         launch_trav_step(cells_of(ctx), a, ctx->tstate.as<TravState>(), (int)odd,
-                         ++ctx->trav_tag, ctx->twords.as<unsigned long long>(), nblocks, cm, cp,
+                         ++ctx->scan_tag, ctx->twords.as<unsigned long long>(), nblocks, cm, cp,
                          cf, i == batch - 1 ? dst : nullptr, s);
       }
       TC_CHECK(spin_wait(ctx, s));
@@ -1213,8 +1221,7 @@ int tc_destroy(tc_context *ctx) {
                  &ctx->key_b, &ctx->val_a, &ctx->val_b, &ctx->sort_tmp, &ctx->part, &ctx->tp,
                  &ctx->dshift, &ctx->clevel, &ctx->cnchild, &ctx->cchild, &ctx->cparent, &ctx->cbody,
                  &ctx->cnbody, &ctx->cXg, &ctx->cRg, &ctx->cX, &ctx->cR, &ctx->cmin, &ctx->csink,
-                 &ctx->cM, &ctx->cMd, &ctx->cL, &ctx->cLd, &ctx->split_offs, &ctx->split_nch,
-                 &ctx->split_scan, &ctx->scan_tmp, &ctx->leaf_ids, &ctx->front_a, &ctx->front_b,
+                 &ctx->cM, &ctx->cMd, &ctx->cL, &ctx->cLd, &ctx->scan_tmp, &ctx->leaf_ids, &ctx->front_a, &ctx->front_b,
                  &ctx->m2l, &ctx->p2p, &ctx->tstate, &ctx->twords, &ctx->tcls, &ctx->tree_state,
                  &ctx->gsort1[0], &ctx->gsort1[1], &ctx->gsort1[2], &ctx->gsort1[3], &ctx->gsort2[0], &ctx->gsort2[1], &ctx->gsort2[2], &ctx->gsort2[3], &ctx->m2l_cnt, &ctx->m2l_off, &ctx->m2l_cur,
                  &ctx->m2l_src, &ctx->m2l_coff, &ctx->m2l_chunks, &ctx->p2p_cnt, &ctx->p2p_off,

@@ -87,25 +87,26 @@ int launch_sort(uint64_t *key_a, uint64_t *key_b, int *val_a, int *val_b, const 
 int launch_gather(const double *x3, const double *v3, const double *q,
                   const unsigned char *flags_in, const int *perm, int n, BodiesDev b,
                   hipStream_t s);
-// Device-side state of a tree build (ints): the level being split [ls, le),
-// leaves and levels so far, the level being placed (cls, cle, its first leaf
-// slot cbase, go), done, overflow (1: the cell arrays are too small, need
-// cells; 2: deeper than kMaxTreeLevels) and level_start[0..nlev].
+// Device-side state of a tree build, by level parity: the level to split
+// [ls, le) (empty when the tree is done), leaves and levels so far, tiles
+// taken; and overflow (1: the cell arrays are too small, need cells; 2: deeper
+// than kMaxTreeLevels) and level_start[0..nlev].
 constexpr int kMaxTreeLevels = 64;
 struct TreeState {
-  int ls, le, nleaf, nlev;
-  int cls, cle, cbase, go;
-  int done, overflow, need, pad;
+  int ls[2], le[2], nleaf[2], nlev[2], ticket[2];
+  int overflow, need;
   int level_start[kMaxTreeLevels + 4];
 };
 // the root cells, and the state of a build that starts with them
 int launch_root(CellsDev c, int n, const TreeParams *d_tp, TreeState *st, hipStream_t s,
                 const int *start = nullptr, int ncl = 1);
-// One level: split (offs, nch), scans (scan), children and leaves.  Arrays of
-// per-level cells hold cap entries (nch and scan: 2 x cap).
+// One level, of parity par, by nblocks blocks; tag, words (tree_words(cap)): as
+// for a walk step; cap: cells that the cell arrays hold.
 // report (or null): pinned host memory that receives the state after the level.
-int launch_tree_level(CellsDev c, BodiesDev b, TreeState *st, int ncrit, int cap, int *offs,
-                      int *nch, int *scan, const TreeParams *d_tp, int *leaf_ids,
+constexpr int kTreeThreads = 512;  // 64 cells a tile
+constexpr size_t tree_words(size_t cells) { return 6 * (cells / (kTreeThreads / 8) + 1); }
+int launch_tree_level(CellsDev c, BodiesDev b, TreeState *st, int par, unsigned tag,
+                      unsigned long long *words, int nblocks, int ncrit, int cap, int *leaf_ids,
                       TreeState *report, hipStream_t s);
 // The whole tree of at most kSmallTree bodies in one launch (one workgroup),
 // for the master time-step sums: bodies gathered into tree order, lend set on

@@ -315,6 +315,83 @@ int launch_gather(const double *x3, const double *v3, const double *q,
   return 0;
 }
 
+// ---------------------------------------------------- scans in a launch -----
+// Exclusive scan of three ints over a block of NW waves; totals to *tot.
+template <int NW>
+__device__ __forceinline__ int3 block_excl_scan3_n(int3 v, int3 *tot) {
+  __shared__ int3 wsum[NW];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int tx, ty, tz;
+  int ex = wave_excl_scan(v.x, &tx), ey = wave_excl_scan(v.y, &ty), ez = wave_excl_scan(v.z, &tz);
+  if (lane == 0) wsum[w] = make_int3(tx, ty, tz);
+  __syncthreads();
+  int3 base = make_int3(0, 0, 0), all = make_int3(0, 0, 0);
+  for (int k = 0; k < NW; k++) {
+    int3 q = wsum[k];
+    if (k < w) base = make_int3(base.x + q.x, base.y + q.y, base.z + q.z);
+    all = make_int3(all.x + q.x, all.y + q.y, all.z + q.z);
+  }
+  *tot = all;
+  __syncthreads();
+  return make_int3(base.x + ex, base.y + ey, base.z + ez);
+}
+
+__device__ __forceinline__ int wave_sum_i(int v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
+  return v;
+}
+
+// A block's words for a scan over a launch's ranges (a tree level's cells, a
+// walk step's pairs): its own three counts and, later, the sums up to and with
+// it.  A word is the value and, above kScanTagShift, the launch's tag: words of
+// other launches read as not there yet, so nothing is cleared in between, and
+// value and tag arrive together (one 64-bit store), so no ordering is needed
+// between the words.
+constexpr int kScanTagShift = 36;
+__device__ __forceinline__ void scan_put(unsigned long long *w, int v, unsigned tag) {
+  __hip_atomic_store(w, (unsigned long long)(unsigned)v | (unsigned long long)tag << kScanTagShift,
+                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ unsigned long long scan_get(const unsigned long long *w) {
+  return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Sums of the counts of the ranges before `range`, by one wave: 64 ranges at a
+// time, nearest first, until one whose sums are known.  Ranges are numbered in
+// the order in which blocks start on them, and a range's counts are stored
+// before its block waits for anything, so every word looked for here arrives.
+__device__ __forceinline__ int3 look_back(const unsigned long long *words, int range,
+                                               unsigned tag) {
+  const int lane = threadIdx.x & (kWave - 1);
+  int3 sum = make_int3(0, 0, 0);
+  for (int last = range - 1; last >= 0;) {
+    const int k = last - lane;
+    unsigned long long w[6] = {0, 0, 0, 0, 0, 0};
+    if (k >= 0)
+      for (int q = 0; q < 6; q++) w[q] = scan_get(words + 6 * k + q);
+    auto here = [&](int q) { return (unsigned)(w[q] >> kScanTagShift) == tag; };
+    const bool counts = here(0) && here(1) && here(2), sums = here(3) && here(4) && here(5);
+    const unsigned long long known = __ballot(k >= 0 && sums);
+    const unsigned long long ready = __ballot(k < 0 || sums || counts);
+    const int stop = known ? __ffsll(known) - 1 : kWave;  // lanes before it add their counts
+    const unsigned long long need = stop < kWave ? (1ull << stop) - 1 : ~0ull;
+    if ((ready & need) != need) {
+      __builtin_amdgcn_s_sleep(1);
+      continue;
+    }
+    int3 v = make_int3(0, 0, 0);
+    if (k >= 0 && lane < stop) v = make_int3((int)(unsigned)w[0], (int)(unsigned)w[1],
+                                             (int)(unsigned)w[2]);
+    if (k >= 0 && lane == stop) v = make_int3((int)(unsigned)w[3], (int)(unsigned)w[4],
+                                              (int)(unsigned)w[5]);
+    sum = make_int3(sum.x + wave_sum_i(v.x), sum.y + wave_sum_i(v.y), sum.z + wave_sum_i(v.z));
+    if (known) break;
+    last -= kWave;
+  }
+  return sum;
+}
+
 // ---------------------------------------------------------------- cells -----
 // Root cells: one (all n bodies), or one per cluster of a forest (cluster k
 // = [start[k], start[k+1]) with its own TreeParams).
@@ -324,7 +401,7 @@ __global__ void k_root(CellsDev c, int n, const TreeParams *__restrict__ tp, Tre
   if (blockIdx.x == 0) {
     int *w = reinterpret_cast<int *>(st);
     for (int t = threadIdx.x; t < (int)(sizeof(TreeState) / sizeof(int)); t += 64)
-      w[t] = t == offsetof(TreeState, le) / sizeof(int) ? ncl : 0;
+      w[t] = t == (int)(offsetof(TreeState, le) / sizeof(int)) ? ncl : 0;  // le[0]
   }
   const int k = blockIdx.x * 64 + threadIdx.x;
   if (k >= ncl) return;
@@ -348,48 +425,69 @@ __device__ __forceinline__ int octant_of(const BodiesDev &b, int i, double X0, d
   return (b.x[i] >= X0) + ((b.y[i] >= X1) << 1) + ((b.z[i] >= X2) << 2);
 }
 
-// One level of the tree build, queued without host reads: the level's range
-// and the running counts live in TreeState.  Arrays of the level's cells
-// (offs: 8 octant starts per cell; nch: child counts, and at nch + cap the
-// leaf flags; scan: their exclusive scans, the same layout) hold up to cap
-// cells.
+// One level of the tree build in one launch, queued without host reads: the
+// level's range and the running counts live in TreeState, two of each by level
+// parity (a level reads its own and the block of its last tile sets the next
+// level's).
 //
-// Split: eight lanes per cell, lane j for octant j; above 32 bodies lane j > 0
-// runs the binary search for the start of octants >= j (the search never
-// tests the cell's first body, as the reference's does not, so its start is
-// l + 1); the seven searches run side by side instead of one after another
-// (the top levels' cells hold up to all N bodies, and their splits are chains
-// of dependent loads).  Up to 32 bodies lane j counts octant j's bodies.
-__global__ __launch_bounds__(256) void k_split(CellsDev c, BodiesDev b,
-                                               const TreeState *__restrict__ st, int ncrit,
-                                               int cap, int *__restrict__ offs,
-                                               int *__restrict__ nch) {
-  if (st->done || st->overflow) return;
-  const int ls = st->ls, nl = st->le - ls;
-  const int j = threadIdx.x & 7, lane = threadIdx.x & (kWave - 1);
-  for (int k = (blockIdx.x * 256 + (int)threadIdx.x) >> 3; k < nl; k += gridDim.x * 32) {
-    const int ci = ls + k;
-    const int nb = c.nbody[ci];
-    if (nb <= ncrit) {
-      if (j == 0) {
-        nch[cap + k] = 1;
-        nch[k] = 0;
-        c.nchild[ci] = 0;
-        c.child[ci] = -1;
-      }
-      continue;
+// Eight lanes per cell, lane j for octant j; above 32 bodies lane j > 0 runs
+// the binary search for the start of octants >= j (the search never tests the
+// cell's first body, as the reference's does not, so its start is l + 1); the
+// seven searches run side by side instead of one after another (the top
+// levels' cells hold up to all N bodies, and their splits are chains of
+// dependent loads).  Up to 32 bodies lane j counts octant j's bodies.  The
+// child counts and leaf flags of a tile of 64 cells are placed by a scan over
+// the tiles while they run (look_back), and each lane writes its child.  A
+// level whose children would not fit the cell arrays sets overflow = 1 and what
+// it needed, a level past kMaxTreeLevels overflow = 2.  N = 10,007 under the
+// profiler: 36 us a level in three launches (split, scan, children), 12 in one.
+__global__ __launch_bounds__(kTreeThreads) void k_tree_level(
+    CellsDev c, BodiesDev b, TreeState *st, int par, unsigned tag,
+    unsigned long long *__restrict__ words, int ncrit, int cap, int *__restrict__ leaf_ids,
+    TreeState *report) {
+#pragma clang fp contract(off)
+  constexpr int T = kTreeThreads, NW = T / kWave, kCells = T / 8;
+  __shared__ int s_tile;
+  __shared__ int3 s_before;
+  const int t = threadIdx.x, j = t & 7, lane = t & (kWave - 1);
+  const int ls = st->ls[par], le = st->le[par], nleaf = st->nleaf[par], nlev = st->nlev[par];
+  const int nl = le - ls;
+  if (nl == 0 || nlev >= kMaxTreeLevels) {
+    // done before this level, or too deep
+    if (blockIdx.x == 0 && t == 0) {
+      if (nl > 0) st->overflow = 2;
+      st->ls[par ^ 1] = st->le[par ^ 1] = le;
+      st->nleaf[par ^ 1] = nleaf;
+      st->nlev[par ^ 1] = nlev;
+      st->ticket[par ^ 1] = 0;
+      if (report) *report = *st;
     }
-    const int begin = c.body[ci], end = begin + nb;
-    const double X0 = c.Xg[3 * ci], X1 = c.Xg[3 * ci + 1], X2 = c.Xg[3 * ci + 2];
+    return;
+  }
+  const int ntiles = (nl + kCells - 1) / kCells;
+  if ((int)blockIdx.x >= ntiles) return;
+  for (;;) {
+    if (t == 0) s_tile = atomicAdd(&st->ticket[par], 1);
+    __syncthreads();
+    const int tile = s_tile;
+    if (tile >= ntiles) return;
+    const int k = tile * kCells + (t >> 3), ci = ls + k;
+    const bool in = k < nl;
+    const int nb = in ? c.nbody[ci] : 0;
+    const bool split = nb > ncrit;
+    const int begin = in ? c.body[ci] : 0, end = begin + nb;
+    double X[3] = {0, 0, 0};
+    if (split)
+      for (int d = 0; d < 3; d++) X[d] = c.Xg[3 * ci + d];
     const bool small = nb <= 32;
     int o = begin, sz = 0;
-    if (small) {
-      for (int i = begin; i < end; i++) sz += octant_of(b, i, X0, X1, X2) == j;
-    } else if (j > 0) {
+    if (split && small) {
+      for (int i = begin; i < end; i++) sz += octant_of(b, i, X[0], X[1], X[2]) == j;
+    } else if (split && j > 0) {
       int l = begin, r = end;
       while (l < r - 1) {
         const int mid = (l + r) / 2;
-        if (octant_of(b, mid, X0, X1, X2) >= j)
+        if (octant_of(b, mid, X[0], X[1], X[2]) >= j)
           r = mid;
         else
           l = mid;
@@ -400,180 +498,84 @@ __global__ __launch_bounds__(256) void k_split(CellsDev c, BodiesDev b,
     int incl = sz;
 #pragma unroll
     for (int d = 1; d < 8; d <<= 1) {
-      const int t = __shfl(incl, lane - d, kWave);
-      if (j >= d) incl += t;
+      const int up = __shfl(incl, lane - d, kWave);
+      if (j >= d) incl += up;
     }
     const int onext = __shfl(o, lane + 1, kWave);
     if (small)
       o = begin + incl - sz;
     else
       sz = (j < 7 ? onext : end) - o;
-    offs[8 * k + j] = o;
-    const unsigned long long nz = __ballot(sz != 0);
-    const int cnt = __popcll((nz >> (lane & ~7)) & 0xffull);
-    if (j == 0) {
-      nch[cap + k] = 0;
-      nch[k] = cnt;
+    if (!split) sz = 0;
+    const unsigned kids = (unsigned)(__ballot(sz != 0) >> (lane & ~7)) & 0xffu;
+    const int cnt = __popc(kids), rank = __popc(kids & ((1u << j) - 1));
+    const bool leaf = in && !split;
+    int3 tot;
+    const int3 ex =
+        block_excl_scan3_n<NW>(make_int3(j == 0 ? cnt : 0, j == 0 && leaf, 0), &tot);
+    if (t < kWave) {
+      unsigned long long *w = words + 6 * (size_t)tile;
+      if (t == 0) {
+        scan_put(w, tot.x, tag);
+        scan_put(w + 1, tot.y, tag);
+        scan_put(w + 2, 0, tag);
+      }
+      const int3 before = look_back(words, tile, tag);
+      if (t == 0) {
+        const int children = before.x + tot.x, leaves = before.y + tot.y;
+        scan_put(w + 3, children, tag);
+        scan_put(w + 4, leaves, tag);
+        scan_put(w + 5, 0, tag);
+        s_before = before;
+        if (tile == ntiles - 1) {
+          const long long all = (long long)le + children;
+          const bool fits = all <= cap;
+          if (!fits) {
+            st->overflow = 1;
+            st->need = (int)(all < 0x7fffffff ? all : 0x7fffffff);
+          }
+          st->ls[par ^ 1] = le;
+          st->le[par ^ 1] = fits ? (int)all : le;
+          st->nleaf[par ^ 1] = nleaf + leaves;
+          st->nlev[par ^ 1] = nlev + 1;
+          st->level_start[nlev + 1] = le;
+          st->ticket[par ^ 1] = 0;
+          if (report) *report = *st;
+        }
+      }
+    }
+    __syncthreads();
+    // lane 0 of a group holds the cell's own offsets
+    const int first = le + s_before.x + __shfl(ex.x, lane & ~7, kWave);
+    if (in && j == 0) {
       c.nchild[ci] = cnt;
+      c.child[ci] = split ? first : -1;
+      if (leaf) leaf_ids[nleaf + s_before.y + ex.y] = ci;
     }
-  }
-}
-
-// Exclusive scans of the level's child counts and leaf flags (one block), and
-// the state: the level the children kernel places (cls, cle, cbase, go), the
-// next level, the leaves and levels so far.  A level whose children would not
-// fit the cell arrays sets overflow = 1 and what it needed; a level past
-// kMaxTreeLevels sets overflow = 2.
-__global__ __launch_bounds__(1024) void k_level_scan(const int *__restrict__ nch,
-                                                     int *__restrict__ scan, TreeState *st,
-                                                     int cap, TreeState *report) {
-  __shared__ int wsum[2][16];
-  __shared__ int carry[2];
-  if (st->done || st->overflow) {
-    if (threadIdx.x == 0) {
-      st->go = 0;
-      if (report) *report = *st;
-    }
-    return;
-  }
-  const int ls = st->ls, le = st->le, nl = le - ls;
-  const int t = threadIdx.x, lane = t & (kWave - 1), w = t / kWave;
-  if (t < 2) carry[t] = 0;
-  __syncthreads();
-  // both arrays in one pass over tiles of 16 per thread (a 24k-cell level is
-  // two tiles): each tile is a few global-load and barrier round trips
-  constexpr int PER = 16, TILE = 1024 * PER;
-  for (int base = 0; base < nl; base += TILE) {
-    int v0[PER], v1[PER], s0 = 0, s1 = 0;
-#pragma unroll
-    for (int q = 0; q < PER; q++) {
-      const int i = base + t * PER + q;
-      v0[q] = i < nl ? nch[i] : 0;
-      v1[q] = i < nl ? nch[(size_t)cap + i] : 0;
-      s0 += v0[q];
-      s1 += v1[q];
-    }
-    int wt0, wt1;
-    const int ex0 = wave_excl_scan(s0, &wt0);
-    const int ex1 = wave_excl_scan(s1, &wt1);
-    if (lane == 0) {
-      wsum[0][w] = wt0;
-      wsum[1][w] = wt1;
-    }
-    __syncthreads();
-    int r0 = carry[0], r1 = carry[1], all0 = 0, all1 = 0;
-    for (int k = 0; k < 16; k++) {
-      if (k < w) {
-        r0 += wsum[0][k];
-        r1 += wsum[1][k];
-      }
-      all0 += wsum[0][k];
-      all1 += wsum[1][k];
-    }
-    r0 += ex0;
-    r1 += ex1;
-#pragma unroll
-    for (int q = 0; q < PER; q++) {
-      const int i = base + t * PER + q;
-      if (i < nl) {
-        scan[i] = r0;
-        scan[(size_t)cap + i] = r1;
-      }
-      r0 += v0[q];
-      r1 += v1[q];
-    }
-    __syncthreads();
-    if (t == 0) {
-      carry[0] += all0;
-      carry[1] += all1;
-    }
-    __syncthreads();
-  }
-  if (t == 0) {
-    const int total = carry[0], leaves = carry[1];
-    st->cls = ls;
-    st->cle = le;
-    st->cbase = st->nleaf;
-    if ((long long)le + total > cap) {
-      st->overflow = 1;
-      st->need = (int)((long long)le + total < 0x7fffffff ? le + total : 0x7fffffff);
-      st->go = 0;
-    } else if (st->nlev >= kMaxTreeLevels) {
-      st->overflow = 2;
-      st->go = 0;
-    } else {
-      st->go = 1;
-      st->nleaf += leaves;
-      st->nlev += 1;
-      st->level_start[st->nlev] = le;
-      if (total == 0) {
-        st->done = 1;
-      } else {
-        st->ls = le;
-        st->le = le + total;
-      }
-    }
-    if (report) *report = *st;
-  }
-}
-
-// The children of the level the scan kernel set up (cls, cle), and its leaves
-// appended to leaf_ids from cbase, in cell order.
-__global__ __launch_bounds__(256) void k_children(CellsDev c, const TreeState *__restrict__ st,
-                                                  int cap, const int *__restrict__ offs,
-                                                  const int *__restrict__ scan,
-                                                  const TreeParams *__restrict__ tp,
-                                                  int *__restrict__ leaf_ids) {
-#pragma clang fp contract(off)
-  if (!st->go) return;
-  const int ls = st->cls, le = st->cle, leaf_base = st->cbase, nl = le - ls;
-  for (int k = blockIdx.x * 256 + (int)threadIdx.x; k < nl; k += gridDim.x * 256) {
-    const int ci = ls + k;
-    const int nc = c.nchild[ci];
-    if (nc == 0) {
-      leaf_ids[leaf_base + scan[cap + k]] = ci;
-      continue;
-    }
-    const int first = le + scan[k];
-    c.child[ci] = first;
-    const int level = c.level[ci];
-    const int end = c.body[ci] + c.nbody[ci];
-    // R0 2^-(level+1), from the parent's radius (exact: a power-of-two scaling),
-    // so that the roots of a forest may each have their own R0
-    const double r = ldexp(c.Rg[ci], -1);
-    (void)tp;
-    int jc = 0;
-    for (int i = 0; i < 8; i++) {
-      const int o = offs[8 * k + i];
-      const int e = (i < 7) ? offs[8 * k + i + 1] : end;
-      const int size = e - o;
-      if (!size) continue;
-      const int cc = first + jc;
-      for (int d = 0; d < 3; d++)
-        c.Xg[3 * cc + d] = c.Xg[3 * ci + d] + r * (((i >> d) & 1) * 2 - 1);
+    const int cc = first + rank;
+    if (sz != 0 && cc < cap) {
+      // R0 2^-(level+1), from the parent's radius (exact: a power-of-two scaling),
+      // so that the roots of a forest may each have their own R0
+      const double r = ldexp(c.Rg[ci], -1);
+      for (int d = 0; d < 3; d++) c.Xg[3 * cc + d] = X[d] + r * (((j >> d) & 1) * 2 - 1);
       c.Rg[cc] = r;
-      c.level[cc] = level + 1;
+      c.level[cc] = c.level[ci] + 1;
       c.parent[cc] = ci;
       c.body[cc] = o;
-      c.nbody[cc] = size;
+      c.nbody[cc] = sz;
       c.nchild[cc] = 0;
       c.child[cc] = -1;
-      jc++;
     }
+    if (ntiles <= (int)gridDim.x) return;  // a tile a block
+    __syncthreads();                       // s_tile, s_before are written again
   }
 }
 
-int launch_tree_level(CellsDev c, BodiesDev b, TreeState *st, int ncrit, int cap, int *offs,
-                      int *nch, int *scan, const TreeParams *d_tp, int *leaf_ids,
+int launch_tree_level(CellsDev c, BodiesDev b, TreeState *st, int par, unsigned tag,
+                      unsigned long long *words, int nblocks, int ncrit, int cap, int *leaf_ids,
                       TreeState *report, hipStream_t s) {
-  // grids cover the widest levels in a few sweeps; narrow levels leave most
-  // blocks idle for a few microseconds
-  hipLaunchKernelGGL(k_split, dim3(512), dim3(256), 0, s, c, b, (const TreeState *)st, ncrit, cap,
-                     offs, nch);
-  hipLaunchKernelGGL(k_level_scan, dim3(1), dim3(1024), 0, s, (const int *)nch, scan, st, cap,
-                     report);
-  hipLaunchKernelGGL(k_children, dim3(256), dim3(256), 0, s, c, (const TreeState *)st, cap,
-                     (const int *)offs, (const int *)scan, d_tp, leaf_ids);
+  hipLaunchKernelGGL(k_tree_level, dim3(nblocks), dim3(kTreeThreads), 0, s, c, b, st, par, tag,
+                     words, ncrit, cap, leaf_ids, report);
   return 0;
 }
 
@@ -592,9 +594,9 @@ int launch_tree_level(CellsDev c, BodiesDev b, TreeState *st, int ncrit, int cap
 //    equal 52-bit prefixes (bodies closer than 2^-17 of the box; rare)
 //    reordered by (high key, low key, index);
 //  * the gather (k_gather);
-//  * levels split as k_split does (eight lanes per cell: a count per octant up
+//  * levels split as k_tree_level does (eight lanes per cell: a count per octant up
 //    to 32 bodies, else the search for the start of octants >= j that never
-//    tests the cell's first body), children placed as k_children does, with
+//    tests the cell's first body), children placed as it does, with
 //    the positions read from LDS.
 // It marks the last body of every leaf in lend (cleared first) and counts
 // the leaves: out[0] = leaves, out[1] = 0, or 2 when the tree would need more
@@ -1234,81 +1236,6 @@ __device__ __forceinline__ int trav_classify(const CellsDev &c, const MacArgs &a
   return 4;
 }
 
-// Exclusive scan of three ints over a block of NW waves; totals to *tot.
-template <int NW>
-__device__ __forceinline__ int3 block_excl_scan3_n(int3 v, int3 *tot) {
-  __shared__ int3 wsum[NW];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  int tx, ty, tz;
-  int ex = wave_excl_scan(v.x, &tx), ey = wave_excl_scan(v.y, &ty), ez = wave_excl_scan(v.z, &tz);
-  if (lane == 0) wsum[w] = make_int3(tx, ty, tz);
-  __syncthreads();
-  int3 base = make_int3(0, 0, 0), all = make_int3(0, 0, 0);
-  for (int k = 0; k < NW; k++) {
-    int3 q = wsum[k];
-    if (k < w) base = make_int3(base.x + q.x, base.y + q.y, base.z + q.z);
-    all = make_int3(all.x + q.x, all.y + q.y, all.z + q.z);
-  }
-  *tot = all;
-  __syncthreads();
-  return make_int3(base.x + ex, base.y + ey, base.z + ez);
-}
-
-__device__ __forceinline__ int wave_sum_i(int v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-  return v;
-}
-
-// A block's words for the scan over the blocks: its own three counts and,
-// later, the sums up to and with it.  A word is the value and, above
-// kTravTagShift, the step's tag: words of other steps read as not there yet, so
-// nothing is cleared between steps, and value and tag arrive together (one
-// 64-bit store), so no ordering is needed between the words.
-constexpr int kTravTagShift = 36;
-__device__ __forceinline__ void trav_put(unsigned long long *w, int v, unsigned tag) {
-  __hip_atomic_store(w, (unsigned long long)(unsigned)v | (unsigned long long)tag << kTravTagShift,
-                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ unsigned long long trav_get(const unsigned long long *w) {
-  return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Sums of the counts of the ranges before `range`, by one wave: 64 ranges at a
-// time, nearest first, until one whose sums are known.  Ranges are numbered in
-// the order in which blocks start on them, and a range's counts are stored
-// before its block waits for anything, so every word looked for here arrives.
-__device__ __forceinline__ int3 trav_look_back(const unsigned long long *words, int range,
-                                               unsigned tag) {
-  const int lane = threadIdx.x & (kWave - 1);
-  int3 sum = make_int3(0, 0, 0);
-  for (int last = range - 1; last >= 0;) {
-    const int k = last - lane;
-    unsigned long long w[6] = {0, 0, 0, 0, 0, 0};
-    if (k >= 0)
-      for (int q = 0; q < 6; q++) w[q] = trav_get(words + 6 * k + q);
-    auto here = [&](int q) { return (unsigned)(w[q] >> kTravTagShift) == tag; };
-    const bool counts = here(0) && here(1) && here(2), sums = here(3) && here(4) && here(5);
-    const unsigned long long known = __ballot(k >= 0 && sums);
-    const unsigned long long ready = __ballot(k < 0 || sums || counts);
-    const int stop = known ? __ffsll(known) - 1 : kWave;  // lanes before it add their counts
-    const unsigned long long need = stop < kWave ? (1ull << stop) - 1 : ~0ull;
-    if ((ready & need) != need) {
-      __builtin_amdgcn_s_sleep(1);
-      continue;
-    }
-    int3 v = make_int3(0, 0, 0);
-    if (k >= 0 && lane < stop) v = make_int3((int)(unsigned)w[0], (int)(unsigned)w[1],
-                                             (int)(unsigned)w[2]);
-    if (k >= 0 && lane == stop) v = make_int3((int)(unsigned)w[3], (int)(unsigned)w[4],
-                                              (int)(unsigned)w[5]);
-    sum = make_int3(sum.x + wave_sum_i(v.x), sum.y + wave_sum_i(v.y), sum.z + wave_sum_i(v.z));
-    if (known) break;
-    last -= kWave;
-  }
-  return sum;
-}
-
 // One step.  The frontier size, list lengths and the counter of ranges taken
 // live in TravState, two of each by step parity: this step reads its own and
 // the block of its last range sets the next step's.  A range is as many whole
@@ -1363,16 +1290,16 @@ __global__ __launch_bounds__(kTravThreads) void k_trav_step(
   if (t < kWave) {
     unsigned long long *w = words + 6 * range;
     if (t == 0) {
-      trav_put(w, tot.x, tag);
-      trav_put(w + 1, tot.y, tag);
-      trav_put(w + 2, tot.z, tag);
+      scan_put(w, tot.x, tag);
+      scan_put(w + 1, tot.y, tag);
+      scan_put(w + 2, tot.z, tag);
     }
-    const int3 before = trav_look_back(words, range, tag);
+    const int3 before = look_back(words, range, tag);
     if (t == 0) {
       const int3 s = make_int3(before.x + tot.x, before.y + tot.y, before.z + tot.z);
-      trav_put(w + 3, s.x, tag);
-      trav_put(w + 4, s.y, tag);
-      trav_put(w + 5, s.z, tag);
+      scan_put(w + 3, s.x, tag);
+      scan_put(w + 4, s.y, tag);
+      scan_put(w + 5, s.z, tag);
       s_before = before;
       if (range == nranges - 1) {
         const long long nm = (long long)bm + s.x, np = (long long)bp + s.y, big = 0x7fffffff;
