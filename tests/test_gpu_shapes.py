@@ -1,0 +1,120 @@
+"""The sizes at which the kernels' shapes change: the slabs of the small all-pairs
+evaluation, four-wave M2L blocks with idle waves, and evaluations that follow
+others on one context (which write their arrays instead of clearing them).
+
+Tolerances (FP64): the all-pairs sums differ from the reference sum in their
+order only, n terms of relative round-off 2^-53 each against the sum of their
+magnitudes; the FMM against the oracle as in test_gpu_parity."""
+import numpy as np
+import pytest
+
+from conftest import relerr_vec
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch_cuda():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return torch
+
+
+def _flags(n, seed, sinks, sources):
+    rng = np.random.default_rng(seed)
+    return ((rng.random(n) < sinks) | ((rng.random(n) < sources).astype(np.uint8) << 1)
+            ).astype(np.uint8)
+
+
+def _eval(torch, f, x, v, m, flags=None):
+    d = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (x, v, m)]
+    fl = None if flags is None else torch.from_numpy(flags).cuda()
+    out = f.eval(*d, flags=fl)
+    torch.cuda.synchronize()
+    return [t.cpu().numpy() for t in out]
+
+
+def _direct(x, v, m, flags):
+    """Sums and sums of magnitudes over all pairs, one target at a time."""
+    n = m.size
+    q = m * ((flags >> 1) & 1)
+    out, mag = [], []
+    for a in (np.zeros(n), np.zeros((n, 3)), np.zeros((n, 3))):
+        out.append(a)
+        mag.append(np.zeros(n))
+    for i in range(n):
+        if not flags[i] & 1:
+            continue
+        d, w = x - x[i], v - v[i]
+        r2 = (d * d).sum(1)
+        ri = np.where(r2 > 0, 1.0 / np.sqrt(np.where(r2 > 0, r2, 1.0)), 0.0)
+        f = q * ri ** 3
+        k = 3.0 * f * (d * w).sum(1) * ri * ri
+        out[0][i], mag[0][i] = (q * ri).sum(), (q * ri).sum()
+        out[1][i], mag[1][i] = (f[:, None] * d).sum(0), (f * np.sqrt(r2)).sum()
+        out[2][i] = (f[:, None] * w - k[:, None] * d).sum(0)
+        mag[2][i] = (f * np.linalg.norm(w, axis=1) + np.abs(k) * np.sqrt(r2)).sum()
+    return out, mag
+
+
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 255, 256, 257, 1009, 8192, 8193])
+@pytest.mark.parametrize("masked", [False, True])
+def test_gpu_small_direct_slabs(torch_cuda, n, masked):
+    import taichi_collisional_amd as tca
+    from taichi_collisional_amd import ics
+    x, v, m = ics.plummer(n, seed=n)
+    if n > 2:
+        x[n // 2] = x[0]  # a coincident pair does not interact
+    flags = _flags(n, n, 0.7, 0.8) if masked else np.full(n, 3, np.uint8)
+    got = _eval(torch_cuda, tca.Fmm(p=4, direct_below=10 ** 6), x, v, m,
+                flags if masked else None)
+    want, mag = _direct(x, v, m, flags)
+    # a pair's own term: some ten roundings; then n additions of partial sums
+    tol = (10 + n) * 2.0 ** -53
+    for g, w, a in zip(got, want, mag):
+        err = np.abs(g - w) if g.ndim == 1 else np.linalg.norm(g - w, axis=1)
+        assert np.all(err <= 4 * tol * a), float(np.max(err / np.maximum(a, 1e-300)))
+
+
+@pytest.mark.parametrize("p", [13, 14, 15, 19, 20])
+def test_gpu_m2l_blocks_with_idle_waves(torch_cuda, oracle_lib, p):
+    """One body in forty takes a force: most targets have no sink, so the
+    four-wave blocks of orders 14 and up hold waves that write nothing, and the
+    last block is not full."""
+    import taichi_collisional_amd as tca
+    from taichi_collisional_amd import ics
+    n, u = 4001, [0.2, -0.3, 0.1]
+    x, v, m = ics.plummer(n, seed=p)
+    flags = _flags(n, p, 0.025, 0.9)
+    f = tca.Fmm(p=p, ncrit=32, theta=0.6, direct_below=0)
+    f.set_shift(u)
+    gp, ga, gj = _eval(torch_cuda, f, x, v, m, flags)
+    o = oracle_lib.Oracle(p, ncrit=32, theta=0.6, shift_frac=u)
+    op, oa, oj, _ = o.eval(x, v, m, issink=flags & 1, issource=(flags >> 1) & 1)
+    on = (flags & 1) == 1
+    assert relerr_vec(ga[on], oa[on])[1] < 1e-10
+    assert relerr_vec(gj[on], oj[on])[1] < 1e-9
+    assert not gp[~on].any() and not ga[~on].any() and not gj[~on].any()
+
+
+@pytest.mark.parametrize("mac", [0, 1])
+def test_gpu_nothing_left_from_the_evaluation_before(torch_cuda, mac):
+    """A context's second evaluation (fewer bodies, other masks) equals a fresh
+    context's: the rows, results and flags that it does not clear are written."""
+    import taichi_collisional_amd as tca
+    from taichi_collisional_amd import ics
+
+    def ctx():
+        f = tca.Fmm(p=6, ncrit=24, theta=0.5, mac=mac, direct_below=0)
+        f.set_shift([0.1, 0.2, -0.3])
+        return f
+
+    f = ctx()
+    _eval(torch_cuda, f, *ics.plummer(20000, seed=1))
+    x, v, m = ics.dehnen(9001, seed=2)
+    flags = _flags(9001, 3, 0.3, 0.6)
+    again, fresh = _eval(torch_cuda, f, x, v, m, flags), _eval(torch_cuda, ctx(), x, v, m, flags)
+    # the same lists and sums; the atomics' order is the only difference
+    for g, w in zip(again, fresh):
+        assert np.max(np.abs(g - w)) <= 1e-12 * np.max(np.abs(w))
