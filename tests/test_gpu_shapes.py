@@ -118,3 +118,43 @@ def test_gpu_nothing_left_from_the_evaluation_before(torch_cuda, mac):
     # the same lists and sums; the atomics' order is the only difference
     for g, w in zip(again, fresh):
         assert np.max(np.abs(g - w)) <= 1e-12 * np.max(np.abs(w))
+
+
+@pytest.mark.parametrize("ncand", [1, 2, 5, 21, 33, 64])
+def test_gpu_leaf_choice(torch_cuda, ncand):
+    """A wave holds 64, 32, 12, 3, 1 and 1 leaves: every leaf gets the cheapest
+    candidate predicted to meet the target, and where none does the first one (in
+    32 bits the key 1e30 + error is 1e30 for all of them)."""
+    import mlp_oracle as mo
+    import taichi_collisional_amd as tca
+    from taichi_collisional_amd import ics
+    rng = np.random.default_rng(ncand)
+    P = (mo.init_params(1) + rng.normal(scale=0.05, size=mo.NPARAM)).astype(np.float32)
+    q = rng.integers(2, 7, ncand)
+    theta = np.linspace(0.3, 0.9, ncand).astype(np.float32)
+    cost = rng.permutation(ncand).astype(np.float32) + 1
+
+    def run(target):
+        f = tca.Fmm(p=6, ncrit=16, theta=0.5, direct_below=0)
+        f.set_shift([0.1, 0.2, -0.3])
+        f.set_order_model(P, q, theta, cost, [-10] * 9, [10] * 9, target)
+        f.set_adaptive(2)
+        _eval(torch_cuda, f, *ics.plummer(3001, seed=7))
+        feat, _, pred = f.leaf_data()
+        return feat.cpu().numpy().clip(-10, 10), pred.cpu().numpy()
+
+    feat, _ = run(1.0)
+    nl = len(feat)
+    X = np.empty((nl, ncand, mo.NIN))
+    X[..., :9] = feat[:, None]
+    X[..., 9] = q / 20.0
+    X[..., 10] = theta
+    y = mo.forward(P.astype(np.float64), X.reshape(-1, mo.NIN)).reshape(nl, ncand)
+    tol = 1e-4 * max(1.0, np.max(np.abs(y)))  # the network's, as for its own kernel
+    for level in (y.min() - 1, np.median(y), y.max() + 1):
+        _, pred = run(10.0 ** level)
+        key = np.where(y <= level, cost, 1e30)
+        want = y[np.arange(nl), key.argmin(1)]
+        clear = np.all(np.abs(y - level) > 2 * tol, axis=1)
+        assert clear.sum() >= nl // 4
+        assert np.all(np.abs(pred - want)[clear] <= tol)
