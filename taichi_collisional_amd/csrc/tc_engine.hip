@@ -78,11 +78,14 @@ static int ensure_cells(tc_context *ctx, int nc, int keep) {
   return 0;
 }
 
-// The scan words of tree levels and walk steps: cleared when they are new or
-// the tags run out, so that no launch finds its own tag there (a tag per
-// launch, fewer than 2^20 between two calls).
-static int scan_words(tc_context *ctx, size_t words) {
-  const size_t bytes = sizeof(unsigned long long) * words;
+// The scan words of tree levels (of cells cells at most) and walk steps, one
+// size for both: a walk that outgrew the tree's would free them, and that waits
+// for the moments on the other stream (a first error-MAC evaluation, N =
+// 300,007: 1 ms).  Cleared when they are new or the tags run out, so that no
+// launch finds its own tag there (a tag per launch, fewer than 2^20 between two
+// calls).
+static int scan_words(tc_context *ctx, size_t cells) {
+  const size_t bytes = sizeof(unsigned long long) * std::max(tree_words(cells), kTravWords);
   if (ctx->twords.bytes < bytes || ctx->scan_tag > (1u << 27)) {
     TC_CHECK(ctx->twords.ensure(bytes));
     TC_CHECK(hipMemsetAsync(ctx->twords.p, 0, ctx->twords.bytes, ctx->stream));
@@ -118,7 +121,7 @@ static int build_tree(tc_context *ctx, int n) {
       return -3;
     }
     const int cap = ctx->cap_c;
-    if (int e = scan_words(ctx, tree_words((size_t)cap))) return e;
+    if (int e = scan_words(ctx, (size_t)cap)) return e;
     // two blocks a CU; a small system's levels are a cell per thousand bodies
     const int nblocks = std::min(512, std::max(8, n / 512));
     // one root, or one per cluster of a forest
@@ -269,7 +272,7 @@ static int traverse(tc_context *ctx, int n, const MacArgs &mac) {
     const long long cm = cap(ctx->m2l), cp = cap(ctx->p2p),
                     cf = std::min({cap(ctx->front_a), cap(ctx->front_b),
                                    (long long)std::min<size_t>(ctx->tcls.bytes, 0x7fffffff)});
-    if (int e = scan_words(ctx, kTravWords)) return e;
+    if (int e = scan_words(ctx, (size_t)ctx->cap_c)) return e;
     // a small system's frontiers are a few pairs per body
     const int nblocks = std::min(kTravBlocks, std::max(64, n / 32));
     launch_root_pairs(ctx->front_a.as<int2>(), ctx->ncl, ctx->tstate.as<TravState>(), s);
