@@ -720,6 +720,13 @@ static int eval_device(tc_context *ctx, int n, const double *x, const double *v,
     ctx->err = "n must be positive";
     return -1;
   }
+  // before the draws below, so that a call that finds no memory takes none
+  // (all pairs need only the slabs' partial sums)
+  const bool direct = cfg.direct_below > 0 && n < cfg.direct_below && ctx->ncl == 1;
+  if (direct)
+    TC_CHECK(ctx->mdpart.ensure(sizeof(double) * 7 * (size_t)direct_eval_slabs(n) * n));
+  else if (int e = ensure_bodies(ctx, n))
+    return e;
   // root-shift values: three drand48() per evaluation, as getBounds draws them
   // (a forest: three per cluster, in cluster order)
   double u[3];
@@ -742,16 +749,14 @@ static int eval_device(tc_context *ctx, int n, const double *x, const double *v,
   std::memcpy(ctx->shift, u, sizeof(u));
   TC_CHECK(hipEventRecord(ctx->ev[0], s));
 
-  if (cfg.direct_below > 0 && n < cfg.direct_below && ctx->ncl == 1) {
+  if (direct) {
     // all-pairs sum in the caller's order (direct(), traverse_eager.h:295-304)
-    TC_CHECK(ctx->mdpart.ensure(sizeof(double) * 7 * (size_t)direct_eval_slabs(n) * n));
     launch_direct_eval(x, v, m, flags, n, ctx->mdpart.as<double>(), pot, acc, jerk, s);
     TC_CHECK(spin_wait(ctx, s));
     TC_CHECK(hipGetLastError());
     return 0;
   }
 
-  if (int e = ensure_bodies(ctx, n)) return e;
   // ---- tree
   if (int e = sort_and_build(ctx, n, x, v, m, flags)) return e;
   const bool err_mac = cfg.mac == TC_MAC_ERROR;
