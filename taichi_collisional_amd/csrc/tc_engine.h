@@ -105,6 +105,7 @@ struct tc_context {
   int p2p_per_lane = 1;
   P2PSplit p2p_split;
   bool p2p_ready = false;  // the last evaluation's near-field inputs are in place
+  bool tree_ready = false;  // the last evaluation's tree is in place
   double shift[3] = {0, 0, 0};
   // bodies
   int cap_n = 0;

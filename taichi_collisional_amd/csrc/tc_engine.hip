@@ -158,6 +158,7 @@ static int build_tree(tc_context *ctx, int n) {
   ctx->st.depth = depth;
   ctx->st.nlevels = (int)ctx->level_start.size() - 1;
   ctx->nleaves = nleaf;
+  ctx->tree_ready = true;
   ctx->st.nleaves = nleaf;
   // leaf ids and body counts for the host-built P2P work items: copied now,
   // read after ev[11] (build_p2p_items, while the GPU runs M2L)
@@ -714,7 +715,7 @@ static int eval_device(tc_context *ctx, int n, const double *x, const double *v,
   std::memset(&ctx->st, 0, sizeof(ctx->st));
   std::memset(ctx->m2l_by_order, 0, sizeof(ctx->m2l_by_order));
   ctx->has_acc_old = false;
-  ctx->p2p_ready = false;
+  ctx->p2p_ready = ctx->tree_ready = false;
   ctx->last_n = n;
   if (n <= 0) {
     ctx->err = "n must be positive";
@@ -1021,6 +1022,7 @@ int master_eval_device(tc_context *ctx, int n, const double *x, const double *v,
   std::memset(&ctx->st, 0, sizeof(ctx->st));
   std::memset(ctx->m2l_by_order, 0, sizeof(ctx->m2l_by_order));
   ctx->has_acc_old = false;
+  ctx->p2p_ready = ctx->tree_ready = false;  // the bodies and the tree are replaced
   ctx->last_n = n;
   const bool steps = mode & TC_MASTER_STEPS, pair_mass = mode & TC_MASTER_PAIR_MASS;
   if (n <= 0 || !x || !v || !m || !pot || !acc) {
@@ -1139,6 +1141,7 @@ int eval_soa_device(tc_context *ctx, int n, const double *x, const double *v, co
 }
 
 int master_direct_prepare(tc_context *ctx, int n, int ns) {
+  ctx->p2p_ready = ctx->tree_ready = false;
   if (int e = ensure_bodies(ctx, n)) return e;
   TC_CHECK(ctx->mlend.ensure((size_t)n));
   const int nslab = std::max(master_direct_slabs(n, n), master_direct_slabs(ns, n));
@@ -1495,7 +1498,7 @@ int tc_leaf_count(const tc_context *ctx) { return ctx ? ctx->nleaves : -1; }
 
 int tc_leaf_data(tc_context *ctx, float *features, int *leaf_of_body, float *pred) {
   if (!ctx) return -1;
-  if (ctx->adaptive == 0 || ctx->last_n <= 0) {
+  if (ctx->adaptive == 0 || !ctx->tree_ready) {
     ctx->err = "tc_leaf_data: the last evaluation did not choose per-cell orders";
     return -2;
   }
@@ -1516,8 +1519,8 @@ int tc_leaf_data(tc_context *ctx, float *features, int *leaf_of_body, float *pre
 
 int tc_leaf_errors(tc_context *ctx, const double *acc, const double *acc_ref, float *out) {
   if (!ctx || !acc || !acc_ref || !out) return -1;
-  if (ctx->last_n <= 0 || ctx->nleaves <= 0) {
-    ctx->err = "tc_leaf_errors: no tree (evaluate first)";
+  if (!ctx->tree_ready) {
+    ctx->err = "tc_leaf_errors: no tree (the last evaluation built none)";
     return -2;
   }
   launch_leaf_errors(cells_of(ctx), bodies_of(ctx), ctx->leaf_ids.as<int>(), ctx->nleaves, acc,

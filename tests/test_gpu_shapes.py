@@ -158,3 +158,38 @@ def test_gpu_leaf_choice(torch_cuda, ncand):
         clear = np.all(np.abs(y - level) > 2 * tol, axis=1)
         assert clear.sum() >= nl // 4
         assert np.all(np.abs(pred - want)[clear] <= tol)
+
+
+def test_gpu_leaf_calls_need_the_last_evaluations_tree(torch_cuda):
+    """After an evaluation without a tree (all pairs) or with another one (the
+    master sum's), the leaf calls and the tuner refuse: the leaves of the tree
+    before it index bodies that the smaller system does not have."""
+    import taichi_collisional_amd as tca
+    from taichi_collisional_amd import ics
+    torch = torch_cuda
+    f = tca.Fmm(p=4, ncrit=32, theta=0.6, direct_below=1000)
+    f.set_adaptive(1, 4, 0.6)
+    big, small = ics.plummer(5000, seed=3), ics.plummer(300, seed=4)
+
+    def refused(n):
+        a = torch.ones(n, 3, dtype=torch.float64, device="cuda")
+        for call in (f.leaf_data, lambda: f.leaf_errors(a, a), f.tune_p2p):
+            with pytest.raises(RuntimeError):
+                call()
+
+    def tree():  # (the master sum takes the shift back to zero)
+        f.set_shift([0.1, 0.2, -0.3])
+        _eval(torch, f, *big)
+
+    tree()
+    feat, lob, _ = f.leaf_data()
+    assert feat.shape[0] == f.stats()["nleaves"] and int(lob.max()) == feat.shape[0] - 1
+    _eval(torch, f, *small)
+    refused(300)
+    tree()
+    d = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in small]
+    f.master_eval(*d, get_steps=True)
+    refused(300)
+    tree()
+    assert f.leaf_errors(*[torch.ones(5000, 3, dtype=torch.float64, device="cuda")] * 2).shape
+    assert torch.equal(f.leaf_data()[1], lob)
