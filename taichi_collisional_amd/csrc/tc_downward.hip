@@ -16,7 +16,8 @@
 //         blocks waited for P2P's last blocks (at N = 2^20 the pass ended
 //         1.4 ms after P2P; now it ends 4 ms before P2P does).
 //       * 512 threads per child, two per output, on levels of at most 1,024
-//         cells where P2P is short: a level 35 -> 13 us at p = 12.
+//         cells where P2P is short: a level 35 -> 13 us at p = 12; and above
+//         p = 13 everywhere.
 //   L2P (kernel_fast_lean.h:1060-1128): two leaves per wave, 32 lanes each
 //       (leaves average ~19 bodies: one leaf per wave left 70% of the lanes
 //       idle); lane = body, Y = Y(X_c - x_b) and
@@ -258,13 +259,15 @@ static void l2p_go(CellsDev c, BodiesDev b, ResultsDev r, const int *ids, int n,
 }
 
 // Whether a level of `cells` takes 512 threads per cell: up to 1,024 cells
-// (four blocks a CU), and at any size above p = 13, where the tables (48 bytes
-// a coefficient) leave room for few one-wave blocks on a CU (p = 20, N = 2^17:
-// the three widest levels 108, 197, 207 us with one wave per cell, 52, 80, 109
-// with eight).
+// (four blocks a CU) where no long P2P runs beside it, and always above p = 13,
+// where the tables (48 bytes a coefficient) leave room for few one-wave blocks
+// on a CU and for none in a finished P2P wave's slot (13 KB).  One wave / eight
+// waves per cell: p = 20, N = 2^17, the three widest levels 108, 197, 207 / 52,
+// 80, 109 us; evaluations beside a long P2P, N = 2^18 (theta 0.4) p = 13 8.74 /
+// 8.84 ms, 14 10.48 / 10.47, 16 13.04 / 12.89, 20 25.35 / 24.83, 24 41.0 / 39.4.
 template <int P>
-constexpr bool l2l_wide(int cells) {
-  return cells <= 1024 || 48 * nterm(P) > 10 * 1024;
+constexpr bool l2l_wide(int cells, bool beside) {
+  return (cells <= 1024 && !beside) || 48 * nterm(P) > 10 * 1024;
 }
 
 int launch_l2l(int p, CellsDev c, int ls, int le, bool beside, hipStream_t s) {
@@ -273,7 +276,7 @@ int launch_l2l(int p, CellsDev c, int ls, int le, bool beside, hipStream_t s) {
 #define TC_CASE(P)\
   case P:\
     if constexpr (in_shard(P, TC_SHARD)) {\
-      l2l_go<P>(c, nullptr, ls, le - ls, !beside && l2l_wide<P>(le - ls), s);\
+      l2l_go<P>(c, nullptr, ls, le - ls, l2l_wide<P>(le - ls, beside), s);\
       return 0;\
     } else {\
       return -1;\
@@ -291,7 +294,7 @@ int launch_l2l_ids(int p, CellsDev c, const int *ids, int nids, hipStream_t s) {
 #define TC_CASE(P)\
   case P:\
     if constexpr (in_shard(P, TC_SHARD)) {\
-      l2l_go<P>(c, ids, 0, 8 * nids, l2l_wide<P>(8 * nids), s);\
+      l2l_go<P>(c, ids, 0, 8 * nids, l2l_wide<P>(8 * nids, false), s);\
       return 0;\
     } else {\
       return -1;\
