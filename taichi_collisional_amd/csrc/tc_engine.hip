@@ -346,9 +346,9 @@ static int build_csr(tc_context *ctx, const int2 *pairs, int npairs, DBuf &cnt, 
 static int build_p2p_items(tc_context *ctx);
 
 // The near field on near_stream, queued after the P2P list's grouping: ranges
-// and cleared results, work items (built on the host once the list's lengths
-// are there), P2P.  after (or null): an event that P2P waits for.
-static int near_field(tc_context *ctx, int n, hipEvent_t after) {
+// and cleared results, work items (built on the host while the GPU runs M2L),
+// and after M2L (ev[5]) P2P.
+static int near_field(tc_context *ctx, int n) {
   hipStream_t s2 = ctx->near_stream;
   const ResultsDev r = results_of(ctx);
   TC_CHECK(ctx->p2p_ranges.ensure(sizeof(int2) * (size_t)std::max<long long>(ctx->st.n_p2p_cells, 1)));
@@ -356,7 +356,7 @@ static int near_field(tc_context *ctx, int n, hipEvent_t after) {
   launch_p2p_setup(cells_of(ctx), ctx->p2p_src.as<int>(), (int)ctx->st.n_p2p_cells,
                    ctx->p2p_ranges.as<int2>(), r, n, ctx->npairs.as<unsigned long long>(), s2);
   if (int e = build_p2p_items(ctx)) return e;
-  if (after) TC_CHECK(hipStreamWaitEvent(s2, after, 0));
+  TC_CHECK(hipStreamWaitEvent(s2, ctx->ev[5], 0));
   TC_CHECK(hipEventRecord(ctx->ev[9], s2));
   launch_p2p(cells_of(ctx), bodies_of(ctx), r, ctx->p2p_items.as<int4>(), (int)ctx->n_items,
              ctx->p2p_off.as<int>(), ctx->p2p_cnt.as<int>(), ctx->p2p_ranges.as<int2>(),
@@ -367,8 +367,7 @@ static int near_field(tc_context *ctx, int n, hipEvent_t after) {
   return 0;
 }
 
-// near: also queue the near field (n bodies) as soon as its list is grouped
-static int build_lists(tc_context *ctx, int &nchunks, bool near = false, int n = 0) {
+static int build_lists(tc_context *ctx, int &nchunks) {
   hipStream_t s = ctx->stream;
   int nc = ctx->st.ncells;
   // the P2P list on near_stream meanwhile (after the walk that wrote it), with
@@ -391,10 +390,7 @@ static int build_lists(tc_context *ctx, int &nchunks, bool near = false, int n =
     return -4;
   TC_CHECK(hipMemcpyAsync(ctx->h_pin + 10, ctx->m2l_coff.as<int>() + nc, sizeof(int),
                           hipMemcpyDeviceToHost, s));
-  TC_CHECK(hipEventRecord(ctx->ev_wait, s));
-  if (near)
-    if (int e = near_field(ctx, n, nullptr)) return e;
-  TC_CHECK(spin_event(ctx->ev_wait));
+  TC_CHECK(spin_wait(ctx, s));
   nchunks = ctx->h_pin[10];
   TC_CHECK(ctx->m2l_chunks.ensure(sizeof(int4) * (size_t)std::max(nchunks, 1)));
   launch_make_chunks(ctx->m2l_off.as<int>(), ctx->m2l_cnt.as<int>(), ctx->m2l_coff.as<int>(), nc,
@@ -407,7 +403,7 @@ static int build_lists(tc_context *ctx, int &nchunks, bool near = false, int n =
 // Each leaf is cut into target groups of <= 64 bodies by the lane model of
 // the kernel (P2PSplit).  The per-leaf list lengths were copied to pinned
 // memory on near_stream, where the upload is queued too; the host loop runs
-// while the GPU groups the M2L list or runs M2L.
+// while the GPU runs M2L.
 static int build_p2p_items(tc_context *ctx) {
   // Slices so that even a small system's list makes thousands of items: a
   // wave's time is its chain of tiles, and two or three waves a SIMD leave the
@@ -791,13 +787,8 @@ static int eval_device(tc_context *ctx, int n, const double *x, const double *v,
     if (int e = traverse(ctx, n, mac_args(ctx, err_mac ? kMacError : kMacTheta))) return e;
   }
   TC_CHECK(hipEventRecord(ctx->ev[3], s));
-  // P2P takes about 1 ms per million list entries.  A short one runs as soon as
-  // its list is there, beside the M2L list's grouping, whose small sorts leave
-  // the chip idle, and is out of the way of the downward pass; a long one runs
-  // after M2L and hides the downward pass.
-  const bool near_late = ctx->st.n_p2p_cells > 1000000;
   int nchunks = 0;
-  if (int e = build_lists(ctx, nchunks, !near_late, n)) return e;
+  if (int e = build_lists(ctx, nchunks)) return e;
   if (!err_mac) TC_CHECK(hipStreamWaitEvent(s, ctx->ev[13], 0));  // the moments
   TC_CHECK(hipEventRecord(ctx->ev[4], s));
   // ---- far field
@@ -822,16 +813,24 @@ static int eval_device(tc_context *ctx, int n, const double *x, const double *v,
     ctx->m2l_by_order[cfg.p] = ctx->st.n_m2l;
   }
   TC_CHECK(hipEventRecord(ctx->ev[5], s));
-  // the GPU runs M2L while the host builds the P2P work items
-  if (near_late)
-    if (int e = near_field(ctx, n, ctx->ev[5])) return e;
+  // P2P, after M2L and alongside the downward pass.  (A short P2P queued before
+  // M2L, beside the list's grouping, is no faster, as the host then builds its
+  // items before it queues M2L: N = 10,007 1.23 ms against 1.22, N = 131,072,
+  // p = 8 2.39 against 2.30, N = 65,536, p = 20 4.83 against 4.63; and a first
+  // evaluation waits for the items' allocations.)
+  if (int e = near_field(ctx, n)) return e;
+  // Beside a long P2P the wide blocks of L2L wait for its waves to drain.
+  // Evaluation, one-wave / wide L2L: 143 K list entries 1.30 / 1.29 ms, 165 K
+  // 1.58 / 1.49, 305 K 1.92 / 1.88 (p = 12), 207 K 1.49 / 1.49, 281 K 1.71 /
+  // 1.75, 457 K 2.27 / 2.30, 644 K 2.76 / 2.79
+  const bool long_p2p = ctx->st.n_p2p_cells > (1 << 18);
   // ---- downward into the far-field result set
   ResultsDev rf = {ctx->fpot.as<double>(), ctx->fax.as<double>(), ctx->fay.as<double>(),
                    ctx->faz.as<double>(), ctx->fjx.as<double>(), ctx->fjy.as<double>(),
                    ctx->fjz.as<double>()};
   int L = (int)ctx->level_start.size() - 1;
   for (int l = 1; l < L; l++)
-    launch_l2l(cfg.p, cells_of(ctx), ctx->level_start[l], ctx->level_start[l + 1], near_late, s);
+    launch_l2l(cfg.p, cells_of(ctx), ctx->level_start[l], ctx->level_start[l + 1], long_p2p, s);
   launch_l2p(cfg.p, cells_of(ctx), bodies_of(ctx), rf, ctx->leaf_ids.as<int>(), ctx->nleaves, s,
              false);
   TC_CHECK(hipEventRecord(ctx->ev[6], s));

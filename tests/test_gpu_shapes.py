@@ -193,3 +193,20 @@ def test_gpu_leaf_calls_need_the_last_evaluations_tree(torch_cuda):
     tree()
     assert f.leaf_errors(*[torch.ones(5000, 3, dtype=torch.float64, device="cuda")] * 2).shape
     assert torch.equal(f.leaf_data()[1], lob)
+
+
+@pytest.mark.parametrize("p", [13, 14])
+def test_gpu_l2l_beside_a_long_p2p(torch_cuda, oracle_lib, p):
+    """Beside a long P2P list L2L takes one wave per child up to order 13 and
+    512 threads above."""
+    import taichi_collisional_amd as tca
+    from taichi_collisional_amd import ics
+    n, u = 9001, [0.2, -0.3, 0.1]
+    x, v, m = ics.plummer(n, seed=p)
+    f = tca.Fmm(p=p, ncrit=5, theta=0.28, direct_below=0)
+    f.set_shift(u)
+    _, ga, gj = _eval(torch_cuda, f, x, v, m)
+    assert f.stats()["n_p2p_cells"] > 1 << 18
+    o = oracle_lib.Oracle(p, ncrit=5, theta=0.28, shift_frac=u)
+    _, oa, oj, _ = o.eval(x, v, m)
+    assert relerr_vec(ga, oa)[1] < 1e-10 and relerr_vec(gj, oj)[1] < 1e-9
