@@ -107,10 +107,11 @@ int tc_set_precision(tc_context *ctx, int p2p_mode, double close_radius);
 /* ---- Launch shape of the near field (no reference counterpart: the
  * reference's P2P, kernel_fast_lean.h:499-699, is a CPU loop over leaf
  * pairs) ----------------------------------------------------------------
- * tile: source bodies per LDS tile (64, 128 or 192); list_slice: the most
- * P2P-list entries per work item (a leaf's list is split into slices that run
- * as separate waves; 1..65535; an evaluation whose whole list is short takes
- * smaller slices, down to 16, to fill the GPU); stage_rounds: the cost of staging one tile, in
+ * tile: source bodies per LDS tile (64, 128 or 192); list_slice: P2P-list
+ * entries per work item (a leaf's list is split into slices that run as
+ * separate waves; 1..65535; as long as no call has set it, an evaluation whose
+ * whole list is short takes fewer than the default 128, down to 16, to fill
+ * the GPU); stage_rounds: the cost of staging one tile, in
  * rounds of pair evaluations, that the cut of each leaf into target groups
  * trades against idle lanes (0 favours groups that fill the wave, larger
  * values fewer groups); targets_per_lane: 1 or 2 (one LDS read of a source
@@ -121,16 +122,21 @@ int tc_set_precision(tc_context *ctx, int p2p_mode, double close_radius);
  * tc_tune_p2p: after an evaluation, time that evaluation's near field under
  * every shape of the grid {1,2} x {64,128,192} x {64,128,256} x {0,2,4,8}
  * (targets per lane x tile x list slice x staging cost), reps launches each,
- * and keep the fastest for the following evaluations; best_ms / default_ms
+ * and keep the fastest for the following evaluations, or the shape set before
+ * the call where none is faster; best_ms / default_ms
  * (may be NULL) receive its time and that of the shape set before the call;
  * grid_ms (NULL or 72 doubles) every shape's time in that nesting order.
- * Returns -1 without a completed tree evaluation. */
+ * Returns -1 without a completed tree evaluation.
+ * tc_p2p_items: the work items of the last near field (the last evaluation's
+ * or the tuner's last) and the list slice that they were cut with (either may
+ * be NULL); -1 without a completed tree evaluation. */
 int tc_set_p2p_shape(tc_context *ctx, int tile, int list_slice, double stage_rounds,
                      int targets_per_lane);
 int tc_get_p2p_shape(tc_context *ctx, int *tile, int *list_slice, double *stage_rounds,
                      int *targets_per_lane);
 int tc_tune_p2p(tc_context *ctx, int reps, double *best_ms, double *default_ms,
                 double *grid_ms);
+int tc_p2p_items(const tc_context *ctx, long long *items, int *list_slice);
 
 /* ---- Per-cell expansion order and opening angle (no reference counterpart;
  * the reference's analogue is its error-controlled walk,

@@ -113,6 +113,7 @@ def lib():
                                        C.POINTER(C.c_double), C.POINTER(C.c_int)]
         L.tc_tune_p2p.argtypes = [vp, C.c_int, C.POINTER(C.c_double), C.POINTER(C.c_double),
                                   C.POINTER(C.c_double)]
+        L.tc_p2p_items.argtypes = [vp, C.POINTER(C.c_longlong), C.POINTER(C.c_int)]
         L.tc_set_adaptive.argtypes = [vp, C.c_int, C.c_int, C.c_double, C.c_double]
         L.tc_eval_clusters.argtypes = [vp, C.c_int, vp, vp, vp, vp, vp, vp, vp, vp]
         L.tc_set_order_model.argtypes = [vp, vp, C.c_int, vp, vp, vp, C.c_int, vp, vp,
@@ -160,7 +161,7 @@ def lib():
 
 EXPORTED_SYMBOLS = ["tc_create", "tc_destroy", "tc_set_seed", "tc_set_shift", "tc_last_shift",
                     "tc_set_precision", "tc_set_p2p_shape", "tc_get_p2p_shape", "tc_tune_p2p",
-                    "tc_set_small_tree",
+                    "tc_p2p_items", "tc_set_small_tree",
                     "tc_eval_clusters", "tc_set_adaptive", "tc_set_order_model", "tc_leaf_count",
                     "tc_leaf_data", "tc_leaf_errors", "tc_m2l_order_counts", "tc_mlp_param_count",
                     "tc_mlp_input_count", "tc_mlp_forward", "tc_mlp_grad", "tc_mlp_adam",
@@ -304,9 +305,10 @@ class Fmm:
 
     def set_p2p_shape(self, tile=128, list_slice=128, stage_rounds=8.0, targets_per_lane=1):
         """Launch shape of the near field (tc_set_p2p_shape): source bodies per
-        LDS tile (64, 128, 192), list entries per work item, the staging cost
-        that sets how leaves are cut into target groups, and targets per lane
-        (1 or 2)."""
+        LDS tile (64, 128, 192), list entries per work item (taken as given;
+        until a call sets it, fewer than 128 where the list is short), the
+        staging cost that sets how leaves are cut into target groups, and
+        targets per lane (1 or 2)."""
         self._check(lib().tc_set_p2p_shape(self.h, int(tile), int(list_slice),
                                            float(stage_rounds), int(targets_per_lane)),
                     "tc_set_p2p_shape")
@@ -322,6 +324,14 @@ class Fmm:
         self._check(lib().tc_get_p2p_shape(self.h, C.byref(t), C.byref(l), C.byref(g),
                                            C.byref(r)), "tc_get_p2p_shape")
         return t.value, l.value, g.value, r.value
+
+    def p2p_items(self):
+        """(work items, list slice they were cut with) of the last evaluation's
+        near field (tc_p2p_items)."""
+        k, l = C.c_longlong(), C.c_int()
+        if lib().tc_p2p_items(self.h, C.byref(k), C.byref(l)) != 0:
+            raise RuntimeError("p2p_items needs a completed tree evaluation")
+        return k.value, l.value
 
     P2P_TUNE_GRID = [(t, l, g, r) for r in (1, 2) for t in (64, 128, 192) for l in (64, 128, 256)
                      for g in (0.0, 2.0, 4.0, 8.0)]

@@ -101,6 +101,7 @@ struct tc_context {
   // the target-group split, and targets per lane (FP64 form)
   int p2p_tile = 128;
   int p2p_list = 128;
+  bool p2p_list_set = false;  // chosen by a call: taken as it is (p2p_slice)
   double p2p_stage = 8.0;
   int p2p_per_lane = 1;
   P2PSplit p2p_split;
@@ -124,6 +125,7 @@ struct tc_context {
   int tree_levels = 0;  // levels of the last tree (batch size of the next build)
   HBuf<int4> h_items;
   size_t n_items = 0;
+  int items_slice = 0;  // the list slice they were cut with
   DBuf p2p_items, p2p_ranges, npairs;
   int nleaves = 0;
   // traversal / lists

@@ -398,22 +398,28 @@ static int build_lists(tc_context *ctx, int &nchunks) {
   return 0;
 }
 
-// P2P work items: every target group x slices of at most p2p_list list entries
-// (fewer where the whole list is short).
+// List entries per P2P work item: a slice that was set or tuned as it is, and
+// by default 128 or, where the whole list is short, as few as 16, so that even
+// a small system's list makes thousands of items: a wave's time is its chain of
+// tiles, and two or three waves a SIMD leave the chip waiting for the longest.
+// P2P, list slice 128 / this rule, in us: N = 10,007 (95 K entries, 16) 416 /
+// 143; 30,000 (296 K, 16) 729 / 369; 131,072 (515 K, 16) 852 / 630; 262,144
+// (2.4 M, 74) 2,705 / 2,480; from 4 M entries on 64 and 128 are level, while 16
+// and less restage too often.
+static int p2p_slice(const tc_context *ctx) {
+  constexpr int kMinSlice = 16, kSliceShare = 1 << 15;
+  if (ctx->p2p_list_set) return ctx->p2p_list;
+  return (int)std::min<long long>(
+      ctx->p2p_list, std::max<long long>(kMinSlice, ctx->st.n_p2p_cells / kSliceShare));
+}
+
+// P2P work items: every target group x slices of p2p_slice() list entries.
 // Each leaf is cut into target groups of <= 64 bodies by the lane model of
 // the kernel (P2PSplit).  The per-leaf list lengths were copied to pinned
 // memory on near_stream, where the upload is queued too; the host loop runs
 // while the GPU runs M2L.
 static int build_p2p_items(tc_context *ctx) {
-  // Slices so that even a small system's list makes thousands of items: a
-  // wave's time is its chain of tiles, and two or three waves a SIMD leave the
-  // chip waiting for the longest.  P2P, list slice 128 / this rule, in us:
-  // N = 10,007 (95 K entries, 16) 416 / 143; 30,000 (296 K, 16) 729 / 369;
-  // 131,072 (515 K, 16) 852 / 630; 262,144 (2.4 M, 74) 2,705 / 2,480; from 4 M
-  // entries on 64 and 128 are level, while 16 and less restage too often.
-  const int kMinSlice = 16, kSliceShare = 1 << 15;
-  const int kList = std::min<long long>(
-      ctx->p2p_list, std::max<long long>(kMinSlice, ctx->st.n_p2p_cells / kSliceShare));
+  const int kList = p2p_slice(ctx);
   TC_CHECK(spin_event(ctx->ev[11]));  // leaf ids and body counts (build_tree)
   TC_CHECK(spin_event(ctx->ev[15]));  // list lengths (build_lists)
   const int *pcnt = ctx->h_pcnt.p, *leaves = ctx->h_leaves.p, *nbd = ctx->h_nbd.p;
@@ -443,6 +449,7 @@ static int build_p2p_items(tc_context *ctx) {
     }
   }
   ctx->n_items = nitem;
+  ctx->items_slice = kList;
   TC_CHECK(ctx->p2p_items.ensure(sizeof(int4) * std::max<size_t>(nitem, 1)));
   TC_CHECK(hipMemcpyAsync(ctx->p2p_items.p, items, sizeof(int4) * nitem, hipMemcpyHostToDevice,
                           ctx->near_stream));
@@ -1323,6 +1330,7 @@ int tc_set_p2p_shape(tc_context *ctx, int tile, int list_slice, double stage_rou
   }
   ctx->p2p_tile = tile;
   ctx->p2p_list = list_slice;
+  ctx->p2p_list_set = true;
   ctx->p2p_stage = stage_rounds;
   ctx->p2p_per_lane = targets_per_lane;
   return 0;
@@ -1348,10 +1356,19 @@ int tc_get_p2p_shape(tc_context *ctx, int *tile, int *list_slice, double *stage_
   return 0;
 }
 
+int tc_p2p_items(const tc_context *ctx, long long *items, int *list_slice) {
+  if (!ctx || !ctx->p2p_ready) return -1;
+  if (items) *items = (long long)ctx->n_items;
+  if (list_slice) *list_slice = ctx->items_slice;
+  return 0;
+}
+
 // Re-run the last evaluation's near field under every launch shape of a small
 // grid (targets per lane x tile x list slice x staging cost, in that nesting
-// order), each `reps` times, timed with events on the near-field stream; keep
-// the fastest.  The lists, ranges and host copies of the list lengths are
+// order; each slice as it is), each `reps` times, timed with events on the
+// near-field stream; keep the fastest.  Where none is faster than the shape set
+// before, that one stays, with the slice chosen by the list's length if it was
+// not set.  The lists, ranges and host copies of the list lengths are
 // those of the last evaluation; the launches add into the context's own
 // near-field result set (zeroed by the next evaluation), never into the
 // caller's arrays.  The mixed-precision forms run one target per lane, so
@@ -1375,12 +1392,17 @@ int tc_tune_p2p(tc_context *ctx, int reps, double *best_ms, double *default_ms,
   const double stages[] = {0.0, 2.0, 4.0, 8.0};
   const int t0 = ctx->p2p_tile, l0 = ctx->p2p_list, r0 = ctx->p2p_per_lane;
   const double g0 = ctx->p2p_stage;
+  const bool set0 = ctx->p2p_list_set;
   hipStream_t s2 = ctx->near_stream;
-  auto run = [&](int per_lane, int tile, int list, double stage, float *ms) -> int {
+  auto use = [&](int per_lane, int tile, int list, bool set, double stage) {
     ctx->p2p_per_lane = per_lane;
     ctx->p2p_tile = tile;
     ctx->p2p_list = list;
+    ctx->p2p_list_set = set;
     ctx->p2p_stage = stage;
+  };
+  auto run = [&](int per_lane, int tile, int list, bool set, double stage, float *ms) -> int {
+    use(per_lane, tile, list, set, stage);
     if (int e = build_p2p_items(ctx)) return e;
     TC_CHECK(hipStreamSynchronize(s2));  // the item upload
     float best = 1e30f;
@@ -1401,9 +1423,10 @@ int tc_tune_p2p(tc_context *ctx, int reps, double *best_ms, double *default_ms,
     return 0;
   };
   float tdef = 0;
-  if (int e = run(r0, t0, l0, g0, &tdef)) return e;
+  if (int e = run(r0, t0, l0, set0, g0, &tdef)) return e;
   float tbest = tdef;
   int br = r0, bt = t0, bl = l0;
+  bool bset = set0;
   double bg = g0;
   int k = 0;
   for (int per_lane : per_lanes)
@@ -1411,7 +1434,7 @@ int tc_tune_p2p(tc_context *ctx, int reps, double *best_ms, double *default_ms,
       for (int list : lists)
         for (double stage : stages) {
           float t = 0;
-          if (int e = run(per_lane, tile, list, stage, &t)) return e;
+          if (int e = run(per_lane, tile, list, true, stage, &t)) return e;
           if (grid_ms) grid_ms[k] = t;
           k++;
           if (t < tbest) {
@@ -1419,13 +1442,11 @@ int tc_tune_p2p(tc_context *ctx, int reps, double *best_ms, double *default_ms,
             br = per_lane;
             bt = tile;
             bl = list;
+            bset = true;
             bg = stage;
           }
         }
-  ctx->p2p_per_lane = br;
-  ctx->p2p_tile = bt;
-  ctx->p2p_list = bl;
-  ctx->p2p_stage = bg;
+  use(br, bt, bl, bset, bg);
   if (best_ms) *best_ms = tbest;
   if (default_ms) *default_ms = tdef;
   return 0;

@@ -93,3 +93,57 @@ def test_tuner_keeps_results(torch_cuda):
     assert s1["n_p2p_pairs"] == s0["n_p2p_pairs"]
     assert relerr_vec(a1, a0)[1] < 1e-13 and relerr_vec(j1, j0)[1] < 1e-12
     f.close()
+
+
+def test_slices_are_taken_as_set(torch_cuda):
+    """A slice that was set or tuned cuts the list whatever its length; by
+    default a short list takes smaller slices (a 2^15th of it, 16 to 128)."""
+    import taichi_collisional_amd as tca
+    from taichi_collisional_amd import ics
+    torch = torch_cuda
+    x, v, m = ics.plummer(40000, seed=17)
+    dev = tuple(torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (x, v, m))
+    f = tca.Fmm(p=4, ncrit=64, theta=0.5, direct_below=0)
+    f.set_shift([0.15, -0.05, 0.2])
+    with pytest.raises(RuntimeError):  # nothing evaluated yet
+        f.p2p_items()
+    entries = _run(torch, f, dev)[3]["n_p2p_cells"]
+    assert entries < 128 << 15
+    rule = min(128, max(16, entries >> 15))
+    assert f.p2p_items()[1] == rule
+    items = []
+    for lst in (1, rule, 37, 64, 128, 256, 1000):
+        f.set_p2p_shape(128, lst, 8.0, 1)
+        _run(torch, f, dev)
+        items.append(f.p2p_items())
+        assert items[-1][1] == lst
+    n = [k for k, _ in items]
+    # lists average some 100 entries here: up to 128 a longer slice means fewer items
+    assert all(a > b for a, b in zip(n[:5], n[1:5])) and n[4] >= n[5] >= n[6] > 0
+    f.set_p2p_shape(128, 1, 8.0, 1)  # a shape that every one of the tuner's beats
+    _run(torch, f, dev)
+    shape, best, dflt = f.tune_p2p(reps=2)
+    assert shape[1] in (64, 128, 256) and best < dflt
+    _run(torch, f, dev)
+    assert f.p2p_items()[1] == shape[1]
+    f.close()
+
+
+def test_tuner_times_every_slice_of_its_grid(torch_cuda):
+    """Where the default shape is the fastest, it stays with the slice chosen by
+    the list's length; the last shape that the tuner timed was cut at 256."""
+    import taichi_collisional_amd as tca
+    from taichi_collisional_amd import ics
+    torch = torch_cuda
+    x, v, m = ics.plummer(12000, seed=5)
+    dev = tuple(torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (x, v, m))
+    f = tca.Fmm(p=4, ncrit=64, theta=0.5, direct_below=0)
+    f.set_shift([0.15, -0.05, 0.2])
+    _run(torch, f, dev)
+    k16, l16 = f.p2p_items()
+    shape, best, dflt = f.tune_p2p(reps=2)
+    k256, l256 = f.p2p_items()
+    assert (l16, l256) == (16, 256) and k256 < k16
+    _run(torch, f, dev)
+    assert f.p2p_items()[1] == (16 if best == dflt else shape[1])
+    f.close()
