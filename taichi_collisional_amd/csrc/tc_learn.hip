@@ -254,7 +254,7 @@ __global__ void k_count_targets(const int2 *__restrict__ pairs, int n, int *__re
 // One lane per (leaf, candidate (q, theta)), as many whole leaves per wave as
 // fit: predicted log10 error (the features clamped to their training range: no
 // extrapolation), then per leaf the cheapest candidate at or below log_target
-// (where none is, the keys 1e30f + y are all 1e30f: the first of the grid); the
+// or, where none is, the most accurate (equal ones: the first of the grid); the
 // leaf's choice goes to q[leaf cell], theta[leaf cell].  With the five angles
 // that a model offers at one order, a leaf per wave left 59 lanes idle: 14,200
 // leaves 466 -> 100 us.
@@ -276,15 +276,18 @@ __global__ __launch_bounds__(64) void k_leaf_select(const float *__restrict__ P,
   x[kLeafFeatures] = (float)g.q[c] / 20.0f;
   x[kLeafFeatures + 1] = (float)g.theta[c];
   const float y = mlp_eval(P, x);
-  // key: feasible candidates by cost, then the rest
-  const float mine = y <= log_target ? g.cost[c] : 1e30f + y;
-  float key = 3e38f;
-  int best = 0;
+  // candidates that meet the target by cost, before the others by error
+  const int meets = y <= log_target;
+  const float mine = meets ? g.cost[c] : y;
+  float key = INFINITY;
+  int best = 0, met = 0;
   for (int k = 0; k < g.ncand; k++) {
     const float k2 = __shfl(mine, slot * g.ncand + k, kWave);
-    if (k2 < key) {
+    const int m2 = __shfl(meets, slot * g.ncand + k, kWave);
+    if (k2 == k2 && (m2 > met || (m2 == met && k2 < key))) {
       key = k2;
       best = k;
+      met = m2;
     }
   }
   if (act && c == best) {
