@@ -81,12 +81,14 @@ static int ensure_cells(tc_context *ctx, int nc, int keep) {
 // The scan words of tree levels (of cells cells at most) and walk steps, one
 // size for both: a walk that outgrew the tree's would free them, and that waits
 // for the moments on the other stream (a first error-MAC evaluation, N =
-// 300,007: 1 ms).  Cleared when they are new or the tags run out, so that no
-// launch finds its own tag there (a tag per launch, fewer than 2^20 between two
-// calls).
+// 300,007: 1 ms).  Cleared when they are new and every kScanTags launches, so
+// that no launch finds its own tag there (a tag per launch; they have 28 bits,
+// and fewer than 2^20 launches come between two calls).  A hundred evaluations
+// pass between two clears, and the clear is part of ordinary use.
+constexpr unsigned kScanTags = 1 << 12;
 static int scan_words(tc_context *ctx, size_t cells) {
   const size_t bytes = sizeof(unsigned long long) * std::max(tree_words(cells), kTravWords);
-  if (ctx->twords.bytes < bytes || ctx->scan_tag > (1u << 27)) {
+  if (ctx->twords.bytes < bytes || ctx->scan_tag > kScanTags) {
     TC_CHECK(ctx->twords.ensure(bytes));
     TC_CHECK(hipMemsetAsync(ctx->twords.p, 0, ctx->twords.bytes, ctx->stream));
     ctx->scan_tag = 0;

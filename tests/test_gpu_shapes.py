@@ -212,3 +212,42 @@ def test_gpu_l2l_beside_a_long_p2p(torch_cuda, oracle_lib, p):
     o = oracle_lib.Oracle(p, ncrit=5, theta=0.28, shift_frac=u)
     _, oa, oj, _ = o.eval(x, v, m)
     assert relerr_vec(ga, oa)[1] < 1e-10 and relerr_vec(gj, oj)[1] < 1e-9
+
+
+@pytest.mark.parametrize("n,ncrit,theta", [(4096, 1, 0.3), (5000, 2, 0.3), (4097, 3, 0.3)])
+def test_gpu_levels_and_steps_of_many_tiles(torch_cuda, oracle_lib, n, ncrit, theta):
+    """Levels of more cells than the launch's blocks hold at once (64 each, n / 512
+    but at least 8 blocks) and walk steps of several rounds per block (256 pairs a
+    round, n / 32 but at least 64 blocks): the oracle's tree and lists."""
+    import taichi_collisional_amd as tca
+    u = [0.2, -0.3, 0.1]
+    rng = np.random.default_rng(n)
+    x, v, m = rng.random((n, 3)), rng.normal(size=(n, 3)), np.full(n, 1.0 / n)
+    f = tca.Fmm(p=6, ncrit=ncrit, theta=theta, direct_below=0)
+    f.set_shift(u)
+    _, ga, gj = _eval(torch_cuda, f, x, v, m)
+    o = oracle_lib.Oracle(6, ncrit=ncrit, theta=theta, shift_frac=u)
+    _, oa, oj, _ = o.eval(x, v, m)
+    st = f.stats()
+    for k in ("ncells", "nleaves", "depth", "n_m2l", "n_p2p_cells", "n_p2p_pairs"):
+        assert st[k] == o.stats[k], k
+    # the widest level holds at least the average one's cells, the widest of at
+    # most 2 depth + 1 steps at least that share of the lists' pairs
+    assert st["ncells"] / (st["depth"] + 1) > 64 * max(8, n // 512)
+    assert (st["n_m2l"] + st["n_p2p_cells"]) / (2 * st["depth"] + 1) > 256 * max(64, n // 32)
+    assert relerr_vec(ga, oa)[1] < 1e-10 and relerr_vec(gj, oj)[1] < 1e-9
+
+
+def test_gpu_many_evaluations_on_one_context(torch_cuda):
+    """The scans' tags start again after some hundred evaluations: all of them give
+    the first one's forces (the atomics' order is the only difference)."""
+    import taichi_collisional_amd as tca
+    from taichi_collisional_amd import ics
+    torch = torch_cuda
+    d = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in ics.plummer(2001, seed=1)]
+    f = tca.Fmm(p=4, ncrit=16, theta=0.6, direct_below=0)
+    f.set_shift([0.1, 0.2, -0.3])
+    first = [t.clone() for t in f.eval(*d)]
+    for _ in range(400):
+        for g, w in zip(f.eval(*d), first):
+            assert float((g - w).abs().max()) <= 1e-12 * float(w.abs().max())
