@@ -142,7 +142,7 @@ struct tc_context {
   bool has_acc_old = false;  // the last evaluation ran the pre-pass
   int last_n = 0;
   // direct
-  DBuf dtg, dpot, dacc, djerk, dx3, dv3, dm, dfl;
+  DBuf dtg, dx3, dv3, dm, dfl;
   // host Body records: page-locked staging and device result buffers
   HBuf<double> h_stage;
   DBuf hop, hoa, hoj;

@@ -99,8 +99,7 @@ static int scan_words(tc_context *ctx, size_t cells) {
 // Tree levels are queued in batches without host reads (TreeState on the
 // device holds the level range and counts); a batch's last level reports the
 // state to pinned memory, which says whether it had no children.  A level whose
-// children do not fit
-// the cell arrays ends the build with a flag and what it needed: the arrays
+// children do not fit the cell arrays ends the build with a flag and what it needed: the arrays
 // grow and the build starts again from the root (a new workload's first
 // evaluation, or a tree that a new root shift makes larger).
 static int build_tree(tc_context *ctx, int n) {
@@ -1244,7 +1243,7 @@ int tc_destroy(tc_context *ctx) {
                  &ctx->m2l, &ctx->p2p, &ctx->tstate, &ctx->twords, &ctx->tcls, &ctx->tree_state,
                  &ctx->gsort1[0], &ctx->gsort1[1], &ctx->gsort1[2], &ctx->gsort1[3], &ctx->gsort2[0], &ctx->gsort2[1], &ctx->gsort2[2], &ctx->gsort2[3], &ctx->m2l_cnt, &ctx->m2l_off, &ctx->m2l_cur,
                  &ctx->m2l_src, &ctx->m2l_coff, &ctx->m2l_chunks, &ctx->p2p_cnt, &ctx->p2p_off,
-                 &ctx->p2p_cur, &ctx->p2p_src, &ctx->dtg, &ctx->dpot, &ctx->dacc, &ctx->djerk,
+                 &ctx->p2p_cur, &ctx->p2p_src, &ctx->dtg,
                  &ctx->dx3, &ctx->dv3, &ctx->dm, &ctx->dfl, &ctx->hop, &ctx->hoa, &ctx->hoj, &ctx->mlend, &ctx->mts, &ctx->mts_sorted,
                  &ctx->msym_cnt, &ctx->msym_off, &ctx->msym_tmp, &ctx->m2l_sym, &ctx->mdpart,
                  &ctx->fpot, &ctx->fax, &ctx->fay, &ctx->faz, &ctx->fjx, &ctx->fjy, &ctx->fjz,
@@ -1678,8 +1677,6 @@ int tc_eval_bodies(tc_context *ctx, tc_body *bodies, int n) {
   TC_CHECK(hipMemcpyAsync(ctx->dv3.p, hv, 24 * N, hipMemcpyHostToDevice, s));
   TC_CHECK(hipMemcpyAsync(ctx->dm.p, hm, 8 * N, hipMemcpyHostToDevice, s));
   TC_CHECK(hipMemcpyAsync(ctx->dfl.p, hf, N, hipMemcpyHostToDevice, s));
-  // the all-pairs branch of eval_device uses dpot/dacc/djerk as its own
-  // scratch, so the results land in separate buffers
   double *op = ctx->hop.as<double>(), *oa = ctx->hoa.as<double>(), *oj = ctx->hoj.as<double>();
   int e = eval_device(ctx, n, ctx->dx3.as<double>(), ctx->dv3.as<double>(), ctx->dm.as<double>(),
                       ctx->dfl.as<unsigned char>(), op, oa, oj);

@@ -18,8 +18,9 @@
 //
 // Layout (default build): one thread per target body in tree (sorted) order, so each block's
 // targets are neighbours; sources stream through LDS in tiles of kMT bodies in
-// the same sorted order, with a flag byte per source marking "is a source" and
-// "last body of its leaf".  Results are written at the caller's index.
+// the same sorted order, with mass 0 for a body that is not a source; with time
+// steps the last bodies of the leaves are a bit per source (k_master_direct_steps).
+// Results are written at the caller's index.
 #include <hip/hip_runtime.h>
 
 #include "tc_common.h"

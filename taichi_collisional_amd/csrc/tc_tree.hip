@@ -1135,8 +1135,8 @@ int launch_scan(const int *in, int *out, int n, void *temp, size_t temp_bytes, h
 // ------------------------------------------------------------ traversal -----
 // One breadth-first step in one launch: every block classifies its range of
 // the frontier, its counts (M2L, P2P, child pairs) are turned into list
-// positions by a scan over the blocks that runs while they do (decoupled
-// look-back, below), and it writes its outputs there, so the lists come out in
+// positions by a scan over the blocks that runs while they do (look_back,
+// above), and it writes its outputs there, so the lists come out in
 // frontier order (deterministic).
 // The walks' squared distance norm(dX) (kernel_fast_lean.h:113-116) and one
 // error-MAC term (traverse_eager.h:80-88, master :82-90) rounded as the
