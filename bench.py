@@ -763,10 +763,12 @@ def main():
                      "hw_fp64_flops_per_launch": hw_flops,
                      "hw_frac": (hw_flops / (m2l_ms * 1e-3) / 1e12 / PEAK_FP64_TFLOPS
                                  if hw_flops else None),
-                     "note": "k_m2l issues no MFMA: it is bound by FP64 VALU issue "
-                             "(v_fma_f64; 78.6 TFLOP/s vector peak). frac counts the "
+                     "note": "k_m2l is bound by FP64 issue (v_fma_f64; 78.6 TFLOP/s "
+                             "vector peak); only the sums over a wave's pairs run on the "
+                             "matrix unit (v_mfma_f64_4x4x4). frac counts the "
                              "reference's algorithmic flops; hw_frac the FP64 flops the "
-                             "kernel executes (SQ_INSTS_VALU_{FMA,MUL,ADD}_F64 counters)"},
+                             "kernel executes on the vector unit "
+                             "(SQ_INSTS_VALU_{FMA,MUL,ADD}_F64 counters)"},
         "cpu_baseline": cpu,
         "near_field": {"kernel": "k_p2p (P2P, FP64)", "ms_per_launch": phases["p2p"],
                        "flops_per_launch": 44.0 * st["n_p2p_pairs"],
